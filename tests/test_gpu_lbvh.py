@@ -184,3 +184,17 @@ def test_device_collapse_is_host_collapse(torch_gpu, idx):
     ch, nh = _canonical(hn, hp)
     assert nd == nh == len(dn)
     assert cd == ch
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 16, 17, 64, 65, 255, 256, 257, 1024, 1025, 4097, 65537])
+def test_stage_lbvh_boxes_at_level_edges(torch_gpu, n):
+    """Node boxes from the leaf-order levels (groups of 4, 16, 64, ...) where
+    a level is full, one short and one over; equal to the climb's, bit for
+    bit, since min and max do not depend on the order."""
+    rng = np.random.default_rng(n)
+    codes = np.unique(rng.integers(0, 1 << 63, size=n + 8, dtype=np.uint64))[:n]
+    order, aabbs = _lbvh_inputs(codes, n + 1)
+    nodes, boxes = _gpu_lbvh(codes, order, aabbs)
+    rnodes, rboxes = refcpu.lbvh_from_sorted(codes, order, aabbs)
+    assert np.array_equal(nodes, rnodes)
+    assert np.array_equal(boxes.view(np.uint32), rboxes.view(np.uint32))
