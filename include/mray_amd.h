@@ -215,7 +215,7 @@ size_t mray_lbvh_temp_bytes(uint32_t count);
 /* The radix sort above with no workspace argument and no allocation.  No
  * counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc).  Its scratch (12.3 MiB, sized for
+ * forbid hipMalloc).  Its scratch (12.5 MiB, sized for
  * MRAY_NOALLOC_SORT_MAX pairs) is a static device array, one copy per GPU,
  * held until the process ends; larger counts return MRAY_ERR_INVALID.
  * Every call on one GPU shares that GPU's scratch: calls that overlap on one

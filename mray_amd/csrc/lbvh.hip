@@ -3,6 +3,7 @@
 #include "common.h"
 #include "lbvh.h"
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 
@@ -155,18 +156,96 @@ KCMorton30(const float* __restrict__ centers, uint32_t n, const float* __restric
 }
 
 // ---------------------------------------------------------------------------
-// Stable LSD radix sort of (u64 key, u32 value), 8 bits per pass.
-// Per pass: tile histograms -> one exclusive scan (digit-major) -> stable
-// scatter.  The scatter ranks a 4096-key tile in 16 rounds of 256 keys; inside
-// a round each wave64 splits its keys by digit with 8 ballots (peers of a lane
-// = lanes holding the same digit), and the four waves are merged through a
-// [4][256] LDS count table, so equal digits keep input order.
+// Stable LSD radix sort of (u64 key, u32 value), 8 bits per pass, in one of
+// two forms by count:
+//
+// Up to 12288 pairs: one workgroup of 16 waves keeps every pair in registers
+// and permutes them through LDS between passes (KCRadixSortOneGroup), one
+// launch and no global traffic between passes.  Bound by the latency of its
+// serial ranking rounds.  9,800 pairs: 24 launches, 195 us -> one launch,
+// 69 us.  Beyond that the 160 KiB of LDS are full.
+//
+// More: per pass a tile histogram, a scan and a scatter.
+//   KCRadixHist     counts of each tile, digit-major
+//   KCRadixScan     one workgroup per digit scans its row over the tiles (the
+//                   256 digit totals are scanned by every scatter block)
+//   KCRadixScatter  ranks a tile, sorts it by digit in LDS and writes it out,
+//                   so that a digit's keys leave in one run: bound by HBM
+//                   (24 B per pair and pass)
+// The scan was one workgroup walking all 256 x tiles counts: 247 us a pass
+// at 2.25 M pairs, now 4.8 us; the scatter 40.1 -> 22.2 us.
+//
+// Ranking (both forms): a wave owns 64 R consecutive pairs and takes them 64
+// at a time; 8 ballots give each lane the lanes with its digit (its peers),
+// and a per-wave count table in LDS gives the pairs of that digit in the
+// wave's earlier rounds, so equal digits keep input order.
 // ---------------------------------------------------------------------------
 static constexpr uint32_t kRsThreads = 256;
-static constexpr uint32_t kRsRounds = 16;
-static constexpr uint32_t kRsTile = kRsThreads * kRsRounds;
 static constexpr uint32_t kRsWaves = kRsThreads / 64;
+static constexpr uint32_t kRsOneThreads = 1024;
+static constexpr uint32_t kRsOneMax = kRsOneThreads * 12u;
+// Rounds per wave of a tile: small tiles until they fill the 256 CUs about
+// twice over (a tile's rounds are serial), then large ones, whose digit runs
+// are longer (64 B at 2048 pairs, 128 B at 4096).
+static constexpr uint32_t kRsSmallRounds = 4, kRsLargeRounds = 16;
+static constexpr uint32_t kRsLargeFrom = 1u << 19;
+static constexpr uint32_t RsTile(uint32_t n)
+{
+    return kRsThreads * ((n < kRsLargeFrom) ? kRsSmallRounds : kRsLargeRounds);
+}
 
+// Lanes of the wave whose key has this lane's digit (valid lanes only).
+__device__ __forceinline__ uint64_t DigitPeers(uint32_t digit, bool valid)
+{
+    const uint64_t in = __ballot(valid);
+    uint32_t lo = uint32_t(in), hi = uint32_t(in >> 32);
+    #pragma unroll
+    for(uint32_t b = 0; b < 8; b++)
+    {
+        const uint32_t one = (digit >> b) & 1u;
+        const uint64_t bb = __ballot(one != 0u);
+        const uint32_t mask = 0u - one;
+        lo &= ~(uint32_t(bb) ^ mask);
+        hi &= ~(uint32_t(bb >> 32) ^ mask);
+    }
+    return (uint64_t(hi) << 32) | lo;
+}
+
+// One ranking round: pairs of this digit that the wave met before this lane's
+// (in earlier rounds and in lower lanes); `cnt` is the wave's count table.
+template<class C>
+__device__ __forceinline__ uint32_t RankRound(C* cnt, uint32_t digit, bool valid, uint64_t ltMask)
+{
+    const uint64_t peers = DigitPeers(digit, valid);
+    const uint32_t rank = uint32_t(__popcll(peers & ltMask));
+    const uint32_t before = cnt[digit];
+    __builtin_amdgcn_wave_barrier();
+    if(valid && rank == 0) cnt[digit] = C(before + uint32_t(__popcll(peers)));
+    __builtin_amdgcn_wave_barrier();
+    return before + rank;
+}
+
+// Exclusive scan over the 256 threads of waves 0..3 (every thread of the
+// block calls it; threads past 255 only join the barriers).
+__device__ __forceinline__ uint32_t ScanDigits(uint32_t v, uint32_t* waveSum)
+{
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint32_t incl = v;
+    for(uint32_t o = 1; o < 64; o <<= 1)
+    {
+        const uint32_t up = __shfl_up(incl, o);
+        if(lane >= o) incl += up;
+    }
+    if(wave < 4 && lane == 63) waveSum[wave] = incl;
+    __syncthreads();
+    uint32_t excl = incl - v;
+    for(uint32_t w = 0; w < 3; w++)
+        if(w < wave) excl += waveSum[w];
+    __syncthreads();
+    return excl;
+}
+
+template<uint32_t R>
 __global__ void __launch_bounds__(kRsThreads)
 KCRadixHist(const uint64_t* __restrict__ keys, uint32_t n, uint32_t shift, uint32_t numTiles,
             uint32_t* __restrict__ hist)
@@ -174,97 +253,181 @@ KCRadixHist(const uint64_t* __restrict__ keys, uint32_t n, uint32_t shift, uint3
     __shared__ uint32_t h[256];
     h[threadIdx.x] = 0;
     __syncthreads();
-    uint32_t base = blockIdx.x * kRsTile;
-    for(uint32_t r = 0; r < kRsRounds; r++)
+    const uint32_t base = blockIdx.x * kRsThreads * R;
+    #pragma unroll
+    for(uint32_t r = 0; r < R; r++)
     {
-        uint32_t i = base + r * kRsThreads + threadIdx.x;
+        const uint32_t i = base + r * kRsThreads + threadIdx.x;
         if(i < n) atomicAdd(&h[uint32_t(keys[i] >> shift) & 255u], 1u);
     }
     __syncthreads();
     hist[size_t(threadIdx.x) * numTiles + blockIdx.x] = h[threadIdx.x];
 }
 
-// Single-workgroup exclusive scan of `count` u32 values in place.
-__global__ void __launch_bounds__(1024)
-KCExclusiveScanSingle(uint32_t* __restrict__ data, uint32_t count, uint32_t* __restrict__ total)
+// Block d: exclusive scan of digit d's counts over the tiles, in place, and
+// the digit's total.
+__global__ void __launch_bounds__(kRsThreads)
+KCRadixScan(uint32_t* __restrict__ hist, uint32_t numTiles, uint32_t* __restrict__ total)
 {
-    __shared__ uint32_t s[1024];
-    __shared__ uint32_t carry;
-    if(threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for(uint32_t base = 0; base < count; base += 1024)
+    __shared__ uint32_t waveSum[4];
+    __shared__ uint32_t blockSum;
+    uint32_t* row = hist + size_t(blockIdx.x) * numTiles;
+    uint32_t carry = 0;
+    for(uint32_t base = 0; base < numTiles; base += kRsThreads)
     {
-        uint32_t i = base + threadIdx.x;
-        uint32_t v = (i < count) ? data[i] : 0u;
-        s[threadIdx.x] = v;
+        const uint32_t i = base + threadIdx.x;
+        const uint32_t v = (i < numTiles) ? row[i] : 0u;
+        const uint32_t excl = ScanDigits(v, waveSum);
+        if(i < numTiles) row[i] = carry + excl;
+        if(threadIdx.x == kRsThreads - 1u) blockSum = excl + v;
         __syncthreads();
-        for(uint32_t off = 1; off < 1024; off <<= 1)
-        {
-            uint32_t add = (threadIdx.x >= off) ? s[threadIdx.x - off] : 0u;
-            __syncthreads();
-            s[threadIdx.x] += add;
-            __syncthreads();
-        }
-        uint32_t incl = s[threadIdx.x];
-        if(i < count) data[i] = carry + incl - v;
-        __syncthreads();
-        if(threadIdx.x == 1023) carry += incl;
+        carry += blockSum;
         __syncthreads();
     }
-    if(total && threadIdx.x == 0) *total = carry;
+    if(threadIdx.x == 0) total[blockIdx.x] = carry;
 }
 
+template<uint32_t R>
 __global__ void __launch_bounds__(kRsThreads)
 KCRadixScatter(const uint64_t* __restrict__ keysIn, const uint32_t* __restrict__ valsIn,
                uint64_t* __restrict__ keysOut, uint32_t* __restrict__ valsOut, uint32_t n,
-               uint32_t shift, uint32_t numTiles, const uint32_t* __restrict__ histScan)
+               uint32_t shift, uint32_t numTiles, const uint32_t* __restrict__ histScan,
+               const uint32_t* __restrict__ total)
 {
-    __shared__ uint32_t base[256];
-    __shared__ uint32_t waveCnt[kRsWaves][256];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u;
-    const uint32_t wave = tid >> 6;
+    constexpr uint32_t kTile = kRsThreads * R;
+    __shared__ uint64_t sKey[kTile];
+    __shared__ uint32_t sVal[kTile];
+    __shared__ uint32_t cnt[kRsWaves][256];
+    __shared__ uint32_t start[256];     // first local position of a digit
+    __shared__ uint32_t outBase[256];   // its first output position - start
+    __shared__ uint32_t waveSum[4];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint64_t ltMask = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-    base[tid] = histScan[size_t(tid) * numTiles + blockIdx.x];
-    uint32_t running = 0;   // keys of digit `tid` already placed by this tile
-    const uint32_t tileStart = blockIdx.x * kRsTile;
-    for(uint32_t r = 0; r < kRsRounds; r++)
+    const uint32_t tileStart = blockIdx.x * kTile;
+    const uint32_t tileCount = min(kTile, n - tileStart);
+    const uint32_t first = wave * 64u * R + lane;
+    uint64_t key[R];
+    uint32_t val[R], rank[R];
+    #pragma unroll
+    for(uint32_t r = 0; r < R; r++)
     {
-        for(uint32_t w = 0; w < kRsWaves; w++) waveCnt[w][tid] = 0;
+        const uint32_t k = first + r * 64u;
+        key[r] = (k < tileCount) ? keysIn[tileStart + k] : 0ull;
+        val[r] = (k < tileCount) ? valsIn[tileStart + k] : 0u;
+    }
+    const uint32_t tileOff = histScan[size_t(tid) * numTiles + blockIdx.x];
+    const uint32_t digitOff = ScanDigits(total[tid], waveSum);
+    for(uint32_t w = 0; w < kRsWaves; w++) cnt[w][tid] = 0;
+    __syncthreads();
+    #pragma unroll
+    for(uint32_t r = 0; r < R; r++)
+        rank[r] = RankRound(cnt[wave], uint32_t(key[r] >> shift) & 255u, first + r * 64u < tileCount, ltMask);
+    __syncthreads();
+    uint32_t acc = 0;
+    for(uint32_t w = 0; w < kRsWaves; w++)
+    {
+        const uint32_t c = cnt[w][tid];
+        cnt[w][tid] = acc;
+        acc += c;
+    }
+    const uint32_t s = ScanDigits(acc, waveSum);
+    start[tid] = s;
+    outBase[tid] = digitOff + tileOff - s;
+    __syncthreads();
+    #pragma unroll
+    for(uint32_t r = 0; r < R; r++)
+    {
+        if(first + r * 64u >= tileCount) continue;
+        const uint32_t d = uint32_t(key[r] >> shift) & 255u;
+        const uint32_t at = start[d] + cnt[wave][d] + rank[r];
+        sKey[at] = key[r];
+        sVal[at] = val[r];
+    }
+    __syncthreads();
+    #pragma unroll
+    for(uint32_t r = 0; r < R; r++)
+    {
+        const uint32_t j = r * kRsThreads + tid;
+        if(j >= tileCount) continue;
+        const uint64_t k = sKey[j];
+        const uint32_t dst = outBase[uint32_t(k >> shift) & 255u] + j;
+        keysOut[dst] = k;
+        valsOut[dst] = sVal[j];
+    }
+}
+
+// The whole sort of at most 1024 R pairs in one workgroup, in place.
+template<uint32_t R>
+__global__ void __launch_bounds__(kRsOneThreads)
+KCRadixSortOneGroup(uint64_t* __restrict__ keys, uint32_t* __restrict__ vals, uint32_t n)
+{
+    constexpr uint32_t kWaves = kRsOneThreads / 64u;
+    __shared__ uint64_t sKey[kRsOneThreads * R];
+    __shared__ uint32_t sVal[kRsOneThreads * R];
+    __shared__ uint16_t cnt[kWaves][256];     // counts and positions stay below 12288
+    __shared__ uint16_t start[256];
+    __shared__ uint32_t waveSum[4];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint64_t ltMask = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
+    // the pairs in use split evenly over the waves, in 64s
+    const uint32_t rounds = (n + kRsOneThreads - 1u) / kRsOneThreads;
+    const uint32_t first = wave * 64u * rounds + lane;
+    uint64_t key[R];
+    uint32_t val[R], rank[R];
+    #pragma unroll
+    for(uint32_t r = 0; r < R; r++)
+    {
+        const uint32_t k = first + r * 64u;
+        const bool in = r < rounds && k < n;
+        key[r] = in ? keys[k] : 0ull;
+        val[r] = in ? vals[k] : 0u;
+    }
+    for(uint32_t shift = 0; shift < 64u; shift += 8u)
+    {
+        for(uint32_t e = tid; e < kWaves * 256u; e += kRsOneThreads) cnt[0][e] = 0;
         __syncthreads();
-        uint32_t i = tileStart + r * kRsThreads + tid;
-        bool valid = (i < n);
-        uint64_t key = valid ? keysIn[i] : 0ull;
-        uint32_t val = valid ? valsIn[i] : 0u;
-        uint32_t digit = uint32_t(key >> shift) & 255u;
-        uint64_t peers = __ballot(valid);
         #pragma unroll
-        for(uint32_t b = 0; b < 8; b++)
-        {
-            uint64_t bb = __ballot((digit >> b) & 1u);
-            peers &= ((digit >> b) & 1u) ? bb : ~bb;
-        }
-        uint32_t rank = uint32_t(__popcll(peers & ltMask));
-        if(valid && rank == 0) waveCnt[wave][digit] = uint32_t(__popcll(peers));
+        for(uint32_t r = 0; r < R; r++)
+            if(r < rounds)
+                rank[r] = RankRound(cnt[wave], uint32_t(key[r] >> shift) & 255u, first + r * 64u < n, ltMask);
         __syncthreads();
-        {
-            uint32_t acc = running;
-            for(uint32_t w = 0; w < kRsWaves; w++)
+        uint32_t acc = 0;
+        if(tid < 256u)
+            for(uint32_t w = 0; w < kWaves; w++)
             {
-                uint32_t c = waveCnt[w][tid];
-                waveCnt[w][tid] = acc;
+                const uint32_t c = cnt[w][tid];
+                cnt[w][tid] = uint16_t(acc);
                 acc += c;
             }
-            running = acc;
-        }
+        const uint32_t s = ScanDigits(acc, waveSum);
+        if(tid < 256u) start[tid] = uint16_t(s);
         __syncthreads();
-        if(valid)
+        #pragma unroll
+        for(uint32_t r = 0; r < R; r++)
         {
-            uint32_t dst = base[digit] + waveCnt[wave][digit] + rank;
-            keysOut[dst] = key;
-            valsOut[dst] = val;
+            if(r >= rounds || first + r * 64u >= n) continue;
+            const uint32_t d = uint32_t(key[r] >> shift) & 255u;
+            const uint32_t at = uint32_t(start[d]) + cnt[wave][d] + rank[r];
+            sKey[at] = key[r];
+            sVal[at] = val[r];
         }
         __syncthreads();
+        #pragma unroll
+        for(uint32_t r = 0; r < R; r++)
+        {
+            const uint32_t k = first + r * 64u;
+            if(r >= rounds || k >= n) continue;
+            key[r] = sKey[k];
+            val[r] = sVal[k];
+        }
+    }
+    #pragma unroll
+    for(uint32_t r = 0; r < R; r++)
+    {
+        const uint32_t k = first + r * 64u;
+        if(r >= rounds || k >= n) continue;
+        keys[k] = key[r];
+        vals[k] = val[r];
     }
 }
 
@@ -600,12 +763,28 @@ int LaunchMorton30(const float* dCenters, uint32_t n, const float* dBox, uint32_
     return MRAY_OK;
 }
 
+// Temporary area: tile histograms, digit totals, then the other half of the
+// ping-pong pair.
+static constexpr size_t RsHistBytes(uint32_t n)
+{
+    const size_t tiles = (size_t(n) + RsTile(n) - 1) / RsTile(n);
+    return ((256u * (tiles ? tiles : 1u) + 256u) * sizeof(uint32_t) + 255) / 256 * 256;
+}
+
 size_t RadixSortTempBytes(uint32_t n)
 {
-    uint32_t tiles = std::max(1u, DivUp(n, kRsTile));
-    size_t hist = size_t(256) * tiles * sizeof(uint32_t);
-    size_t kv = size_t(n) * (sizeof(uint64_t) + sizeof(uint32_t));
-    return ((hist + 255) / 256) * 256 + kv + 256;
+    return RsHistBytes(n) + size_t(n) * (sizeof(uint64_t) + sizeof(uint32_t)) + 256;
+}
+
+template<uint32_t R>
+static void LaunchRadixPass(const uint64_t* srcK, const uint32_t* srcV, uint64_t* dstK, uint32_t* dstV,
+                            uint32_t n, uint32_t shift, uint32_t* hist, hipStream_t s)
+{
+    const uint32_t tiles = DivUp(n, kRsThreads * R);
+    uint32_t* total = hist + size_t(256) * tiles;
+    KCRadixHist<R><<<tiles, kRsThreads, 0, s>>>(srcK, n, shift, tiles, hist);
+    KCRadixScan<<<256, kRsThreads, 0, s>>>(hist, tiles, total);
+    KCRadixScatter<R><<<tiles, kRsThreads, 0, s>>>(srcK, srcV, dstK, dstV, n, shift, tiles, hist, total);
 }
 
 int LaunchRadixSort(uint64_t* dKeys, uint32_t* dVals, uint32_t n, void* dTemp, size_t tempBytes,
@@ -617,11 +796,16 @@ int LaunchRadixSort(uint64_t* dKeys, uint32_t* dVals, uint32_t n, void* dTemp, s
         SetError("radix sort: temporary buffer too small");
         return MRAY_ERR_INVALID;
     }
-    uint32_t tiles = DivUp(n, kRsTile);
+    if(n <= kRsOneMax)
+    {
+        if(n <= kRsOneThreads * 4u) KCRadixSortOneGroup<4><<<1, kRsOneThreads, 0, s>>>(dKeys, dVals, n);
+        else KCRadixSortOneGroup<12><<<1, kRsOneThreads, 0, s>>>(dKeys, dVals, n);
+        MRAY_HIP_CHECK(hipGetLastError());
+        return MRAY_OK;
+    }
     char* t = static_cast<char*>(dTemp);
     uint32_t* hist = reinterpret_cast<uint32_t*>(t);
-    size_t histBytes = ((size_t(256) * tiles * sizeof(uint32_t) + 255) / 256) * 256;
-    uint64_t* altK = reinterpret_cast<uint64_t*>(t + histBytes);
+    uint64_t* altK = reinterpret_cast<uint64_t*>(t + RsHistBytes(n));
     uint32_t* altV = reinterpret_cast<uint32_t*>(altK + n);
     uint64_t* srcK = dKeys;
     uint32_t* srcV = dVals;
@@ -629,12 +813,9 @@ int LaunchRadixSort(uint64_t* dKeys, uint32_t* dVals, uint32_t n, void* dTemp, s
     uint32_t* dstV = altV;
     for(uint32_t pass = 0; pass < 8; pass++)
     {
-        uint32_t shift = pass * 8;
-        KCRadixHist<<<tiles, kRsThreads, 0, s>>>(srcK, n, shift, tiles, hist);
-        MRAY_HIP_CHECK(hipGetLastError());
-        KCExclusiveScanSingle<<<1, 1024, 0, s>>>(hist, 256 * tiles, nullptr);
-        MRAY_HIP_CHECK(hipGetLastError());
-        KCRadixScatter<<<tiles, kRsThreads, 0, s>>>(srcK, srcV, dstK, dstV, n, shift, tiles, hist);
+        if(RsTile(n) == kRsThreads * kRsSmallRounds)
+            LaunchRadixPass<kRsSmallRounds>(srcK, srcV, dstK, dstV, n, pass * 8u, hist, s);
+        else LaunchRadixPass<kRsLargeRounds>(srcK, srcV, dstK, dstV, n, pass * 8u, hist, s);
         MRAY_HIP_CHECK(hipGetLastError());
         std::swap(srcK, dstK);
         std::swap(srcV, dstV);
@@ -646,12 +827,12 @@ int LaunchRadixSort(uint64_t* dKeys, uint32_t* dVals, uint32_t n, void* dTemp, s
 // ---------------------------------------------------------------------------
 // Allocation-free sort (mray_radix_sort_u64_u32_noalloc): the same passes over
 // a scratch area that lives in the code object, one copy per GPU, held until
-// the process ends.  Its size is RadixSortTempBytes(kNoAllocSortMax).
+// the process ends, large enough for every count up to kNoAllocSortMax.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kNoAllocSortMax = MRAY_NOALLOC_SORT_MAX;
 static_assert(kNoAllocSortMax == (1u << 20), "scratch size is stated as 2^20 pairs");
-constexpr size_t kNoAllocSortHistBytes =
-    ((size_t(256) * ((kNoAllocSortMax + kRsTile - 1) / kRsTile) * sizeof(uint32_t) + 255) / 256) * 256;
+// the histograms are largest just below the count where tiles grow
+constexpr size_t kNoAllocSortHistBytes = std::max(RsHistBytes(kNoAllocSortMax), RsHistBytes(kRsLargeFrom - 1u));
 constexpr size_t kNoAllocSortBytes =
     kNoAllocSortHistBytes + size_t(kNoAllocSortMax) * (sizeof(uint64_t) + sizeof(uint32_t)) + 256;
 static __device__ __align__(256) unsigned char scratch[kNoAllocSortBytes];

@@ -186,6 +186,26 @@ def test_device_collapse_is_host_collapse(torch_gpu, idx):
     assert cd == ch
 
 
+@pytest.mark.parametrize("n", [63, 64, 65, 1023, 4097, 12287, 12288, 12289, 16385, 524287, 524288, 600001])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_stage_radix_sort_forms(torch_gpu, n, noalloc):
+    """Both sort forms around their limits: one workgroup up to 12288 pairs,
+    small tiles below 2^19, large tiles from there; ties everywhere, keys with
+    the top bit set."""
+    from mray_amd import native
+    torch = torch_gpu
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, 1 << 64, size=n, dtype=np.uint64)
+    keys[::3] &= np.uint64(0xFF00000000000003)      # long runs of equal keys
+    vals = rng.permutation(n).astype(np.uint32)
+    dk = torch.from_numpy(keys.view(np.int64).copy()).cuda()
+    dv = torch.from_numpy(vals.view(np.int32).copy()).cuda()
+    (native.radix_sort_u64_u32_noalloc if noalloc else native.radix_sort_u64_u32)(dk, dv)
+    order = np.argsort(keys, kind="stable")
+    assert np.array_equal(dk.cpu().numpy().view(np.uint64), keys[order])
+    assert np.array_equal(dv.cpu().numpy().view(np.uint32), vals[order])
+
+
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 16, 17, 64, 65, 255, 256, 257, 1024, 1025, 4097, 65537])
 def test_stage_lbvh_boxes_at_level_edges(torch_gpu, n):
     """Node boxes from the leaf-order levels (groups of 4, 16, 64, ...) where
