@@ -197,15 +197,16 @@ BF16_PEAK_TFLOPS = 2500.0                       # MI355X dense bf16 MFMA
 
 def mlp_roofline(kernel_ms, batch):
     """MFMA roofline of the training GEMM kernels from per-kernel HIP-event
-    times: forward (with the hash encoding fused in), data backward and
-    weight gradients each do one 64 x 64 product per layer and sample."""
+    times: forward with the data gradients (one kernel, the hash encoding
+    fused in: two 64 x 64 products per layer and sample) and the weight
+    gradients (one product)."""
     out = {}
     flops = 0.0
     ms = 0.0
-    for k in ("train_forward", "backward", "wgrad"):
+    for k, products in (("train_forward", 2), ("wgrad", 1)):
         t, n = kernel_ms[k]
         if n:
-            f = MLP_FLOP_PER_SAMPLE * batch
+            f = products * MLP_FLOP_PER_SAMPLE * batch
             out[k] = {"avg_ms": round(t / n, 4),
                       "tflops": round(f / (t / n * 1e-3) / 1e12, 2)}
             flops += f * n

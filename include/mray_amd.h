@@ -594,7 +594,9 @@ int mray_nrc_zero_grads(MRayNrc* nrc, void* stream);
  * MFMA roofline): while on, every launch is timed; mray_nrc_kernel_times
  * synchronises and returns accumulated ms and launch counts [6] for
  * inference forward, training forward, backward, weight gradients, grid
- * scatter and Adam.                                                        */
+ * scatter and Adam.  A fused kernel counts under the first of its parts:
+ * training forward includes the data gradients (backward stays 0), and
+ * mray_nrc_train's Adam counts with the gradients it applies.               */
 int mray_nrc_set_profiling(MRayNrc* nrc, uint32_t on);
 int mray_nrc_kernel_times(MRayNrc* nrc, double* hMs, uint64_t* hLaunches);
 

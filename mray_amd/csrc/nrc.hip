@@ -13,15 +13,24 @@
 // scalars, albedo, a constant 1, zero padding.  Six 64x64 layers (the output
 // layer's columns 3..63 stay zero), ReLU after the first five.
 //
-// Kernels (one wave = 32 samples as one 32x64 activation tile in LDS; the
-// MFMA is gfx950's v_mfma_f32_32x32x16_bf16, 16 k per instruction):
-//   KNrcForward<TRAIN>  encode + 6 layers; inference writes RGB, training also
-//                       stores every layer input (bf16) and dL/dy
-//   KNrcBackward        dZ of every layer (bf16) and dL/d(grid features)
-//   KNrcWgrad           dW = X^T dZ per layer, split over sample chunks
-//   KNrcGridBwd         scatter of the grid-feature gradient (fp32 atomics)
-//   KNrcAdam            Adam on fp32 masters, refreshes the bf16 / fp16 copies
-//                       and clears the gradients for the next step
+// Kernels (one wave = 32 samples; the MFMA is gfx950's v_mfma_f32_32x32x16_bf16,
+// 16 k per instruction, with weights as A and samples as columns of B, so a
+// lane's accumulators are consecutive features of its own sample: packed to
+// bf16 they are the next layer's B operand, and activations never leave
+// registers):
+//   KNrcInfer      encode + 6 layers for queries, weights in LDS
+//   KNrcTrain      encode, forward, loss gradient and the data gradients of
+//                  every layer in one pass; stores each layer's input and
+//                  output gradient transposed (samples contiguous) and the
+//                  gradient of the grid features
+//   KNrcWgrad      dW = X^T dZ, one workgroup per 16 x 16 tile over all
+//                  samples, no atomics; with Adam fused in a training step
+//   KNrcGridOwner  grid gradient: a workgroup owns a table segment in LDS and
+//                  scans the batch for corners inside it; with Adam fused in
+//                  a training step
+//   KNrcGridBwd    grid gradient by global atomics (tables too large or
+//                  batches too small for the scan)
+//   KNrcAdam*      Adam on fp32 masters as a separate pass (mray_nrc_adam)
 #include "common.h"
 #include "scene.h"
 
@@ -40,14 +49,16 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr uint32_t kNrcLayers = 6;
 constexpr uint32_t kW = 64;                  // width of every layer
-constexpr uint32_t kLdsRow = 72;             // padded LDS row: 16-B aligned, conflict-free b128 reads
 constexpr uint32_t kNrcFeat = 2;
 constexpr uint32_t kNrcMaxLevels = 16;
-constexpr uint32_t kFwdWaves = 4;            // 128 samples per block
+constexpr uint32_t kInferTPB = 512;          // 8 waves: 256 queries per block and round
 constexpr uint32_t kLayerParams = kW * kW;
 constexpr uint32_t kMlpParams = kNrcLayers * kLayerParams;
 // kernel kinds timed by mray_nrc_kernel_times: inference forward, training
-// forward, backward (data gradients), weight gradients, grid scatter, Adam
+// forward, backward (data gradients), weight gradients, grid scatter, Adam.
+// A fused kernel counts under the first of its parts: forward and data
+// gradients as training forward, and in a training step Adam with the
+// gradients it applies.
 constexpr uint32_t kNrcKernelKinds = 6;
 
 __device__ __forceinline__ uint16_t F2Bf(float f)
@@ -56,59 +67,136 @@ __device__ __forceinline__ uint16_t F2Bf(float f)
     u += 0x7FFFu + ((u >> 16) & 1u);         // round to nearest even
     return uint16_t(u >> 16);
 }
-__device__ __forceinline__ float Bf2F(uint16_t b) { return __uint_as_float(uint32_t(b) << 16); }
 
 struct NrcView
 {
-    const uint16_t* wT;       // [6][n][k] bf16 (forward operand)
-    const uint16_t* wK;       // [6][k][n] bf16 (backward operand)
+    const uint16_t* wT;       // bf16, fragment order: forward operand (rows n)
+    const uint16_t* wK;       // bf16, fragment order: backward operand (rows k)
     const __half* grid;       // [L][T][2]
     float scale[kNrcMaxLevels];
-    uint32_t res[kNrcMaxLevels];
+    uint32_t my[kNrcMaxLevels];      // index multipliers of y and z: the level's
+    uint32_t mz[kNrcMaxLevels];      // resolution and its square, or the hash primes
     uint32_t dense[kNrcMaxLevels];
     uint32_t levels;
     uint32_t log2T;
 };
 
-// ---- encoding --------------------------------------------------------------
-__device__ __forceinline__ uint32_t GridIndex(const NrcView& v, uint32_t l, uint32_t x, uint32_t y,
-                                              uint32_t z)
+// ---- operand layout ----------------------------------------------------------
+// v_mfma_f32_32x32x16_bf16 D = A B: lane (r, h) = (l mod 32, l / 32) supplies
+// row r of A and column r of B over eight of the step's 16 k, and receives
+// column r of D, rows 8 (e / 4) + 4 h + (e mod 4) for e = 0..15.  The k order
+// inside a step is free as long as A and B agree: slot j of half h in step kt
+// is k = 16 kt + 8 (j / 4) + 4 h + (j mod 4), so D's rows, packed in pairs,
+// are the next product's B operand in the lane that holds them.
+// Element (row, k) of layer l's A operand in fragment order
+// [layer][32-row tile][step][lane][8]: a lane's operand is 16 contiguous
+// bytes and a wave's 1 KiB, conflict-free in LDS and coalesced from memory.
+__host__ __device__ constexpr uint32_t FragIndex(uint32_t l, uint32_t row, uint32_t k)
 {
-    if(v.dense[l])
-    {
-        uint32_t r = v.res[l];
-        return x + y * r + z * r * r;
-    }
-    uint32_t h = (x * 1u) ^ (y * 2654435761u) ^ (z * 805459861u);
-    return h & ((1u << v.log2T) - 1u);
+    const uint32_t c = k & 15u, j = 4u * (c >> 3) + (c & 3u), h = (c >> 2) & 1u;
+    return (((l * 2u + (row >> 5)) * 4u + (k >> 4)) * 64u + (row & 31u) + 32u * h) * 8u + j;
+}
+constexpr uint32_t kFragLayer = 2u * 4u * 64u;   // uint4 words of one layer
+
+__device__ __forceinline__ uint32_t PackBf(float a, float b)
+{
+    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+    const v2bf v = {__bf16(a), __bf16(b)};       // v_cvt_pk_bf16_f32, nearest even
+    return __builtin_bit_cast(uint32_t, v);
 }
 
-struct Corners
+// B operand of one wave: 64 features of the lane's sample, word 4 kt + i =
+// slots 2i, 2i + 1 of step kt.
+struct XRow
 {
-    uint32_t idx[8];
-    float w[8];
+    uint32_t u[32 / 2];
 };
 
-__device__ __forceinline__ void LevelCorners(const NrcView& v, uint32_t l, const float* pos, Corners& c)
+__device__ __forceinline__ v8bf StepOf(const XRow& x, uint32_t kt)
 {
-    float p[3], fr[3];
-    uint32_t i0[3];
-    for(int d = 0; d < 3; d++)
+    const uint4 v = make_uint4(x.u[4 * kt], x.u[4 * kt + 1], x.u[4 * kt + 2], x.u[4 * kt + 3]);
+    return __builtin_bit_cast(v8bf, v);
+}
+
+// One layer's A operand in registers.
+struct Frags
+{
+    uint4 f[8];
+};
+__device__ __forceinline__ Frags LoadFrags(const uint4* __restrict__ w)
+{
+    Frags a;
+    #pragma unroll
+    for(uint32_t i = 0; i < 8; i++) a.f[i] = w[i * 64u + (threadIdx.x & 63u)];
+    return a;
+}
+template<uint32_t TILES, uint32_t STEPS>
+__device__ __forceinline__ void LayerProduct(const Frags& w, const XRow& x, v16f (&acc)[2])
+{
+    acc[0] = v16f{0};
+    acc[1] = v16f{0};
+    #pragma unroll
+    for(uint32_t kt = 0; kt < STEPS; kt++)
+        #pragma unroll
+        for(uint32_t t = 0; t < TILES; t++)
+            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, w.f[t * 4u + kt]),
+                                                             StepOf(x, kt), acc[t], 0, 0, 0);
+}
+
+// acc[t] = rows 32 t.. of one layer's A times x, over the first `steps` k steps.
+template<uint32_t TILES, uint32_t STEPS>
+__device__ __forceinline__ void LayerProduct(const uint4* __restrict__ w, const XRow& x, v16f (&acc)[2])
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    acc[0] = v16f{0};
+    acc[1] = v16f{0};
+    #pragma unroll
+    for(uint32_t kt = 0; kt < STEPS; kt++)
     {
-        p[d] = pos[d] * v.scale[l] + 0.5f;
-        float fl = floorf(p[d]);
-        i0[d] = uint32_t(fl);
-        fr[d] = p[d] - fl;
+        const v8bf b = StepOf(x, kt);
+        #pragma unroll
+        for(uint32_t t = 0; t < TILES; t++)
+        {
+            const v8bf a = __builtin_bit_cast(v8bf, w[(t * 4u + kt) * 64u + lane]);
+            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[t], 0, 0, 0);
+        }
     }
-    for(uint32_t k = 0; k < 8; k++)
-    {
-        uint32_t ox = k & 1u, oy = (k >> 1) & 1u, oz = (k >> 2) & 1u;
-        float w = (ox ? fr[0] : 1.0f - fr[0]);
-        w = w * (oy ? fr[1] : 1.0f - fr[1]);
-        w = w * (oz ? fr[2] : 1.0f - fr[2]);
-        c.w[k] = w;
-        c.idx[k] = GridIndex(v, l, i0[0] + ox, i0[1] + oy, i0[2] + oz);
-    }
+}
+
+__device__ __forceinline__ XRow ReluPack(const v16f (&acc)[2])
+{
+    XRow x;
+    #pragma unroll
+    for(uint32_t t = 0; t < 2; t++)
+        #pragma unroll
+        for(uint32_t i = 0; i < 8; i++)
+            x.u[8 * t + i] = PackBf(MaxF(acc[t][2 * i], 0.0f), MaxF(acc[t][2 * i + 1], 0.0f));
+    return x;
+}
+
+// ---- encoding --------------------------------------------------------------
+__device__ __forceinline__ uint32_t GridIndex(uint32_t dense, uint32_t mask, uint32_t x, uint32_t y, uint32_t z)
+{
+    return dense ? x + y + z : ((x ^ y ^ z) & mask);
+}
+
+// Cell and fraction of a position on one level; iy and iz already multiplied.
+struct Cell
+{
+    uint32_t x, y, z;
+    float fx, fy, fz;
+};
+__device__ __forceinline__ Cell LevelCell(const float* pos, float scale, uint32_t my, uint32_t mz)
+{
+    const float px = pos[0] * scale + 0.5f, py = pos[1] * scale + 0.5f, pz = pos[2] * scale + 0.5f;
+    const float gx = floorf(px), gy = floorf(py), gz = floorf(pz);
+    return {uint32_t(gx), uint32_t(gy) * my, uint32_t(gz) * mz, px - gx, py - gy, pz - gz};
+}
+__device__ __forceinline__ float CornerWeight(const Cell& c, uint32_t k)
+{
+    float w = (k & 1u) ? c.fx : 1.0f - c.fx;
+    w = w * ((k & 2u) ? c.fy : 1.0f - c.fy);
+    return w * ((k & 4u) ? c.fz : 1.0f - c.fz);
 }
 
 __device__ __forceinline__ float OneBlob(float s, uint32_t j)
@@ -118,340 +206,293 @@ __device__ __forceinline__ float OneBlob(float s, uint32_t j)
     return expf(-d * d * 8.0f);              // sigma = 1/4
 }
 
-// Input row of one sample, written by two lanes: `half` 0 takes levels 0..7
-// and columns 32..47, `half` 1 levels 8..15 and columns 48..63.
-__device__ __forceinline__ void EncodeHalf(const NrcView& v, const float* rec, uint32_t half,
-                                           uint16_t* row)
+__device__ __forceinline__ void RecordPos(const float* __restrict__ rec, float pos[3])
 {
-    float pos[3] = {ClampF(rec[0], 0.0f, 1.0f), ClampF(rec[1], 0.0f, 1.0f), ClampF(rec[2], 0.0f, 1.0f)};
-    const uint32_t l0 = half * 8u;
-    for(uint32_t l = l0; l < l0 + 8u; l++)
-    {
-        float f0 = 0.0f, f1 = 0.0f;
-        if(l < v.levels)
-        {
-            Corners c;
-            LevelCorners(v, l, pos, c);
-            const __half2* g = reinterpret_cast<const __half2*>(v.grid) + (size_t(l) << v.log2T);
-            for(uint32_t k = 0; k < 8; k++)
-            {
-                float2 e = __half22float2(g[c.idx[k]]);
-                f0 += c.w[k] * e.x;
-                f1 += c.w[k] * e.y;
-            }
-        }
-        row[2 * l] = F2Bf(f0);
-        row[2 * l + 1] = F2Bf(f1);
-    }
-    if(half == 0)
-    {
-        // one-blob of dir.theta, dir.phi, normal.theta, normal.phi (cols 32..47)
-        for(uint32_t q = 0; q < 4; q++)
-            for(uint32_t j = 0; j < 4; j++) row[32 + 4 * q + j] = F2Bf(OneBlob(rec[3 + q], j));
-    }
-    else
-    {
-        for(uint32_t j = 0; j < 4; j++) row[48 + j] = F2Bf(OneBlob(rec[7], j));
-        row[52] = F2Bf(rec[8]);
-        row[53] = F2Bf(rec[9]);
-        row[54] = F2Bf(rec[10]);
-        row[55] = F2Bf(1.0f);
-        for(uint32_t j = 56; j < 64; j++) row[j] = 0;
-    }
+    for(int k = 0; k < 3; k++) pos[k] = ClampF(rec[k], 0.0f, 1.0f);
 }
 
-// ---- MFMA tile products ------------------------------------------------------
-// acc[nt] = X(32x64, LDS rows of kLdsRow) * B, where the operand for output
-// column n and reduction index k is bRow(n)[k] (4 consecutive k per lane).
-__device__ __forceinline__ void TileProduct(const uint16_t* sA, const uint16_t* sB, v16f acc[2])
+// Interpolated features of one level, corners summed in order.  The two corners
+// along x are one entry apart in the low index bits, so an aligned 16-byte
+// load of four entries brings both unless x mod 4 is 3: 5 gathers per 4 pairs
+// instead of 8 (QUADS; otherwise 8 single gathers).
+template<bool QUADS>
+__device__ __forceinline__ uint32_t LevelFeatures(const uint32_t* __restrict__ table, const float pos[3],
+                                                  float scale, uint32_t my, uint32_t mz, uint32_t dense,
+                                                  uint32_t mask)
 {
-    // v_mfma_f32_32x32x16_bf16: lane l supplies row (l mod 32) of A and
-    // column (l mod 32) of B over k = 8 (l / 32) .. +7 of the 16-k step
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t r = lane & 31u, kh = (lane >> 5) * 8u;
-    acc[0] = v16f{0};
-    acc[1] = v16f{0};
+    const Cell c = LevelCell(pos, scale, my, mz);
+    uint4 quad[4];
+    uint32_t i0[4], i1[4], e0[4], e1[4];
     #pragma unroll
-    for(uint32_t kt = 0; kt < kW / 16u; kt++)
+    for(uint32_t q = 0; q < 4; q++)
     {
-        const uint32_t k = kt * 16u + kh;
-        v8bf a = *reinterpret_cast<const v8bf*>(sA + r * kLdsRow + k);
-        v8bf b0 = *reinterpret_cast<const v8bf*>(sB + r * kLdsRow + k);
-        v8bf b1 = *reinterpret_cast<const v8bf*>(sB + (r + 32u) * kLdsRow + k);
-        acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b0, acc[0], 0, 0, 0);
-        acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b1, acc[1], 0, 0, 0);
+        const uint32_t y = c.y + ((q & 1u) ? my : 0u), z = c.z + ((q & 2u) ? mz : 0u);
+        i0[q] = GridIndex(dense, mask, c.x, y, z);
+        i1[q] = GridIndex(dense, mask, c.x + 1u, y, z);
+        if constexpr(QUADS)
+        {
+            quad[q] = *reinterpret_cast<const uint4*>(table + (i0[q] & ~3u));
+            e1[q] = 0u;
+            if((i0[q] ^ i1[q]) > 3u) e1[q] = table[i1[q]];
+        }
+        else
+        {
+            e0[q] = table[i0[q]];
+            e1[q] = table[i1[q]];
+        }
     }
-}
-
-// Row of accumulator element e for this lane (32x32 output layout).
-__device__ __forceinline__ uint32_t AccRow(uint32_t e)
-{
-    const uint32_t lane = threadIdx.x & 63u;
-    return 8u * (e >> 2) + 4u * (lane >> 5) + (e & 3u);
-}
-
-__device__ __forceinline__ void StageWeights(const uint16_t* __restrict__ g, uint16_t* s)
-{
-    // [6][64][64] -> padded LDS rows
-    for(uint32_t i = threadIdx.x; i < kNrcLayers * kW * kW / 4u; i += blockDim.x)
+    float f0 = 0.0f, f1 = 0.0f;
+    #pragma unroll
+    for(uint32_t q = 0; q < 4; q++)
     {
-        uint32_t e = i * 4u;
-        uint32_t row = e / kW, col = e % kW;
-        *reinterpret_cast<uint2*>(s + row * kLdsRow + col) = reinterpret_cast<const uint2*>(g)[i];
+        auto pick = [&](uint32_t i)
+        {
+            const uint32_t lo = (i & 2u) ? quad[q].z : quad[q].x, hi = (i & 2u) ? quad[q].w : quad[q].y;
+            return (i & 1u) ? hi : lo;
+        };
+        if constexpr(QUADS)
+        {
+            e0[q] = pick(i0[q]);
+            if((i0[q] ^ i1[q]) <= 3u) e1[q] = pick(i1[q]);
+        }
+        #pragma unroll
+        for(uint32_t k = 0; k < 2; k++)
+        {
+            const float w = CornerWeight(c, 2u * q + k);
+            const float2 g = __half22float2(__builtin_bit_cast(__half2, k ? e1[q] : e0[q]));
+            f0 += w * g.x;
+            f1 += w * g.y;
+        }
     }
+    return PackBf(f0, f1);
 }
 
-// ---- forward ---------------------------------------------------------------
-struct NrcTrainBuf
+// Words 8..13 of half h's operand: one-blobs h and 2 + h, then its share of
+// the last 16 columns (words 14 and 15 are zero).
+__device__ __forceinline__ void EncodeTail(const float* __restrict__ rec, bool hi, XRow& x)
 {
-    uint16_t* x;       // [6][B][64] bf16 layer inputs
-    uint16_t* dz;      // [6][B][64] bf16 gradients of the layer outputs
-    float* dy;         // [B][3]
-    float* dx0;        // [B][32]
-    float* loss;       // [1]
-};
+    const float qa = hi ? rec[4] : rec[3], qb = hi ? rec[6] : rec[5], r7 = rec[7];
+    x.u[8] = PackBf(OneBlob(qa, 0), OneBlob(qa, 1));
+    x.u[9] = PackBf(OneBlob(qa, 2), OneBlob(qa, 3));
+    x.u[10] = PackBf(OneBlob(qb, 0), OneBlob(qb, 1));
+    x.u[11] = PackBf(OneBlob(qb, 2), OneBlob(qb, 3));
+    x.u[12] = hi ? PackBf(rec[8], rec[9]) : PackBf(OneBlob(r7, 0), OneBlob(r7, 1));
+    x.u[13] = hi ? PackBf(rec[10], 1.0f) : PackBf(OneBlob(r7, 2), OneBlob(r7, 3));
+    x.u[14] = 0u;
+    x.u[15] = 0u;
+}
 
-template<bool TRAIN>
-__global__ void __launch_bounds__(kFwdWaves * 64)
-KNrcForward(NrcView v, const float* __restrict__ rec, const uint32_t* __restrict__ dCount,
-            uint32_t count, float* __restrict__ out, const float* __restrict__ target,
-            NrcTrainBuf tb, uint32_t batch)
+// Word m of an operand holds level LevelOfWord(m) in the lower half of the
+// wave and that level plus 2 in the upper.
+__device__ constexpr uint32_t LevelOfWord(uint32_t m) { return 4u * (m >> 1) + (m & 1u); }
+
+// Operand of sample (lane mod 32), two lanes per sample: each takes the 8
+// levels its words hold.  Both halves run one instruction stream: a step's
+// two levels' constants are picked per half from scalar registers.
+// QUADS = false issues 8 independent gathers per level and has no branch, so
+// that the gathers of several levels are in flight together: for kernels with
+// few waves, where latency counts and not the gather rate.
+template<bool QUADS>
+__device__ __forceinline__ XRow EncodePair(const NrcView& v, const float* __restrict__ rec, const float pos[3])
 {
-    __shared__ __attribute__((aligned(16))) uint16_t sW[kNrcLayers * kW * kLdsRow];
-    __shared__ __attribute__((aligned(16))) uint16_t sX[kFwdWaves][32 * kLdsRow];
+    const bool hi = (threadIdx.x & 32u) != 0u;
+    const uint32_t mask = (1u << v.log2T) - 1u;
+    const uint32_t* __restrict__ grid = reinterpret_cast<const uint32_t*>(v.grid);
+    XRow x;
+    #pragma unroll
+    for(uint32_t m = 0; m < 8; m++)
+    {
+        // levels past the last read the last one and are dropped
+        const uint32_t la = LevelOfWord(m), lb = la + 2u;
+        x.u[m] = 0u;
+        if(QUADS && la >= v.levels) continue;
+        const uint32_t ra = min(la, v.levels - 1u), rb = min(lb, v.levels - 1u);
+        const uint32_t f = LevelFeatures<QUADS>(grid + (size_t(hi ? rb : ra) << v.log2T), pos,
+                                                hi ? v.scale[rb] : v.scale[ra], hi ? v.my[rb] : v.my[ra],
+                                                hi ? v.mz[rb] : v.mz[ra], hi ? v.dense[rb] : v.dense[ra], mask);
+        x.u[m] = ((hi ? lb : la) < v.levels) ? f : 0u;
+    }
+    EncodeTail(rec, hi, x);
+    return x;
+}
+
+// ---- inference ---------------------------------------------------------------
+// A tile's six layers and its three outputs.
+__device__ __forceinline__ void InferLayers(const uint4* sW, XRow& x, float* __restrict__ out, size_t s, size_t n)
+{
+    v16f acc[2];
+    #pragma unroll 1
+    for(uint32_t l = 0; l + 1u < kNrcLayers; l++)
+    {
+        LayerProduct<2, 4>(sW + l * kFragLayer, x, acc);
+        x = ReluPack(acc);
+    }
+    LayerProduct<1, 4>(sW + (kNrcLayers - 1u) * kFragLayer, x, acc);
+    if((threadIdx.x & 32u) == 0u && s < n)
+        for(uint32_t c = 0; c < 3; c++) out[s * 3u + c] = acc[0][c];
+}
+
+__device__ __forceinline__ void StageWeights(const NrcView& v, uint4* sW)
+{
+    for(uint32_t i = threadIdx.x; i < kNrcLayers * kFragLayer; i += kInferTPB)
+        sW[i] = reinterpret_cast<const uint4*>(v.wT)[i];
+    __syncthreads();
+}
+
+// Persistent waves over 32-query tiles, weights staged once per block (48 KiB
+// in fragment order).  Bound by the grid gathers, not by the products.
+__global__ void __launch_bounds__(kInferTPB)
+KNrcInfer(NrcView v, const float* __restrict__ rec, const uint32_t* __restrict__ dCount, uint32_t count,
+          float* __restrict__ out)
+{
+    __shared__ uint4 sW[kNrcLayers * kFragLayer];
     const uint32_t n = dCount ? *dCount : count;
+    constexpr uint32_t kWaves = kInferTPB / 64u;
     // a block without a tile (few or no queries this bounce) skips the
     // weight staging: the test is uniform over the block
-    if(blockIdx.x * kFwdWaves * 32u >= n) return;
-    StageWeights(v.wT, sW);
-    __syncthreads();
+    if(size_t(blockIdx.x) * kWaves * 32u >= n) return;
+    StageWeights(v, sW);
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    uint16_t* X = sX[wave];
-    float lossAcc = 0.0f;
-    for(uint32_t tile = blockIdx.x * kFwdWaves + wave; tile * 32u < n; tile += gridDim.x * kFwdWaves)
+    for(size_t tile = blockIdx.x * kWaves + wave; tile * 32u < n; tile += gridDim.x * kWaves)
     {
-        const uint32_t base = tile * 32u;
-        // encode: lane -> (sample lane%32, half lane/32)
-        {
-            const uint32_t s = base + (lane & 31u);
-            uint16_t* row = X + (lane & 31u) * kLdsRow;
-            if(s < n) EncodeHalf(v, rec + size_t(s) * 11u, lane >> 5, row);
-            else
-                for(uint32_t j = (lane >> 5) * 32u; j < (lane >> 5) * 32u + 32u; j++) row[j] = 0;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        for(uint32_t l = 0; l < kNrcLayers; l++)
-        {
-            if(TRAIN)
-            {
-                // store this layer's input rows (32 x 64 bf16)
-                for(uint32_t e = lane; e < 32u * 16u; e += 64u)
-                {
-                    uint32_t rr = e >> 4, c4 = (e & 15u) * 4u;
-                    uint32_t s = base + rr;
-                    if(s < n)
-                        *reinterpret_cast<uint2*>(tb.x + (size_t(l) * batch + s) * kW + c4) =
-                            *reinterpret_cast<const uint2*>(X + rr * kLdsRow + c4);
-                }
-            }
-            v16f acc[2];
-            TileProduct(X, sW + l * kW * kLdsRow, acc);
-            __builtin_amdgcn_wave_barrier();
-            if(l + 1u < kNrcLayers)
-            {
-                #pragma unroll
-                for(uint32_t t = 0; t < 2; t++)
-                    #pragma unroll
-                    for(uint32_t e = 0; e < 16; e++)
-                        X[AccRow(e) * kLdsRow + t * 32u + (lane & 31u)] = F2Bf(MaxF(acc[t][e], 0.0f));
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            }
-            else
-            {
-                // output columns 0..2 live in lanes 0..2 and 32..34 of tile 0
-                const uint32_t c = lane & 31u;
-                if(c < 3u)
-                {
-                    #pragma unroll
-                    for(uint32_t e = 0; e < 16; e++)
-                    {
-                        uint32_t s = base + AccRow(e);
-                        if(s >= n) continue;
-                        float y = acc[0][e];
-                        if(!TRAIN) out[size_t(s) * 3u + c] = y;
-                        else
-                        {
-                            float t = target[size_t(s) * 3u + c];
-                            float den = y * y + 0.01f;
-                            float d = y - t;
-                            lossAcc += d * d / den;
-                            tb.dy[size_t(s) * 3u + c] = 2.0f * d / den / float(batch * 3u);
-                        }
-                    }
-                }
-            }
-        }
-    }
-    if(TRAIN)
-    {
-        for(uint32_t o = 32; o > 0; o >>= 1) lossAcc += __shfl_down(lossAcc, o);
-        if(lane == 0 && lossAcc != 0.0f) atomicAdd(tb.loss, lossAcc / float(batch * 3u));
+        // lanes past the last query repeat it and write nothing
+        const size_t s = tile * 32u + (lane & 31u);
+        const float* r = rec + min(s, size_t(n) - 1u) * 11u;
+        float pos[3];
+        RecordPos(r, pos);
+        XRow x = EncodePair<true>(v, r, pos);
+        InferLayers(sW, x, out, s, n);
     }
 }
 
-// ---- backward (data gradients) ----------------------------------------------
-__global__ void __launch_bounds__(kFwdWaves * 64)
-KNrcBackward(NrcView v, NrcTrainBuf tb, uint32_t batch)
+// ---- training: forward and data gradients -----------------------------------
+struct NrcTrainBuf
 {
-    __shared__ __attribute__((aligned(16))) uint16_t sW[kNrcLayers * kW * kLdsRow];
-    __shared__ __attribute__((aligned(16))) uint16_t sG[kFwdWaves][32 * kLdsRow];
-    StageWeights(v.wK, sW);
-    __syncthreads();
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    uint16_t* G = sG[wave];
-    for(uint32_t tile = blockIdx.x * kFwdWaves + wave; tile * 32u < batch; tile += gridDim.x * kFwdWaves)
-    {
-        const uint32_t base = tile * 32u;
-        // dZ of the output layer: dL/dy in columns 0..2, zero elsewhere
-        for(uint32_t e = lane; e < 32u * kW; e += 64u)
-        {
-            uint32_t rr = e / kW, c = e % kW;
-            uint32_t s = base + rr;
-            float g = (c < 3u && s < batch) ? tb.dy[size_t(s) * 3u + c] : 0.0f;
-            G[rr * kLdsRow + c] = F2Bf(g);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        for(int l = int(kNrcLayers) - 1; l >= 0; l--)
-        {
-            // keep dZ_{l+1} for the weight gradient of layer l
-            for(uint32_t e = lane; e < 32u * 16u; e += 64u)
-            {
-                uint32_t rr = e >> 4, c4 = (e & 15u) * 4u;
-                uint32_t s = base + rr;
-                if(s < batch)
-                    *reinterpret_cast<uint2*>(tb.dz + (size_t(l) * batch + s) * kW + c4) =
-                        *reinterpret_cast<const uint2*>(G + rr * kLdsRow + c4);
-            }
-            v16f acc[2];
-            // dX = dZ * W^T: output column k, reduction over n -> W[k][n] rows
-            TileProduct(G, sW + uint32_t(l) * kW * kLdsRow, acc);
-            __builtin_amdgcn_wave_barrier();
-            if(l > 0)
-            {
-                // ReLU of layer l-1's output = this layer's input X_l
-                #pragma unroll
-                for(uint32_t t = 0; t < 2; t++)
-                    #pragma unroll
-                    for(uint32_t e = 0; e < 16; e++)
-                    {
-                        uint32_t rr = AccRow(e), c = t * 32u + (lane & 31u);
-                        uint32_t s = base + rr;
-                        float xin = (s < batch) ? Bf2F(tb.x[(size_t(l) * batch + s) * kW + c]) : 0.0f;
-                        G[rr * kLdsRow + c] = F2Bf(xin > 0.0f ? acc[t][e] : 0.0f);
-                    }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            }
-            else
-            {
-                // gradient of the 32 grid features
-                #pragma unroll
-                for(uint32_t e = 0; e < 16; e++)
-                {
-                    uint32_t s = base + AccRow(e);
-                    if(s < batch) tb.dx0[size_t(s) * 32u + (lane & 31u)] = acc[0][e];
-                }
-            }
-        }
-    }
-}
+    uint32_t* x;       // [6][B/32][64 features][32 samples] bf16 layer inputs
+    uint32_t* dz;      // the same for the gradients of the layer outputs
+    float2* dx0;       // [16 levels][B] gradient of the grid features
+    float* pos;        // [3][B] clamped positions
+    float* loss;       // [B/32] each tile's part of the loss
+};
 
-// ---- weight gradients -------------------------------------------------------
-// blockIdx.y = layer; each block reduces a chunk of samples; wave w owns the
-// 32x32 tile (w/2, w%2) of dW[k][n] = sum_s X[s][k] dZ[s][n].
-__global__ void __launch_bounds__(256)
-KNrcWgrad(NrcTrainBuf tb, uint32_t batch, uint32_t chunk, float* __restrict__ wgrad)
+// Stores packed features (word q of XRow: q and q + 1 of the lane's sample)
+// with the samples contiguous: neighbouring lanes swap a feature, so each lane
+// writes two samples of one feature.
+__device__ __forceinline__ void StoreTransposed(uint32_t* __restrict__ rows, const XRow& x, uint32_t words)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t sXc[64 * kLdsRow];
-    __shared__ __attribute__((aligned(16))) uint16_t sGc[64 * kLdsRow];
-    const uint32_t l = blockIdx.y;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t mt = wave >> 1, nt = wave & 1u;
-    const uint32_t s0 = blockIdx.x * chunk;
-    const uint32_t s1 = min(batch, s0 + chunk);
-    v16f acc = v16f{0};
-    for(uint32_t sb = s0; sb < s1; sb += 64u)
-    {
-        for(uint32_t e = threadIdx.x; e < 64u * 16u; e += 256u)
-        {
-            uint32_t rr = e >> 4, c4 = (e & 15u) * 4u;
-            uint32_t s = sb + rr;
-            uint2 xv = make_uint2(0, 0), gv = make_uint2(0, 0);
-            if(s < s1)
-            {
-                xv = *reinterpret_cast<const uint2*>(tb.x + (size_t(l) * batch + s) * kW + c4);
-                gv = *reinterpret_cast<const uint2*>(tb.dz + (size_t(l) * batch + s) * kW + c4);
-            }
-            *reinterpret_cast<uint2*>(sXc + rr * kLdsRow + c4) = xv;
-            *reinterpret_cast<uint2*>(sGc + rr * kLdsRow + c4) = gv;
-        }
-        __syncthreads();
-        const uint32_t kRow = mt * 32u + (lane & 31u);
-        const uint32_t nCol = nt * 32u + (lane & 31u);
-        #pragma unroll
-        for(uint32_t kt = 0; kt < 4; kt++)
-        {
-            // reduction over 16 samples per instruction: lane half h takes
-            // samples 8h .. 8h+7 of the step
-            const uint32_t sr = kt * 16u + (lane >> 5) * 8u;
-            v8bf a, b;
-            #pragma unroll
-            for(uint32_t j = 0; j < 8; j++)
-            {
-                a[j] = __builtin_bit_cast(__bf16, sXc[(sr + j) * kLdsRow + kRow]);
-                b[j] = __builtin_bit_cast(__bf16, sGc[(sr + j) * kLdsRow + nCol]);
-            }
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    float* g = wgrad + size_t(l) * kLayerParams;
+    const uint32_t lane = threadIdx.x & 63u, h = lane >> 5, s = lane & 31u, odd = s & 1u;
+    const uint32_t sel = odd ? 0x03020706u : 0x05040100u;
     #pragma unroll
-    for(uint32_t e = 0; e < 16; e++)
+    for(uint32_t q = 0; q < 16; q++)
     {
-        uint32_t k = mt * 32u + AccRow(e);
-        uint32_t nn = nt * 32u + (lane & 31u);
-        if(acc[e] != 0.0f) atomicAdd(g + k * kW + nn, acc[e]);
+        if(q >= words) break;
+        const uint32_t i = q & 7u;
+        const uint32_t f = 32u * (q >> 3) + 8u * (i >> 1) + 4u * h + 2u * (i & 1u) + odd;
+        const uint32_t other = uint32_t(__builtin_amdgcn_update_dpp(0, int(x.u[q]), 0xB1, 0xF, 0xF, true));
+        rows[f * 16u + (s >> 1)] = __builtin_amdgcn_perm(other, x.u[q], sel);
+    }
+}
+
+// One wave per 32 samples, everything in registers; weights come straight from
+// L2 in fragment order (a training batch is about two waves per CU, so staging
+// them in LDS would cost more than the products): batch 16384: 23 us,
+// from 53 + 55 us as two LDS-staged kernels.
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2)))
+KNrcTrain(NrcView v, const float* __restrict__ rec, const float* __restrict__ target, NrcTrainBuf tb,
+          uint32_t batch)
+{
+    const uint32_t lane = threadIdx.x & 63u, tiles = batch / 32u, tile = blockIdx.x;
+    const uint32_t s = tile * 32u + (lane & 31u);
+    const float* r = rec + size_t(s) * 11u;
+    const uint4* __restrict__ wT = reinterpret_cast<const uint4*>(v.wT);
+    const uint4* __restrict__ wK = reinterpret_cast<const uint4*>(v.wK);
+    float pos[3];
+    RecordPos(r, pos);
+    if(lane < 32u)
+        for(uint32_t k = 0; k < 3; k++) tb.pos[size_t(k) * batch + s] = pos[k];
+    auto rows = [&](uint32_t* base, uint32_t l) { return base + (size_t(l) * tiles + tile) * 64u * 16u; };
+    XRow x[kNrcLayers];
+    v16f acc[2];
+    // each layer's weights are loaded while the layer before it is computed
+    Frags w = LoadFrags(wT);
+    x[0] = EncodePair<false>(v, r, pos);
+    #pragma unroll
+    for(uint32_t l = 0; l + 1u < kNrcLayers; l++)
+    {
+        const Frags next = LoadFrags(wT + (l + 1u) * kFragLayer);
+        StoreTransposed(rows(tb.x, l), x[l], 16);
+        LayerProduct<2, 4>(w, x[l], acc);
+        x[l + 1] = ReluPack(acc);
+        w = next;
+    }
+    {
+        const Frags next = LoadFrags(wK + (kNrcLayers - 1u) * kFragLayer);
+        StoreTransposed(rows(tb.x, kNrcLayers - 1u), x[kNrcLayers - 1], 16);
+        LayerProduct<1, 4>(w, x[kNrcLayers - 1], acc);
+        w = next;
+    }
+    // relative L2 loss and its gradient: outputs 0..2 sit in the lower half
+    float loss = 0.0f, dy[3] = {0.0f, 0.0f, 0.0f};
+    if(lane < 32u)
+        for(uint32_t c = 0; c < 3; c++)
+        {
+            const float y = acc[0][c], d = y - target[size_t(s) * 3u + c], den = y * y + 0.01f;
+            loss += d * d / den;
+            dy[c] = 2.0f * d / den / float(batch * 3u);
+        }
+    for(uint32_t o = 32; o > 0; o >>= 1) loss += __shfl_down(loss, o);
+    if(lane == 0) tb.loss[tile] = loss / float(batch * 3u);
+    XRow g;
+    for(uint32_t q = 0; q < 16; q++) g.u[q] = 0u;
+    g.u[0] = PackBf(dy[0], dy[1]);
+    g.u[1] = PackBf(dy[2], 0.0f);
+    // the output layer's gradient has 3 rows; its weight tile reads 16
+    StoreTransposed(rows(tb.dz, kNrcLayers - 1u), g, 4);
+    #pragma unroll
+    for(uint32_t l = kNrcLayers - 1u; l > 0u; l--)
+    {
+        // dX = W dZ, then the ReLU that produced X
+        const Frags next = LoadFrags(wK + (l - 1u) * kFragLayer);
+        if(l == kNrcLayers - 1u) LayerProduct<2, 1>(w, g, acc);
+        else LayerProduct<2, 4>(w, g, acc);
+        w = next;
+        #pragma unroll
+        for(uint32_t q = 0; q < 16; q++)
+        {
+            const uint32_t in = x[l].u[q], t = q >> 3, i = q & 7u;
+            g.u[q] = PackBf((in & 0xFFFFu) ? acc[t][2 * i] : 0.0f, (in >> 16) ? acc[t][2 * i + 1] : 0.0f);
+        }
+        StoreTransposed(rows(tb.dz, l - 1u), g, 16);
+    }
+    // gradient of the 32 grid features: rows 2 level, 2 level + 1
+    LayerProduct<1, 4>(w, g, acc);
+    #pragma unroll
+    for(uint32_t i = 0; i < 8; i++)
+    {
+        const uint32_t level = 4u * (i >> 1) + 2u * (lane >> 5) + (i & 1u);
+        tb.dx0[size_t(level) * batch + s] = make_float2(acc[0][2 * i], acc[0][2 * i + 1]);
     }
 }
 
 // ---- grid gradients -----------------------------------------------------------
 // One thread per (sample, level): the 16 atomics of a level's 8 corners.
 __global__ void __launch_bounds__(256)
-KNrcGridBwd(NrcView v, const float* __restrict__ rec, const float* __restrict__ dx0,
-            uint32_t batch, float* __restrict__ ggrad)
+KNrcGridBwd(NrcView v, NrcTrainBuf tb, uint32_t batch, float* __restrict__ ggrad)
 {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t s = t / v.levels, l = t % v.levels;
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x, l = blockIdx.y;
     if(s >= batch) return;
-    const float g0 = dx0[size_t(s) * 32u + 2u * l], g1 = dx0[size_t(s) * 32u + 2u * l + 1u];
-    if(g0 == 0.0f && g1 == 0.0f) return;
-    const float* r = rec + size_t(s) * 11u;
-    float pos[3] = {ClampF(r[0], 0.0f, 1.0f), ClampF(r[1], 0.0f, 1.0f), ClampF(r[2], 0.0f, 1.0f)};
-    Corners c;
-    LevelCorners(v, l, pos, c);
+    const float2 g = tb.dx0[size_t(l) * batch + s];
+    if(g.x == 0.0f && g.y == 0.0f) return;
+    const float pos[3] = {tb.pos[s], tb.pos[batch + s], tb.pos[2 * size_t(batch) + s]};
+    const Cell c = LevelCell(pos, v.scale[l], v.my[l], v.mz[l]);
     float* gl = ggrad + (size_t(l) << v.log2T) * 2u;
     for(uint32_t k = 0; k < 8; k++)
     {
-        atomicAdd(gl + size_t(c.idx[k]) * 2u, c.w[k] * g0);
-        atomicAdd(gl + size_t(c.idx[k]) * 2u + 1u, c.w[k] * g1);
+        const size_t i = GridIndex(v.dense[l], (1u << v.log2T) - 1u, c.x + (k & 1u),
+                                   c.y + ((k & 2u) ? v.my[l] : 0u), c.z + ((k & 4u) ? v.mz[l] : 0u));
+        const float w = CornerWeight(c, k);
+        atomicAdd(gl + i * 2u, w * g.x);
+        atomicAdd(gl + i * 2u + 1u, w * g.y);
     }
 }
 
@@ -472,52 +513,227 @@ __device__ __forceinline__ float AdamOne(float& p, float& m, float& vv, float& g
     return p;
 }
 
-__global__ void __launch_bounds__(256)
-KNrcAdamMlp(float* __restrict__ w, float* __restrict__ m, float* __restrict__ vv,
-            float* __restrict__ g, uint16_t* __restrict__ wT, uint16_t* __restrict__ wK, AdamArgs a)
+// One MLP parameter's update: columns past the three outputs stay zero.
+struct MlpAdam
 {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= kMlpParams) return;
-    uint32_t l = i / kLayerParams, e = i % kLayerParams, k = e / kW, n = e % kW;
-    float p = w[i], mm = m[i], v2 = vv[i], gg = g[i];
-    if(l == kNrcLayers - 1u && n >= 3u) { p = 0.0f; gg = 0.0f; }
-    AdamOne(p, mm, v2, gg, a);
-    if(l == kNrcLayers - 1u && n >= 3u) p = 0.0f;
-    w[i] = p; m[i] = mm; vv[i] = v2; g[i] = 0.0f;
-    uint16_t b = F2Bf(p);
-    wK[i] = b;
-    wT[l * kLayerParams + n * kW + k] = b;
+    float* w;
+    float* m;
+    float* v;
+    uint16_t* wT;
+    uint16_t* wK;
+};
+__device__ __forceinline__ void StoreWeight(uint16_t* wT, uint16_t* wK, uint32_t l, uint32_t k, uint32_t n, float p)
+{
+    const uint16_t b = F2Bf(p);
+    wT[FragIndex(l, n, k)] = b;
+    wK[FragIndex(l, k, n)] = b;
+}
+__device__ __forceinline__ void AdamWeight(const MlpAdam& u, uint32_t i, float g, const AdamArgs& a)
+{
+    const uint32_t l = i / kLayerParams, e = i % kLayerParams, k = e / kW, n = e % kW;
+    const bool unused = l == kNrcLayers - 1u && n >= 3u;
+    float p = u.w[i], m = u.m[i], v = u.v[i];
+    if(unused) { p = 0.0f; g = 0.0f; }
+    AdamOne(p, m, v, g, a);
+    if(unused) p = 0.0f;
+    u.w[i] = p; u.m[i] = m; u.v[i] = v;
+    StoreWeight(u.wT, u.wK, l, k, n, p);
 }
 
-// Four parameters per thread (count is a multiple of 4).  LAZY: entries
-// with a zero gradient keep parameter and moments, and are not written.
+__global__ void __launch_bounds__(256)
+KNrcAdamMlp(MlpAdam u, float* __restrict__ g, AdamArgs a)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if(i >= kMlpParams) return;
+    const float gg = g[i];
+    g[i] = 0.0f;
+    AdamWeight(u, i, gg, a);
+}
+
+// ---- weight gradients -------------------------------------------------------
+// One block per 16 x 16 tile of dW[k][n] = sum_s X[s][k] dZ[s][n]: its 16 waves
+// take every 16th sample tile (one v_mfma_f32_16x16x32_bf16 each; with samples
+// contiguous both operands are 1 KiB contiguous loads) and are summed through
+// LDS in wave order, so there are no atomics and the sum is deterministic.
+// ADAM: the block also updates its 256 parameters (wgrad must be clear).
+// Bound by L2 reads (each operand tile is read by four blocks): 17 us a batch of
+// 16384 (17.9 with atomics and LDS transposes, plus the MLP's Adam pass, 4.9).
+constexpr uint32_t kWgradWaves = 16;
+constexpr uint32_t kWgradBlocks = 8u * 16u;   // an XCD per layer, two of them idle
+typedef float v4f __attribute__((ext_vector_type(4)));
+template<bool ADAM>
+__global__ void __launch_bounds__(kWgradWaves * 64)
+KNrcWgrad(NrcTrainBuf tb, uint32_t batch, float* __restrict__ wgrad, MlpAdam u, AdamArgs a)
+{
+    __shared__ float part[kWgradWaves][256];
+    // workgroups go round-robin over the 8 XCDs: a layer's 16 tiles share an L2
+    const uint32_t l = blockIdx.x & 7u, kt = blockIdx.x >> 5, nt = (blockIdx.x >> 3) & 3u;
+    if(l >= kNrcLayers) return;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, tiles = batch / 32u;
+    v4f acc = v4f{0};
+    // outputs past the third have no gradient (and none is stored)
+    const bool live = l + 1u < kNrcLayers || nt == 0u;
+    if(live)
+    {
+        // lane (r, q): row r of the tile, samples 8 q .. 8 q + 7
+        const uint32_t at = (lane & 15u) * 4u + (lane >> 4);
+        const uint4* __restrict__ X = reinterpret_cast<const uint4*>(tb.x) + size_t(l) * tiles * 256u + kt * 64u + at;
+        const uint4* __restrict__ G = reinterpret_cast<const uint4*>(tb.dz) + size_t(l) * tiles * 256u + nt * 64u + at;
+        constexpr uint32_t kAhead = 8;       // tiles whose loads are in flight together
+        for(uint32_t t = wave; t < tiles; t += kAhead * kWgradWaves)
+        {
+            uint4 xv[kAhead], gv[kAhead];
+            #pragma unroll
+            for(uint32_t j = 0; j < kAhead; j++)
+            {
+                // past the last tile: that one again, as zeros
+                const uint32_t tj = t + j * kWgradWaves, tr = min(tj, tiles - 1u);
+                xv[j] = X[size_t(tr) * 256u];
+                gv[j] = G[size_t(tr) * 256u];
+                if(tj != tr) xv[j] = gv[j] = make_uint4(0u, 0u, 0u, 0u);
+            }
+            #pragma unroll
+            for(uint32_t j = 0; j < kAhead; j++)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, xv[j]),
+                                                              __builtin_bit_cast(v8bf, gv[j]), acc, 0, 0, 0);
+        }
+    }
+    // lane (c, q) holds column c, rows 4 q .. 4 q + 3
+    for(uint32_t e = 0; e < 4; e++) part[wave][(4u * (lane >> 4) + e) * 16u + (lane & 15u)] = acc[e];
+    __syncthreads();
+    if(threadIdx.x >= 256u) return;
+    float g = 0.0f;
+    for(uint32_t w = 0; w < kWgradWaves; w++) g += part[w][threadIdx.x];
+    const uint32_t k = kt * 16u + (threadIdx.x >> 4), n = nt * 16u + (threadIdx.x & 15u);
+    const uint32_t i = l * kLayerParams + k * kW + n;
+    if constexpr(ADAM) AdamWeight(u, i, g, a);
+    else if(live && g != 0.0f) wgrad[i] += g;
+}
+
+// Grid parameters, four at a time (two table entries).  LAZY: entries with a
+// zero gradient keep parameter and moments, and are not written.
+struct GridAdam
+{
+    float* p;
+    float* m;
+    float* v;
+    __half* h;
+};
+template<bool LAZY>
+__device__ __forceinline__ void AdamGrid4(const GridAdam& u, size_t i, float4 g4, const AdamArgs& a)
+{
+    if(LAZY && g4.x == 0.0f && g4.y == 0.0f && g4.z == 0.0f && g4.w == 0.0f) return;
+    float4 p4 = reinterpret_cast<const float4*>(u.p)[i];
+    float4 m4 = reinterpret_cast<const float4*>(u.m)[i];
+    float4 v4 = reinterpret_cast<const float4*>(u.v)[i];
+    float* pp = &p4.x;
+    float* mm = &m4.x;
+    float* v2 = &v4.x;
+    float* gg = &g4.x;
+    #pragma unroll
+    for(int k = 0; k < 4; k++)
+        if(!LAZY || gg[k] != 0.0f) AdamOne(pp[k], mm[k], v2[k], gg[k], a);
+    reinterpret_cast<float4*>(u.p)[i] = p4;
+    reinterpret_cast<float4*>(u.m)[i] = m4;
+    reinterpret_cast<float4*>(u.v)[i] = v4;
+    reinterpret_cast<__half2*>(u.h)[2 * i] = __floats2half2_rn(p4.x, p4.y);
+    reinterpret_cast<__half2*>(u.h)[2 * i + 1] = __floats2half2_rn(p4.z, p4.w);
+}
+
 template<bool LAZY>
 __global__ void __launch_bounds__(256)
-KNrcAdamGrid(float* __restrict__ p, float* __restrict__ m, float* __restrict__ vv,
-             float* __restrict__ g, __half* __restrict__ h, size_t count, AdamArgs a)
+KNrcAdamGrid(GridAdam u, float* __restrict__ g, size_t count, AdamArgs a)
 {
     const size_t n4 = count / 4u;
     size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
     for(; i < n4; i += size_t(gridDim.x) * blockDim.x)
     {
-        float4 g4 = reinterpret_cast<const float4*>(g)[i];
+        const float4 g4 = reinterpret_cast<const float4*>(g)[i];
         if(LAZY && g4.x == 0.0f && g4.y == 0.0f && g4.z == 0.0f && g4.w == 0.0f) continue;
-        float4 p4 = reinterpret_cast<const float4*>(p)[i];
-        float4 m4 = reinterpret_cast<const float4*>(m)[i];
-        float4 v4 = reinterpret_cast<const float4*>(vv)[i];
-        float* pp = &p4.x;
-        float* mm = &m4.x;
-        float* v2 = &v4.x;
-        float* gg = &g4.x;
-        for(int k = 0; k < 4; k++)
-            if(!LAZY || gg[k] != 0.0f) AdamOne(pp[k], mm[k], v2[k], gg[k], a);
-        reinterpret_cast<float4*>(p)[i] = p4;
-        reinterpret_cast<float4*>(m)[i] = m4;
-        reinterpret_cast<float4*>(vv)[i] = v4;
         reinterpret_cast<float4*>(g)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        __half2 h01 = __floats2half2_rn(p4.x, p4.y), h23 = __floats2half2_rn(p4.z, p4.w);
-        reinterpret_cast<__half2*>(h)[2 * i] = h01;
-        reinterpret_cast<__half2*>(h)[2 * i + 1] = h23;
+        AdamGrid4<LAZY>(u, i, g4, a);
+    }
+}
+
+// Grid gradient by segments: a block owns kSegEntries entries of one level in
+// LDS, scans every sample of the batch for corners that fall inside (an index
+// costs a few integer operations, a global float atomic into a table that no
+// L2 holds about 0.05 ns of the whole chip), adds them with LDS atomics and
+// then either adds the segment to the gradient buffer or, in a training step,
+// runs Adam on it, so that the gradient never goes to memory.
+// 8192 entries: 64 KiB of LDS, two workgroups per CU; a level has at least 32
+// segments, because a small level's corners all fall into its few entries.
+// 16384 samples, 16 levels of 2^19: 83 us with Adam (its parameters and
+// moments, 26 B each, take 61 us at the card's copy rate), from 245 us of
+// atomics and 97 us of Adam; with one segment for each small level 336 us.
+constexpr uint32_t kSegEntries = 8192;
+constexpr uint32_t kSegMinPerLevel = 32;
+constexpr uint32_t kOwnerTPB = 1024;
+// Segments of one level up to which the scan is the faster way: it costs
+// every sample about 4 ps a segment, the 16 atomics about 0.8 ns.
+constexpr uint32_t kOwnerMaxSegs = 128;
+struct OwnerLevels
+{
+    uint32_t first[kNrcMaxLevels + 1];   // first block of each level
+    uint32_t used[kNrcMaxLevels];        // entries an index can reach
+    uint32_t size[kNrcMaxLevels];        // entries of a segment (even)
+};
+enum : int { OWNER_ADD = 0, OWNER_ADAM = 1, OWNER_LAZY = 2 };
+template<int MODE>
+__global__ void __launch_bounds__(kOwnerTPB)
+KNrcGridOwner(NrcView v, NrcTrainBuf tb, uint32_t batch, OwnerLevels ol, float* __restrict__ ggrad,
+              GridAdam u, AdamArgs a)
+{
+    __shared__ __attribute__((aligned(16))) float seg[kSegEntries * 2u];
+    uint32_t l = 0;
+    while(blockIdx.x >= ol.first[l + 1]) l++;
+    const uint32_t base = (blockIdx.x - ol.first[l]) * ol.size[l];
+    const uint32_t count = min(ol.size[l], ol.used[l] - base);
+    for(uint32_t e = threadIdx.x; e < (count + 1u) / 2u; e += kOwnerTPB)
+        reinterpret_cast<float4*>(seg)[e] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    __syncthreads();
+    const uint32_t mask = (1u << v.log2T) - 1u, dense = v.dense[l], dy = v.my[l], dz = v.mz[l];
+    const float scale = v.scale[l];
+    for(uint32_t s = threadIdx.x; s < batch; s += kOwnerTPB)
+    {
+        const float2 g = tb.dx0[size_t(l) * batch + s];
+        const float pos[3] = {tb.pos[s], tb.pos[batch + s], tb.pos[2 * size_t(batch) + s]};
+        const Cell c = LevelCell(pos, scale, dy, dz);
+        // the two corners along x differ in the low index bits only, so a
+        // pair mostly falls in or out together
+        #pragma unroll
+        for(uint32_t q = 0; q < 4; q++)
+        {
+            const uint32_t y = c.y + ((q & 1u) ? dy : 0u), z = c.z + ((q & 2u) ? dz : 0u);
+            const uint32_t i0 = GridIndex(dense, mask, c.x, y, z) - base;
+            const uint32_t i1 = GridIndex(dense, mask, c.x + 1u, y, z) - base;
+            if(min(i0, i1) >= count) continue;
+            const float w0 = CornerWeight(c, 2u * q), w1 = CornerWeight(c, 2u * q + 1u);
+            if(i0 < count)
+            {
+                atomicAdd(&seg[2u * i0], w0 * g.x);
+                atomicAdd(&seg[2u * i0 + 1u], w0 * g.y);
+            }
+            if(i1 < count)
+            {
+                atomicAdd(&seg[2u * i1], w1 * g.x);
+                atomicAdd(&seg[2u * i1 + 1u], w1 * g.y);
+            }
+        }
+    }
+    __syncthreads();
+    const size_t first = ((size_t(l) << v.log2T) + base) / 2u;      // in pairs of entries
+    for(uint32_t e = threadIdx.x; e < (count + 1u) / 2u; e += kOwnerTPB)
+    {
+        const float4 g4 = reinterpret_cast<const float4*>(seg)[e];
+        if constexpr(MODE == OWNER_ADD)
+        {
+            if(g4.x == 0.0f && g4.y == 0.0f && g4.z == 0.0f && g4.w == 0.0f) continue;
+            float4 t = reinterpret_cast<const float4*>(ggrad)[first + e];
+            t.x += g4.x; t.y += g4.y; t.z += g4.z; t.w += g4.w;
+            reinterpret_cast<float4*>(ggrad)[first + e] = t;
+        }
+        else AdamGrid4<MODE == OWNER_LAZY>(u, first + e, g4, a);
     }
 }
 
@@ -536,9 +752,7 @@ __global__ void KNrcRefresh(const float* __restrict__ w, uint16_t* __restrict__ 
     {
         uint32_t l = uint32_t(j / kLayerParams), e = uint32_t(j % kLayerParams);
         uint32_t k = e / kW, n = e % kW;
-        uint16_t b = F2Bf(w[j]);
-        wK[j] = b;
-        wT[l * kLayerParams + n * kW + k] = b;
+        StoreWeight(wT, wK, l, k, n, w[j]);
     }
     for(size_t j = i; j < gridCount; j += size_t(gridDim.x) * blockDim.x) h[j] = __float2half(grid[j]);
 }
@@ -570,8 +784,11 @@ struct MRayNrc
     NrcTrainBuf tb{};
     uint32_t maxBatch = 0;
     uint64_t step = 0;
-    float* hLoss = nullptr;       // pinned
-    uint32_t fwdBlocks = 0;
+    uint32_t inferBlocks = 0;     // resident inference blocks
+    uint32_t lossTiles = 0;       // tiles of the last backward pass
+    bool gradsClear = true;       // no backward pass since the last Adam or clear
+    OwnerLevels owner{};
+    uint32_t ownerSegs = 0;       // segments of the largest level
     // per-kernel timing (mray_nrc_set_profiling): event pairs around each
     // launch, harvested by mray_nrc_kernel_times
     bool profiling = false;
@@ -639,16 +856,28 @@ int mray_nrc_create(const MRayNrcConfig* hCfg, MRayNrc** out)
     {
         float s = (l < c.levels) ? float(double(c.minResolution) * std::pow(b, double(l)) - 1.0) : 1.0f;
         v.scale[l] = s;
-        v.res[l] = uint32_t(std::ceil(s)) + 2u;
-        uint64_t cells = uint64_t(v.res[l]) * v.res[l] * v.res[l];
+        const uint32_t res = uint32_t(std::ceil(s)) + 2u;
+        const uint64_t cells = uint64_t(res) * res * res;
         v.dense[l] = (cells <= (1ull << c.log2TableSize)) ? 1u : 0u;
+        v.my[l] = v.dense[l] ? res : 2654435761u;
+        v.mz[l] = v.dense[l] ? res * res : 805459861u;
+        // entries an index of this level reaches.  The rest of a dense level's
+        // table never gets a gradient, and Adam on zero moments leaves it as
+        // it is (with eps = 0 it would not: 0 / 0)
+        const uint64_t used = (v.dense[l] && c.epsilon > 0.0f) ? cells : (1ull << c.log2TableSize);
+        n->owner.used[l] = uint32_t(used);
+        const uint32_t size = std::min(kSegEntries, (DivUp(used, kSegMinPerLevel) + 1u) & ~1u);
+        n->owner.size[l] = size;
+        const uint32_t segs = (l < c.levels) ? DivUp(used, size) : 0u;
+        n->owner.first[l + 1] = n->owner.first[l] + segs;
+        n->ownerSegs = std::max(n->ownerSegs, segs);
     }
     n->gridCount = size_t(c.levels) << c.log2TableSize;
     n->gridCount *= kNrcFeat;
     n->maxBatch = c.maxBatch;
     auto A = [&](void** p, size_t bytes) { return DevAlloc(n->arena, p, bytes); };
     int rv = MRAY_OK;
-    auto fail = [&](int r) { n->arena.Release(); if(n->hLoss) (void)hipHostFree(n->hLoss); delete n; return r; };
+    auto fail = [&](int r) { n->arena.Release(); delete n; return r; };
     if((rv = A((void**)&n->wT, kMlpParams * 2)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->wK, kMlpParams * 2)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->w, kMlpParams * 4)) != MRAY_OK) return fail(rv);
@@ -663,15 +892,9 @@ int mray_nrc_create(const MRayNrcConfig* hCfg, MRayNrc** out)
     const size_t B = c.maxBatch;
     if((rv = A((void**)&n->tb.x, kNrcLayers * B * kW * 2)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->tb.dz, kNrcLayers * B * kW * 2)) != MRAY_OK) return fail(rv);
-    if((rv = A((void**)&n->tb.dy, B * 3 * 4)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->tb.dx0, B * 32 * 4)) != MRAY_OK) return fail(rv);
-    if((rv = A((void**)&n->tb.loss, 4)) != MRAY_OK) return fail(rv);
-    if(hipHostMalloc((void**)&n->hLoss, sizeof(float), hipHostMallocDefault) != hipSuccess)
-    {
-        n->hLoss = nullptr;
-        SetError("nrc_create: pinned allocation failed");
-        return fail(MRAY_ERR_HIP);
-    }
+    if((rv = A((void**)&n->tb.pos, B * 3 * 4)) != MRAY_OK) return fail(rv);
+    if((rv = A((void**)&n->tb.loss, B / 32 * 4)) != MRAY_OK) return fail(rv);
     v.wT = n->wT;
     v.wK = n->wK;
     v.grid = n->gridH;
@@ -714,7 +937,10 @@ int mray_nrc_create(const MRayNrcConfig* hCfg, MRayNrc** out)
     hipDeviceProp_t prop;
     if(hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess)
         return fail(MRAY_ERR_HIP);
-    n->fwdBlocks = uint32_t(std::max(1, prop.multiProcessorCount)) * 2u;
+    int perCu = 0;
+    if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, KNrcInfer, int(kInferTPB), 0) != hipSuccess || perCu < 1)
+        perCu = 1;
+    n->inferBlocks = uint32_t(std::max(1, prop.multiProcessorCount)) * uint32_t(perCu);
     *out = n;
     return MRAY_OK;
 }
@@ -723,7 +949,6 @@ int mray_nrc_destroy(MRayNrc* n)
 {
     if(!n) return MRAY_OK;
     (void)hipDeviceSynchronize();
-    if(n->hLoss) (void)hipHostFree(n->hLoss);
     for(auto& p : n->evPending)
     {
         (void)hipEventDestroy(p.second.first);
@@ -740,56 +965,20 @@ int mray_nrc_infer(MRayNrc* n, const float* dRecords, uint32_t count, const uint
 {
     if(!n || !dRecords || !dOut) { SetError("nrc_infer: NULL argument"); return MRAY_ERR_INVALID; }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    uint32_t blocks = dCount ? n->fwdBlocks
-                             : std::min(n->fwdBlocks, DivUp(std::max(count, 1u), 32u * kFwdWaves));
+    const uint32_t all = DivUp(std::max(count, 1u), 32u * (kInferTPB / 64u));
+    const uint32_t blocks = dCount ? n->inferBlocks : std::min(n->inferBlocks, all);
     {
         NrcTimer t(n, 0, s);
-        KNrcForward<false><<<blocks, kFwdWaves * 64, 0, s>>>(n->view, dRecords, dCount, count, dOut,
-                                                             nullptr, NrcTrainBuf{}, 0);
+        KNrcInfer<<<blocks, kInferTPB, 0, s>>>(n->view, dRecords, dCount, count, dOut);
     }
     return NrcLaunchCheck();
 }
 
-int mray_nrc_backward(MRayNrc* n, const float* dRecords, const float* dTargets, uint32_t count,
-                      void* stream)
-{
-    if(!n || !dRecords || !dTargets) { SetError("nrc_backward: NULL argument"); return MRAY_ERR_INVALID; }
-    if(count == 0 || count > n->maxBatch || (count % 32u) != 0)
-    {
-        SetError("nrc_backward: count must be a non-zero multiple of 32, at most maxBatch");
-        return MRAY_ERR_INVALID;
-    }
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    KNrcZero<<<1, 64, 0, s>>>(n->tb.loss, 1);
-    uint32_t tiles = count / 32u;
-    uint32_t blocks = std::min(n->fwdBlocks, DivUp(tiles, kFwdWaves));
-    {
-        NrcTimer t(n, 1, s);
-        KNrcForward<true><<<blocks, kFwdWaves * 64, 0, s>>>(n->view, dRecords, nullptr, count, nullptr,
-                                                            dTargets, n->tb, count);
-    }
-    {
-        NrcTimer t(n, 2, s);
-        KNrcBackward<<<blocks, kFwdWaves * 64, 0, s>>>(n->view, n->tb, count);
-    }
-    uint32_t chunk = 512;
-    dim3 wg(DivUp(count, chunk), kNrcLayers);
-    {
-        NrcTimer t(n, 3, s);
-        KNrcWgrad<<<wg, 256, 0, s>>>(n->tb, count, chunk, n->wg);
-    }
-    {
-        NrcTimer t(n, 4, s);
-        KNrcGridBwd<<<DivUp(size_t(count) * n->view.levels, 256u), 256, 0, s>>>(n->view, dRecords,
-                                                                             n->tb.dx0, count, n->gg);
-    }
-    return NrcLaunchCheck();
-}
+static MlpAdam MlpOf(const MRayNrc* n) { return {n->w, n->wm, n->wv, n->wT, n->wK}; }
+static GridAdam GridOf(const MRayNrc* n) { return {n->grid, n->gm, n->gv, n->gridH}; }
 
-int mray_nrc_adam(MRayNrc* n, void* stream)
+static AdamArgs NextAdam(MRayNrc* n)
 {
-    if(!n) { SetError("nrc_adam: NULL argument"); return MRAY_ERR_INVALID; }
-    hipStream_t s = static_cast<hipStream_t>(stream);
     n->step++;
     AdamArgs a;
     a.lr = n->cfg.learningRate;
@@ -798,27 +987,105 @@ int mray_nrc_adam(MRayNrc* n, void* stream)
     a.eps = n->cfg.epsilon;
     a.c1 = float(1.0 / (1.0 - std::pow(double(a.b1), double(n->step))));
     a.c2 = float(1.0 / (1.0 - std::pow(double(a.b2), double(n->step))));
-    NrcTimer t(n, 5, s);
-    KNrcAdamMlp<<<DivUp(kMlpParams, 256u), 256, 0, s>>>(n->w, n->wm, n->wv, n->wg, n->wT, n->wK, a);
-    if(n->cfg.flags & MRAY_NRC_LAZY_ADAM)
-        KNrcAdamGrid<true><<<4096, 256, 0, s>>>(n->grid, n->gm, n->gv, n->gg, n->gridH, n->gridCount, a);
-    else
-        KNrcAdamGrid<false><<<4096, 256, 0, s>>>(n->grid, n->gm, n->gv, n->gg, n->gridH, n->gridCount, a);
+    return a;
+}
+
+static int CheckBatch(const MRayNrc* n, const float* dRecords, const float* dTargets, uint32_t count)
+{
+    if(!n || !dRecords || !dTargets) { SetError("nrc_backward: NULL argument"); return MRAY_ERR_INVALID; }
+    if(count == 0 || count > n->maxBatch || (count % 32u) != 0)
+    {
+        SetError("nrc_backward: count must be a non-zero multiple of 32, at most maxBatch");
+        return MRAY_ERR_INVALID;
+    }
+    return MRAY_OK;
+}
+
+// Forward and data gradients of one batch.
+static void LaunchTrain(MRayNrc* n, const float* dRecords, const float* dTargets, uint32_t count, hipStream_t s)
+{
+    NrcTimer t(n, 1, s);
+    KNrcTrain<<<count / 32u, 64, 0, s>>>(n->view, dRecords, dTargets, n->tb, count);
+    n->lossTiles = count / 32u;
+}
+
+int mray_nrc_backward(MRayNrc* n, const float* dRecords, const float* dTargets, uint32_t count,
+                      void* stream)
+{
+    MRAY_TRY(CheckBatch(n, dRecords, dTargets, count));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    n->gradsClear = false;
+    LaunchTrain(n, dRecords, dTargets, count, s);
+    {
+        NrcTimer t(n, 3, s);
+        KNrcWgrad<false><<<kWgradBlocks, kWgradWaves * 64, 0, s>>>(n->tb, count, n->wg, MlpAdam{}, AdamArgs{});
+    }
+    {
+        NrcTimer t(n, 4, s);
+        // the segments' fixed cost (clearing and reading all of them, about
+        // 10 us) is that of the atomics of about 1000 samples
+        if(n->ownerSegs <= kOwnerMaxSegs && count >= 1024u)
+            KNrcGridOwner<OWNER_ADD><<<n->owner.first[kNrcMaxLevels], kOwnerTPB, 0, s>>>(
+                n->view, n->tb, count, n->owner, n->gg, GridAdam{}, AdamArgs{});
+        else
+            KNrcGridBwd<<<dim3(DivUp(count, 256u), n->view.levels), 256, 0, s>>>(n->view, n->tb, count, n->gg);
+    }
     return NrcLaunchCheck();
 }
 
+int mray_nrc_adam(MRayNrc* n, void* stream)
+{
+    if(!n) { SetError("nrc_adam: NULL argument"); return MRAY_ERR_INVALID; }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const AdamArgs a = NextAdam(n);
+    NrcTimer t(n, 5, s);
+    KNrcAdamMlp<<<DivUp(kMlpParams, 256u), 256, 0, s>>>(MlpOf(n), n->wg, a);
+    if(n->cfg.flags & MRAY_NRC_LAZY_ADAM)
+        KNrcAdamGrid<true><<<4096, 256, 0, s>>>(GridOf(n), n->gg, n->gridCount, a);
+    else
+        KNrcAdamGrid<false><<<4096, 256, 0, s>>>(GridOf(n), n->gg, n->gridCount, a);
+    n->gradsClear = true;
+    return NrcLaunchCheck();
+}
+
+// Backward and Adam.  With no gradients pending from earlier backward passes
+// both gradients are applied where they are formed and never stored.
 int mray_nrc_train(MRayNrc* n, const float* dRecords, const float* dTargets, uint32_t count,
                    void* stream)
 {
-    MRAY_TRY(mray_nrc_backward(n, dRecords, dTargets, count, stream));
-    return mray_nrc_adam(n, stream);
+    MRAY_TRY(CheckBatch(n, dRecords, dTargets, count));
+    if(!n->gradsClear || n->ownerSegs > kOwnerMaxSegs)
+    {
+        MRAY_TRY(mray_nrc_backward(n, dRecords, dTargets, count, stream));
+        return mray_nrc_adam(n, stream);
+    }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    LaunchTrain(n, dRecords, dTargets, count, s);
+    const AdamArgs a = NextAdam(n);
+    {
+        NrcTimer t(n, 3, s);
+        KNrcWgrad<true><<<kWgradBlocks, kWgradWaves * 64, 0, s>>>(n->tb, count, n->wg, MlpOf(n), a);
+    }
+    {
+        NrcTimer t(n, 4, s);
+        const uint32_t blocks = n->owner.first[kNrcMaxLevels];
+        if(n->cfg.flags & MRAY_NRC_LAZY_ADAM)
+            KNrcGridOwner<OWNER_LAZY><<<blocks, kOwnerTPB, 0, s>>>(n->view, n->tb, count, n->owner, n->gg, GridOf(n), a);
+        else
+            KNrcGridOwner<OWNER_ADAM><<<blocks, kOwnerTPB, 0, s>>>(n->view, n->tb, count, n->owner, n->gg, GridOf(n), a);
+    }
+    return NrcLaunchCheck();
 }
 
 int mray_nrc_last_loss(MRayNrc* n, float* hLoss)
 {
     if(!n || !hLoss) { SetError("nrc_last_loss: NULL argument"); return MRAY_ERR_INVALID; }
     MRAY_HIP_CHECK(hipDeviceSynchronize());
-    MRAY_HIP_CHECK(hipMemcpy(hLoss, n->tb.loss, sizeof(float), hipMemcpyDeviceToHost));
+    std::vector<float> part(n->lossTiles);
+    MRAY_HIP_CHECK(hipMemcpy(part.data(), n->tb.loss, part.size() * sizeof(float), hipMemcpyDeviceToHost));
+    double sum = 0.0;
+    for(float x : part) sum += x;
+    *hLoss = float(sum);
     return MRAY_OK;
 }
 
@@ -898,6 +1165,7 @@ int mray_nrc_zero_grads(MRayNrc* n, void* stream)
     hipStream_t s = static_cast<hipStream_t>(stream);
     KNrcZero<<<256, 256, 0, s>>>(n->wg, kMlpParams);
     KNrcZero<<<2048, 256, 0, s>>>(n->gg, n->gridCount);
+    n->gradsClear = true;
     return NrcLaunchCheck();
 }
 
