@@ -38,6 +38,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <random>
 #include <vector>
 
@@ -52,6 +53,8 @@ constexpr uint32_t kW = 64;                  // width of every layer
 constexpr uint32_t kNrcFeat = 2;
 constexpr uint32_t kNrcMaxLevels = 16;
 constexpr uint32_t kInferTPB = 512;          // 8 waves: 256 queries per block and round
+constexpr uint32_t kEncodeTPB = 256;
+constexpr uint32_t kSplitChunk = 1u << 19;   // queries encoded at a time (32 MiB of features)
 constexpr uint32_t kLayerParams = kW * kW;
 constexpr uint32_t kMlpParams = kNrcLayers * kLayerParams;
 // kernel kinds timed by mray_nrc_kernel_times: inference forward, training
@@ -339,8 +342,10 @@ __device__ __forceinline__ void StageWeights(const NrcView& v, uint4* sW)
     __syncthreads();
 }
 
-// Persistent waves over 32-query tiles, weights staged once per block (48 KiB
-// in fragment order).  Bound by the grid gathers, not by the products.
+// The one-kernel form, for a count that only the device knows (the renderer's
+// query queues, mostly empty) and for captured calls: persistent waves over
+// 32-query tiles, weights staged once per block (48 KiB in fragment order).
+// Bound by the latency of the grid gathers.
 __global__ void __launch_bounds__(kInferTPB)
 KNrcInfer(NrcView v, const float* __restrict__ rec, const uint32_t* __restrict__ dCount, uint32_t count,
           float* __restrict__ out)
@@ -361,6 +366,74 @@ KNrcInfer(NrcView v, const float* __restrict__ rec, const uint32_t* __restrict__
         float pos[3];
         RecordPos(r, pos);
         XRow x = EncodePair<true>(v, r, pos);
+        InferLayers(sW, x, out, s, n);
+    }
+}
+
+// A count known on the host: encoding by level first, one lane per query and
+// level.  One level's table (2 MiB at 2^19 entries) fits an XCD's 4 MiB L2, all
+// of them (22 MiB) do not, and waves that walk the levels on their own spread
+// over all of them (33 M of 84 M L2 reads missed per 10^6 queries, now 5.6 of
+// 61).  Workgroups go round-robin over the 8 XCDs, so workgroup 8 j + x is the
+// j-th of XCD x: it first takes its own hashed levels for every query, then an
+// eighth of the queries for each remaining level.
+// 16 levels of 2^19 entries: 10^6 queries 643 -> 290 us of encoding (L2 serves
+// 211 reads/ns, near its 16 channels per XCD a clock) + 70 us of layers; 4096
+// queries 41 -> 26 us, because the lanes are 16 times as many.  Chunks of 2^18
+// and 2^17 queries cost 9 and 22 % more.
+struct EncodePlan
+{
+    uint32_t own;                            // hashed levels per XCD
+    uint32_t shared;                         // levels shared by all XCDs
+    uint32_t ownLevel[kNrcMaxLevels];        // [own][8]
+    uint32_t sharedLevel[kNrcMaxLevels];
+};
+__global__ void __launch_bounds__(kEncodeTPB)
+KNrcEncode(NrcView v, const float* __restrict__ rec, uint32_t n, EncodePlan plan, uint32_t* __restrict__ feat)
+{
+    const uint32_t blocks = (n + kEncodeTPB - 1u) / kEncodeTPB, eighth = (blocks + 7u) / 8u;
+    const uint32_t xcd = blockIdx.x & 7u, j = blockIdx.x >> 3;
+    uint32_t l, b;
+    if(j < plan.own * blocks)
+    {
+        l = plan.ownLevel[(j / blocks) * 8u + xcd];
+        b = j % blocks;
+    }
+    else
+    {
+        const uint32_t i = j - plan.own * blocks;
+        l = plan.sharedLevel[i / eighth];
+        b = (i % eighth) * 8u + xcd;
+    }
+    const uint32_t s = b * kEncodeTPB + threadIdx.x;
+    if(s >= n) return;
+    float pos[3];
+    RecordPos(rec + size_t(s) * 11u, pos);
+    feat[size_t(l) * n + s] = LevelFeatures<true>(reinterpret_cast<const uint32_t*>(v.grid) + (size_t(l) << v.log2T), pos,
+                                                  v.scale[l], v.my[l], v.mz[l], v.dense[l], (1u << v.log2T) - 1u);
+}
+
+// The layers over encoded queries.
+__global__ void __launch_bounds__(kInferTPB)
+KNrcInferEncoded(NrcView v, const float* __restrict__ rec, const uint32_t* __restrict__ feat, uint32_t n,
+                 float* __restrict__ out)
+{
+    __shared__ uint4 sW[kNrcLayers * kFragLayer];
+    constexpr uint32_t kWaves = kInferTPB / 64u;
+    StageWeights(v, sW);
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const bool hi = (lane & 32u) != 0u;
+    for(size_t tile = blockIdx.x * kWaves + wave; tile * 32u < n; tile += gridDim.x * kWaves)
+    {
+        const size_t s = tile * 32u + (lane & 31u), at = min(s, size_t(n) - 1u);
+        XRow x;
+        #pragma unroll
+        for(uint32_t m = 0; m < 8; m++)
+        {
+            const uint32_t l = LevelOfWord(m) + (hi ? 2u : 0u);
+            x.u[m] = (l < v.levels) ? feat[size_t(l) * n + at] : 0u;
+        }
+        EncodeTail(rec + at * 11u, hi, x);
         InferLayers(sW, x, out, s, n);
     }
 }
@@ -789,6 +862,11 @@ struct MRayNrc
     bool gradsClear = true;       // no backward pass since the last Adam or clear
     OwnerLevels owner{};
     uint32_t ownerSegs = 0;       // segments of the largest level
+    // features of one chunk of queries (InferSplit)
+    std::mutex featLock;
+    uint32_t* feat = nullptr;
+    hipEvent_t featDone = nullptr;
+    EncodePlan plan{};
     // per-kernel timing (mray_nrc_set_profiling): event pairs around each
     // launch, harvested by mray_nrc_kernel_times
     bool profiling = false;
@@ -872,12 +950,23 @@ int mray_nrc_create(const MRayNrcConfig* hCfg, MRayNrc** out)
         n->owner.first[l + 1] = n->owner.first[l] + segs;
         n->ownerSegs = std::max(n->ownerSegs, segs);
     }
+    // encoding plan: whole rows of 8 hashed levels, one per XCD; the rest shared
+    {
+        std::vector<uint32_t> hashed, rest;
+        for(uint32_t l = 0; l < c.levels; l++) (v.dense[l] ? rest : hashed).push_back(l);
+        EncodePlan& p = n->plan;
+        p.own = uint32_t(hashed.size()) / 8u;
+        for(uint32_t k = 0; k < 8u * p.own; k++) p.ownLevel[k] = hashed[hashed.size() - 1u - k];
+        for(size_t k = 0; k + 8u * p.own < hashed.size(); k++) rest.push_back(hashed[k]);
+        p.shared = uint32_t(rest.size());
+        std::copy(rest.begin(), rest.end(), p.sharedLevel);
+    }
     n->gridCount = size_t(c.levels) << c.log2TableSize;
     n->gridCount *= kNrcFeat;
     n->maxBatch = c.maxBatch;
     auto A = [&](void** p, size_t bytes) { return DevAlloc(n->arena, p, bytes); };
     int rv = MRAY_OK;
-    auto fail = [&](int r) { n->arena.Release(); delete n; return r; };
+    auto fail = [&](int r) { n->arena.Release(); if(n->featDone) (void)hipEventDestroy(n->featDone); delete n; return r; };
     if((rv = A((void**)&n->wT, kMlpParams * 2)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->wK, kMlpParams * 2)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->w, kMlpParams * 4)) != MRAY_OK) return fail(rv);
@@ -895,6 +984,12 @@ int mray_nrc_create(const MRayNrcConfig* hCfg, MRayNrc** out)
     if((rv = A((void**)&n->tb.dx0, B * 32 * 4)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->tb.pos, B * 3 * 4)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->tb.loss, B / 32 * 4)) != MRAY_OK) return fail(rv);
+    if((rv = A((void**)&n->feat, size_t(kSplitChunk) * kNrcMaxLevels * 4u)) != MRAY_OK) return fail(rv);
+    if(hipEventCreateWithFlags(&n->featDone, hipEventDisableTiming) != hipSuccess)
+    {
+        SetError("nrc_create: event creation failed");
+        return fail(MRAY_ERR_HIP);
+    }
     v.wT = n->wT;
     v.wK = n->wK;
     v.grid = n->gridH;
@@ -955,9 +1050,35 @@ int mray_nrc_destroy(MRayNrc* n)
         (void)hipEventDestroy(p.second.second);
     }
     for(hipEvent_t e : n->evPool) (void)hipEventDestroy(e);
+    if(n->featDone) (void)hipEventDestroy(n->featDone);
     n->arena.Release();
     delete n;
     return MRAY_OK;
+}
+
+// Encoding in its own pass, chunk by chunk through the cache's feature area.
+// Calls on other streams wait for the area's last use; a call under capture
+// (its graph may run beside others) takes the one-kernel form.
+constexpr int kNoSplit = -1;
+static int InferSplit(MRayNrc* n, const float* dRecords, uint32_t count, float* dOut, uint32_t blocks, hipStream_t s)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    MRAY_HIP_CHECK(hipStreamIsCapturing(s, &cap));
+    if(cap != hipStreamCaptureStatusNone) return kNoSplit;
+    std::lock_guard<std::mutex> lock(n->featLock);
+    MRAY_HIP_CHECK(hipStreamWaitEvent(s, n->featDone, 0));
+    const EncodePlan& p = n->plan;
+    for(uint32_t at = 0; at < count; at += kSplitChunk)
+    {
+        const uint32_t c = std::min(kSplitChunk, count - at);
+        const uint32_t b = DivUp(c, kEncodeTPB), perXcd = p.own * b + p.shared * DivUp(b, 8u);
+        const float* rec = dRecords + size_t(at) * 11u;
+        NrcTimer t(n, 0, s);
+        KNrcEncode<<<8u * perXcd, kEncodeTPB, 0, s>>>(n->view, rec, c, p, n->feat);
+        KNrcInferEncoded<<<blocks, kInferTPB, 0, s>>>(n->view, rec, n->feat, c, dOut + size_t(at) * 3u);
+    }
+    MRAY_HIP_CHECK(hipEventRecord(n->featDone, s));
+    return NrcLaunchCheck();
 }
 
 int mray_nrc_infer(MRayNrc* n, const float* dRecords, uint32_t count, const uint32_t* dCount,
@@ -967,6 +1088,11 @@ int mray_nrc_infer(MRayNrc* n, const float* dRecords, uint32_t count, const uint
     hipStream_t s = static_cast<hipStream_t>(stream);
     const uint32_t all = DivUp(std::max(count, 1u), 32u * (kInferTPB / 64u));
     const uint32_t blocks = dCount ? n->inferBlocks : std::min(n->inferBlocks, all);
+    if(!dCount && count > 0)
+    {
+        const int r = InferSplit(n, dRecords, count, dOut, blocks, s);
+        if(r != kNoSplit) return r;
+    }
     {
         NrcTimer t(n, 0, s);
         KNrcInfer<<<blocks, kInferTPB, 0, s>>>(n->view, dRecords, dCount, count, dOut);

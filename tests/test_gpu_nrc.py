@@ -182,6 +182,31 @@ def test_lazy_grid_adam(torch_gpu):
     n.close()
 
 
+@pytest.mark.parametrize("levels,log2_table", [(1, 12), (6, 14), (16, 15)])
+def test_infer_forms_agree(torch_gpu, levels, log2_table):
+    """Queries encoded in a pass of their own (the count known on the host,
+    chunks of 2^19) answer exactly as in the one-kernel form (the count read
+    on the device), at the counts where a tile, a block and the chunk change."""
+    import ctypes
+    from mray_amd import native
+    torch = torch_gpu
+    nrc = native.Nrc(levels=levels, log2_table=log2_table, max_batch=32, seed=levels)
+    rng = np.random.default_rng(levels)
+    nrc.write(abi.NRC_GRID, rng.uniform(-0.5, 0.5, size=(nrc.grid_params,)).astype(np.float32))
+    rec = _records(rng, 600000)
+    rec[:64, 0:3] = rng.integers(0, 2, size=(64, 3))       # corners of the box
+    d = torch.from_numpy(rec).cuda()
+    for n in (1, 31, 32, 33, 255, 256, 257, 511, 513, 524288, 524289, 600000):
+        one = torch.full((n + 1, 3), -7.0, device="cuda")
+        count = torch.tensor([n], dtype=torch.int32, device="cuda")
+        native.check(native.lib().mray_nrc_infer(nrc.h, ctypes.c_void_p(d.data_ptr()), 0,
+                                                 ctypes.c_void_p(count.data_ptr()),
+                                                 ctypes.c_void_p(one.data_ptr()), None))
+        assert torch.equal(nrc.infer(d[:n].contiguous()), one[:n]), n
+        assert torch.all(one[n:] == -7.0)
+    nrc.close()
+
+
 @pytest.mark.parametrize("lazy", [False, True])
 @pytest.mark.parametrize("levels,log2_table,count", [(1, 10, 32), (5, 13, 992), (16, 14, 1024), (16, 16, 4128)])
 def test_train_is_backward_then_adam(torch_gpu, levels, log2_table, count, lazy):
