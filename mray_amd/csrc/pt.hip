@@ -165,39 +165,84 @@ __device__ __forceinline__ uint32_t ShardOfChunk(uint32_t c, uint32_t n)
     const uint32_t C = (n + 63u) / 64u;
     return uint32_t((uint64_t(c) * kShards) / C);
 }
-// Dynamic work fetch, 64 items per atomic, over kXcds counters: the list
-// [0, n) is cut into kXcds contiguous parts, a wave starts on the part of its
-// XCD (workgroups are dispatched round-robin over the 8 XCDs, each with its
-// own L2, so an XCD keeps to one region of the image) and then takes from
-// the others.  A plain load first skips a part already used up; every wave
-// exits after one pass over the parts.  Wave-uniform values stay scalar.
-// f(k) runs for each item k < n.
+// Work fetch, 64 items at a time, over kXcds counters: the list [0, n) is cut
+// into kXcds contiguous parts, a wave starts on the part of its XCD
+// (workgroups are dispatched round-robin over the 8 XCDs, each with its own
+// L2, so an XCD keeps to one region of the image) and then takes from the
+// others.  Every wave's first chunk is its own by position, so a list of at
+// most one chunk per wave is handed out without touching a counter; the
+// counters hand out the rest.  (With every chunk from a counter, a bounce of
+// 200 waves spent 8 dependent agent-scope loads per wave finding the parts
+// empty: KTrace 22.6 us, KShadow 24.2 us; now 10.7 and
+// 8.1.  At 3000 waves, 190 K rays: 70.8 -> 41.1 and 65.6 -> 41.0 us.)
+// Once its part is used up, a wave reads all counters in one load and goes
+// through the parts that still hold chunks, once.  Wave-uniform values stay
+// scalar.  f(k) runs for each item k < n.
 constexpr uint32_t kXcds = 8;
-template<class F>
+struct ListPart
+{
+    uint32_t first, size;     // chunks
+    uint32_t own;             // of which handed out by position
+};
+template<uint32_t TPB>
+__device__ __forceinline__ ListPart PartOf(uint32_t part, uint32_t C)
+{
+    ListPart p;
+    p.first = uint32_t((uint64_t(C) * part) / kXcds);
+    p.size = uint32_t((uint64_t(C) * (part + 1u)) / kXcds) - p.first;
+    p.own = min(p.size, ((gridDim.x + kXcds - 1u - part) / kXcds) * (TPB / 64u));
+    return p;
+}
+template<uint32_t TPB, class F>
 __device__ __forceinline__ void FetchLoop(uint32_t* ctr, uint32_t n, F&& f)
 {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t C = (n + 63u) / 64u;                       // 64-item chunks
     uint32_t part = blockIdx.x % kXcds;
-    for(uint32_t t = 0; t < kXcds; t++)
+    // the wave's own chunk first, then counters
+    uint32_t c = __builtin_amdgcn_readfirstlane((blockIdx.x / kXcds) * (TPB / 64u) + (threadIdx.x >> 6));
+    uint64_t more = 0;                                        // parts with chunks left
+    bool mine = true;                                         // still in the wave's own part
+    ListPart p = PartOf<TPB>(part, C);
+    if(c >= p.size) c = kInvalid;
+    for(;;)
     {
-        const uint32_t c0 = __builtin_amdgcn_readfirstlane(uint32_t((uint64_t(C) * part) / kXcds));
-        const uint32_t c1 = __builtin_amdgcn_readfirstlane(uint32_t((uint64_t(C) * (part + 1u)) / kXcds));
-        uint32_t* fc = ctr + size_t(part) * kCtrStride;
-        for(;;)
+        if(c != kInvalid)
         {
-            uint32_t c = c1 - c0;
-            if(lane == 0)
-            {
-                c = __hip_atomic_load(fc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if(c < c1 - c0) c = atomicAdd(fc, 1u);
-            }
-            c = __builtin_amdgcn_readfirstlane(c);
-            if(c >= c1 - c0) break;
-            const uint32_t k = (c0 + c) * 64u + lane;
+            const uint32_t k = (p.first + c) * 64u + lane;
             if(k < n) f(k);
         }
-        part = (part + 1u) % kXcds;
+        // next chunk of this part, if its counter has one
+        c = kInvalid;
+        if(p.own < p.size)
+        {
+            uint32_t* fc = ctr + size_t(part) * kCtrStride;
+            uint32_t v = p.size;
+            if(lane == 0)
+            {
+                v = p.own + __hip_atomic_load(fc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if(v < p.size) v = p.own + atomicAdd(fc, 1u);
+            }
+            v = __builtin_amdgcn_readfirstlane(v);
+            if(v < p.size) c = v;
+        }
+        if(c != kInvalid) continue;
+        if(mine)
+        {
+            mine = false;
+            const ListPart q = PartOf<TPB>(lane % kXcds, C);
+            bool left = false;
+            if(lane < kXcds && lane != part && q.own < q.size)
+                left = q.own + __hip_atomic_load(ctr + size_t(lane) * kCtrStride, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT) < q.size;
+            more = __ballot(left);
+        }
+        if(more == 0ull) break;
+        // the next part in cyclic order that had chunks
+        const uint64_t after = more & ~((2ull << part) - 1ull);
+        part = uint32_t(__builtin_ctzll(after ? after : more));
+        more &= ~(1ull << part);
+        p = PartOf<TPB>(part, C);
     }
 }
 
@@ -338,11 +383,15 @@ __device__ __forceinline__ SceneView SlotScene(const RenderConst& rc, const Slot
 
 static constexpr uint32_t kSlotTPB = 256;
 static constexpr uint32_t kMatQueues = 5;   // boundary/light + 4 material types
-static constexpr uint32_t kGraphIters = 8;  // bounces per captured hipGraph
+static constexpr uint32_t kGraphIters = 4;  // bounces per captured hipGraph
 // Bursts queued ahead of the one whose scheduler snapshot the host reads: the
 // GPU always holds kLookahead bursts of queued work while the host decides
-// whether the frame is done.
-static constexpr uint32_t kLookahead = 2;
+// whether the frame is done.  What is queued past the frame's end finds no
+// work but still launches (9 us a bounce): bursts of 8, two ahead, ran 22 such
+// bounces after a 26-bounce preview frame (1662 us), bursts of 4, one ahead,
+// 6 (1512 us); bursts of 2 lose as much between graphs (1599 us).  Frames of
+// 20 ms and more differ by under 1 %.
+static constexpr uint32_t kLookahead = 1;
 static constexpr uint32_t kRingBursts = kLookahead + 1;
 
 // ---------------------------------------------------------------------------
@@ -390,6 +439,33 @@ KRefillCount(const uint32_t* __restrict__ meta, const uint32_t* __restrict__ vie
         }
         blockCnt[blockIdx.x] = c;
     }
+}
+
+// The refill amount (ReloadPaths with TotalSampleLimit,
+// PathTracerRendererBase.h:59-67) and the bounce's totals, by one thread.
+// The path counter itself is advanced by the traversal kernel that follows
+// (AdvanceCounter): other blocks of a fused refill still read it here.
+__device__ __forceinline__ void RefillTotals(Sched* __restrict__ sched, unsigned long long freeSlots,
+                                             uint32_t live, unsigned long long finished)
+{
+    const unsigned long long remaining = sched->limit - sched->counter;
+    const unsigned long long fill = (freeSlots < remaining) ? freeSlots : remaining;
+    sched->base = sched->counter;
+    sched->fill = uint32_t(fill);
+    sched->activeCount = live + uint32_t(fill);
+    sched->deadTotal += finished;
+    // a bounce after the frame has drained (queued ahead by the host) does
+    // nothing and is not counted
+    if(sched->activeCount != 0 || finished != 0)
+    {
+        if(sched->iterations == 0) sched->startClock = wall_clock64();
+        sched->iterations += 1;
+    }
+}
+__device__ __forceinline__ void AdvanceCounter(Sched* __restrict__ sched, uint32_t rays)
+{
+    sched->extRays += rays;
+    sched->counter += sched->fill;
 }
 
 // One block: exclusive scans of the free and live counts, then the refill
@@ -487,24 +563,7 @@ KRefillScan(uint4* __restrict__ blockCnt, uint32_t count, Sched* __restrict__ sc
         for(uint32_t v = sched->viewsDone; v < bound; v++) viewClock[v] = now;
         if(bound > sched->viewsDone) sched->viewsDone = bound;
     }
-    if(threadIdx.x == 0)
-    {
-        unsigned long long freeSlots = carryF;
-        unsigned long long remaining = sched->limit - sched->counter;
-        unsigned long long fill = (freeSlots < remaining) ? freeSlots : remaining;
-        sched->base = sched->counter;
-        sched->fill = uint32_t(fill);
-        sched->counter += fill;
-        sched->activeCount = carryL + uint32_t(fill);
-        sched->deadTotal += accum;
-        // a bounce after the frame has drained (queued ahead by the host)
-        // does nothing and is not counted
-        if(sched->activeCount != 0 || accum != 0)
-        {
-            if(sched->iterations == 0) sched->startClock = wall_clock64();
-            sched->iterations += 1;
-        }
-    }
+    if(threadIdx.x == 0) RefillTotals(sched, carryF, carryL, accum);
 }
 
 // Finished path -> film (AddRadianceToRenderBufferThroughput,
@@ -644,11 +703,16 @@ __device__ __forceinline__ void StartCameraPath(const SlotSoA& S, const CameraGP
     S.meta[i] = MPack(0, ST_ALIVE, RT_CAMERA, false, false);
 }
 
-template<bool SPECTRAL, bool BATCH>
+// FUSED: blockOff holds KRefillCount's counts, and every block sums the counts
+// of the blocks before it instead of a scan kernel between the two: for
+// renderers of few slots, where a launch costs more than these reads
+// (kFusedRefillBlocks).  The last block has the totals.
+template<bool SPECTRAL, bool BATCH, bool FUSED = false>
 __global__ void __launch_bounds__(kSlotTPB)
 KRefillApply(SlotSoA S, RenderConst rc, const uint4* __restrict__ blockOff,
-             Sched* __restrict__ sched, uint32_t* __restrict__ active)
+             Sched* __restrict__ sched, uint32_t* __restrict__ active, uint32_t* __restrict__ ctr)
 {
+    static_assert(!(FUSED && BATCH), "batch renderers need the scan's view clocks");
     __shared__ uint32_t wsum[kSlotTPB / 64], asum[kSlotTPB / 64];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -666,15 +730,56 @@ KRefillApply(SlotSoA S, RenderConst rc, const uint4* __restrict__ blockOff,
     __syncthreads();
     uint32_t waveOff = 0;
     for(uint32_t w = 0; w < wave; w++) waveOff += wsum[w];
-    const uint4 off = blockOff[blockIdx.x];
-    const uint32_t fill = sched->fill;
+    uint4 off;
+    uint32_t fill;
+    unsigned long long firstPath;
+    if constexpr(FUSED)
+    {
+        static_assert(CTR_COUNT <= kSlotTPB, "one thread per counter");
+        __shared__ uint32_t psum[3][kSlotTPB / 64];
+        if(blockIdx.x == 0 && threadIdx.x < CTR_COUNT) *Ctr(ctr, threadIdx.x) = 0u;
+        uint32_t f = 0, l = 0, z = 0;
+        for(uint32_t k = threadIdx.x; k < blockIdx.x; k += kSlotTPB)
+        {
+            const uint4 c = blockOff[k];
+            f += c.x; l += c.y; z += c.z;
+        }
+        for(uint32_t o = 32; o > 0; o >>= 1)
+        {
+            f += __shfl_xor(f, o); l += __shfl_xor(l, o); z += __shfl_xor(z, o);
+        }
+        if(lane == 0) { psum[0][wave] = f; psum[1][wave] = l; psum[2][wave] = z; }
+        __syncthreads();
+        off = make_uint4(0, 0, 0, 0);
+        for(uint32_t w = 0; w < kSlotTPB / 64; w++)
+        {
+            off.x += psum[0][w]; off.y += psum[1][w]; off.z += psum[2][w];
+        }
+        // a rank below the free count is below the refill amount if it is
+        // below the remaining paths: the total is not needed here
+        firstPath = sched->counter;
+        const unsigned long long remaining = sched->limit - firstPath;
+        fill = (remaining < 0xFFFFFFFFull) ? uint32_t(remaining) : 0xFFFFFFFFu;
+        if(blockIdx.x == gridDim.x - 1u && threadIdx.x == 0)
+        {
+            const uint4 mine = blockOff[blockIdx.x];
+            RefillTotals(sched, (unsigned long long)off.x + mine.x, off.y + mine.y,
+                         (unsigned long long)off.z + mine.z);
+        }
+    }
+    else
+    {
+        off = blockOff[blockIdx.x];
+        fill = sched->fill;
+        firstPath = sched->base;
+    }
     bool alive = inRange && !freeSlot;
     if(freeSlot)
     {
         uint32_t rank = off.x + waveOff + uint32_t(__popcll(b & lt));
         if(rank < fill)
         {
-            const unsigned long long g = sched->base + rank;
+            const unsigned long long g = firstPath + rank;
             if constexpr(BATCH)
             {
                 uint32_t lo, pix;
@@ -742,9 +847,9 @@ KTrace(TraceCtx ctx, SlotSoA S, const uint32_t* __restrict__ active, Sched* __re
     __shared__ uint2 lstack[kLdsStack * TPB];
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t n = sched->activeCount;
-    if(gtid == 0) sched->extRays += n;
+    if(gtid == 0) AdvanceCounter(sched, n);
     uint32_t nodes = 0, tris = 0;
-    FetchLoop(Ctr(ctr, CTR_TRACE), n, [&](uint32_t k)
+    FetchLoop<TPB>(Ctr(ctr, CTR_TRACE), n, [&](uint32_t k)
     {
         const uint32_t i = active[k];
         const float4 o = S.rayO[i], d = S.rayD[i];
@@ -836,7 +941,7 @@ KTraceRefill(TraceCtx ctx, SlotSoA S, const uint32_t* __restrict__ active, Sched
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t below = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
     const uint32_t n = sched->activeCount;
-    if(gtid == 0) sched->extRays += n;
+    if(gtid == 0) AdvanceCounter(sched, n);
     ChunkSource src(Ctr(ctr, CTR_TRACE), n);
     uint32_t pool = 0, poolEnd = 0;        // wave-uniform: items not yet handed out
     bool more = true;                      // wave-uniform: chunks may remain
@@ -1707,7 +1812,7 @@ KShadow(TraceCtx ctx, SlotSoA S, const uint32_t* __restrict__ shadowQ, Sched* __
     const uint32_t n = g.pre[kShards];
     if(gtid == 0) sched->shadowRays += n;
     uint32_t nodes = 0, tris = 0;
-    FetchLoop(Ctr(ctr, CTR_SHADOW_FETCH), n, [&](uint32_t k)
+    FetchLoop<TPB>(Ctr(ctr, CTR_SHADOW_FETCH), n, [&](uint32_t k)
     {
         uint32_t sh;
         const uint32_t i = shadowQ[ShardItem(g, k, cap, sh)];
@@ -2036,6 +2141,31 @@ static void LaunchShadow(MRayRenderer* r, hipStream_t s)
     else KShadow<4, BATCH, kTraceTPB, false, COUNT><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dShadowQ, r->dSched, r->dViews, r->rc.nrc, r->dCtr, r->rc.N);
 }
 
+// Slot blocks up to which a block sums the earlier blocks' counts itself:
+// at 64 blocks the scan kernel took 4.4 us a bounce and its launch 1.5 more,
+// the sums 0.5; at 2025 blocks 5.2 and 1.5 against 1.2.  Beyond, the sums grow
+// with the square of the blocks.
+constexpr uint32_t kFusedRefillBlocks = 2048;
+template<bool BATCH>
+static void LaunchRefillApply(MRayRenderer* r, bool fused, hipStream_t s)
+{
+    auto launch = [&](auto kernel)
+    {
+        kernel<<<r->nBlocks, kSlotTPB, 0, s>>>(r->S, r->rc, r->dBlockCnt, r->dSched, r->dActive, r->dCtr);
+    };
+    if constexpr(!BATCH)
+    {
+        if(fused)
+        {
+            if(r->rc.spectral) launch(KRefillApply<true, false, true>);
+            else launch(KRefillApply<false, false, true>);
+            return;
+        }
+    }
+    if(r->rc.spectral) launch(KRefillApply<true, BATCH>);
+    else launch(KRefillApply<false, BATCH>);
+}
+
 template<bool BATCH, bool INST>
 static int EnqueueIterationT(MRayRenderer* r, hipStream_t s)
 {
@@ -2049,8 +2179,10 @@ static int EnqueueIterationT(MRayRenderer* r, hipStream_t s)
     int mk;
     if((mk = Mark(r, s)) != MRAY_OK) return mk;
     KRefillCount<BATCH><<<r->nBlocks, kSlotTPB, 0, s>>>(r->S.meta, r->S.view, N, r->dBlockCnt);
+    const bool fused = !BATCH && r->nBlocks <= kFusedRefillBlocks;
     // per-view latency needs views issued in order: not in frame order
-    KRefillScan<<<1, 1024, 0, s>>>(r->dBlockCnt, r->nBlocks, r->dSched, r->rc.viewBegin,
+    if(!fused)
+        KRefillScan<<<1, 1024, 0, s>>>(r->dBlockCnt, r->nBlocks, r->dSched, r->rc.viewBegin,
                                    r->rc.viewCount,
                                    (BATCH && !r->rc.frameMajor) ? r->dViewClock : nullptr, r->dCtr);
     if(r->rc.nrc.on)
@@ -2063,12 +2195,7 @@ static int EnqueueIterationT(MRayRenderer* r, hipStream_t s)
         else
             KNrcEmit<false, BATCH><<<DivUp(lanes, 256), 256, 0, s>>>(r->S, r->rc, r->dSched, r->nrcLog2G);
     }
-    if(r->rc.spectral)
-        KRefillApply<true, BATCH><<<r->nBlocks, kSlotTPB, 0, s>>>(r->S, r->rc, r->dBlockCnt, r->dSched,
-                                                                  r->dActive);
-    else
-        KRefillApply<false, BATCH><<<r->nBlocks, kSlotTPB, 0, s>>>(r->S, r->rc, r->dBlockCnt, r->dSched,
-                                                                   r->dActive);
+    LaunchRefillApply<BATCH>(r, fused, s);
     if((mk = Mark(r, s)) != MRAY_OK) return mk;
     if(r->counting) LaunchTrace<true, BATCH, INST>(r, s);
     else LaunchTrace<false, BATCH, INST>(r, s);
@@ -2403,6 +2530,10 @@ static int SizeLaunches(MRayRenderer* r)
         r->shadowBlocks = uint32_t(w8 ? resident(KShadow<8, true>, tpb, maxTraceBlocks)
                                       : resident(KShadow<4, true>, tpb, maxTraceBlocks));
     }
+    // no more waves than 64-item chunks of N slots, the same number per XCD
+    const uint32_t useful = kXcds * DivUp(DivUp(N, tpb), kXcds);
+    r->traceBlocks = std::min(r->traceBlocks, useful);
+    r->shadowBlocks = std::min(r->shadowBlocks, useful);
     if(p->flags & MRAY_RENDER_MATERIAL_QUEUES)
     {
         if(!r->dQueues)
