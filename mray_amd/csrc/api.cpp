@@ -249,6 +249,11 @@ static int BuildAccel(MRayAccel* a, const MRaySceneDesc* s, uint32_t builder, ui
         MRAY_TRY(Upload(ar, &a->dSoup, soup.data(), soup.size()));
     }
 
+    if(width == 4)
+    {
+        MRAY_TRY(DevAlloc(ar, (void**)&a->dQNodes, size_t(a->wideNodes) * sizeof(QNode4)));
+        MRAY_TRY(QuantizeNodes(a->dNodes, a->wideNodes, a->dQNodes, st));
+    }
     // Traversal stack spill area: <= width-1 entries per level below the root.
     int dev = 0;
     MRAY_HIP_CHECK(hipGetDevice(&dev));
@@ -262,9 +267,11 @@ static int BuildAccel(MRayAccel* a, const MRaySceneDesc* s, uint32_t builder, ui
                       size_t(a->ctx.gstackDepth) * a->ctx.gridThreads * sizeof(uint2)));
     a->ctx.maxVisits = a->wideNodes + 1u;
     a->ctx.nodes = a->dNodes;
+    a->ctx.qnodes = a->dQNodes;
     a->ctx.cnodes = a->dCNodes;
     a->ctx.soup = a->dSoup;
     a->ctx.width = width;
+    a->ctx.exact = (width == 4 && a->wideNodes <= kExactNodes) ? 1u : 0u;
     return MRAY_OK;
 }
 

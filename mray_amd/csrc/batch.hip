@@ -21,7 +21,8 @@ __device__ __forceinline__ uint32_t RelocChild(uint32_t c, uint32_t nodeOff, uin
     return c + nodeOff;
 }
 
-__global__ void KRelocNodes4(BNode4* __restrict__ n, uint32_t count, uint32_t nodeOff, uint32_t triOff)
+template<class NODE>
+__global__ void KRelocNodes4(NODE* __restrict__ n, uint32_t count, uint32_t nodeOff, uint32_t triOff)
 {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if(i >= count) return;
@@ -60,7 +61,7 @@ __global__ void KRelocKeys(uint32_t* __restrict__ k, uint32_t count, uint32_t ma
     if(i < count && !(k[i] & MRAY_LIGHT_FLAG)) k[i] += matOff;
 }
 
-int BuildBatchScene(MRayBatchScene* b, const MRayAccel* const* accels, uint32_t count)
+int BuildBatchScene(MRayBatchScene* b, const MRayAccel* const* accels, uint32_t count, bool instanced)
 {
     b->width = accels[0]->width;
     uint64_t nodes = 0, tris = 0, verts = 0, mats = 0, lights = 0;
@@ -114,7 +115,8 @@ int BuildBatchScene(MRayBatchScene* b, const MRayAccel* const* accels, uint32_t 
     b->lights = uint32_t(lights);
     DeviceArena& ar = b->arena;
     auto A = [&](void** p, size_t bytes) { return DevAlloc(ar, p, std::max<size_t>(bytes, 16)); };
-    BNode4* dNodes = nullptr;
+    BNode4* dNodes = nullptr;        // instance walks
+    QNode4* dQNodes = nullptr;       // batch walks
     CNode8* dCNodes = nullptr;
     SoupTri* dSoup = nullptr;
     float* dPos = nullptr;
@@ -125,7 +127,8 @@ int BuildBatchScene(MRayBatchScene* b, const MRayAccel* const* accels, uint32_t 
     float4* dLightRad = nullptr;
     int rv;
     if(b->width == 8) { if((rv = A((void**)&dCNodes, nodes * sizeof(CNode8))) != MRAY_OK) return rv; }
-    else if((rv = A((void**)&dNodes, nodes * sizeof(BNode4))) != MRAY_OK) return rv;
+    else if(instanced) { if((rv = A((void**)&dNodes, nodes * sizeof(BNode4))) != MRAY_OK) return rv; }
+    else if((rv = A((void**)&dQNodes, nodes * sizeof(QNode4))) != MRAY_OK) return rv;
     if((rv = A((void**)&dSoup, tris * sizeof(SoupTri))) != MRAY_OK) return rv;
     if((rv = A((void**)&dPos, verts * 3 * sizeof(float))) != MRAY_OK) return rv;
     if((rv = A((void**)&dTbn, verts * sizeof(float4))) != MRAY_OK) return rv;
@@ -147,8 +150,13 @@ int BuildBatchScene(MRayBatchScene* b, const MRayAccel* const* accels, uint32_t 
         }
         else
         {
-            MRAY_HIP_CHECK(hipMemcpy(dNodes + p.root, a->dNodes, size_t(a->wideNodes) * sizeof(BNode4), D2D));
-            KRelocNodes4<<<DivUp(a->wideNodes, 256), 256>>>(dNodes + p.root, a->wideNodes, p.root, p.triOff);
+            auto place = [&](auto* dst, const auto* src) -> int
+            {
+                MRAY_HIP_CHECK(hipMemcpy(dst + p.root, src, size_t(a->wideNodes) * sizeof(*src), D2D));
+                KRelocNodes4<<<DivUp(a->wideNodes, 256), 256>>>(dst + p.root, a->wideNodes, p.root, p.triOff);
+                return MRAY_OK;
+            };
+            MRAY_TRY(instanced ? place(dNodes, a->dNodes) : place(dQNodes, a->dQNodes));
         }
         MRAY_HIP_CHECK(hipMemcpy(dSoup + p.triOff, a->dSoup, size_t(T) * sizeof(SoupTri), D2D));
         KRelocSoup<<<DivUp(T, 256), 256>>>(dSoup + p.triOff, T, p.triOff);
@@ -193,6 +201,7 @@ int BuildBatchScene(MRayBatchScene* b, const MRayAccel* const* accels, uint32_t 
         return rv;
     c.maxVisits = b->nodes + 1u;
     c.nodes = dNodes;
+    c.qnodes = dQNodes;
     c.cnodes = dCNodes;
     c.soup = dSoup;
     c.width = b->width;
@@ -220,7 +229,7 @@ int mray_batch_scene_create(const MRayAccel* const* accels, uint32_t count, MRay
             return MRAY_ERR_INVALID;
         }
     MRayBatchScene* b = new MRayBatchScene();
-    int rv = BuildBatchScene(b, accels, count);
+    int rv = BuildBatchScene(b, accels, count, false);
     if(rv != MRAY_OK)
     {
         (void)hipDeviceSynchronize();

@@ -300,6 +300,68 @@ int CollapseToBvh4Device(const uint32_t* dBinNodes, const float* dBinBoxes, cons
     return rc;
 }
 
+// One thread per node; exact sums in double (8-bit times 24-bit products).
+__global__ void __launch_bounds__(kTPB)
+KQuantizeNodes(const BNode4* __restrict__ in, uint32_t n, QNode4* __restrict__ out)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if(i >= n) return;
+    const BNode4 b = in[i];
+    QNode4 q;
+    for(int k = 0; k < 4; k++) q.child[k] = b.child[k];
+    uint32_t words[6];
+    for(int a = 0; a < 3; a++)
+    {
+        const float* lo = (a == 0) ? b.lox : (a == 1) ? b.loy : b.loz;
+        const float* hi = (a == 0) ? b.hix : (a == 1) ? b.hiy : b.hiz;
+        float L = INFINITY, H = -INFINITY;
+        bool finite = true;
+        for(int k = 0; k < 4; k++)
+        {
+            if(b.child[k] == kInvalid) continue;
+            L = MinF(L, lo[k]);
+            H = MaxF(H, hi[k]);
+            finite = finite && isfinite(lo[k]) && isfinite(hi[k]);
+        }
+        const double m = 4.8e-7 * double(MaxF(fabsf(L), fabsf(H)));
+        float o = float(double(L) - 2.0 * m);
+        while(finite && double(o) > double(L) - m) o = nextafterf(o, -INFINITY);
+        float s = MaxF(float((double(H) + 2.0 * m - double(o)) / 255.0), 1e-30f);
+        while(finite && double(o) + 255.0 * double(s) < double(H) + m) s = nextafterf(s, INFINITY);
+        // a plane that is not finite: NaN leaves the walk's interval unbounded
+        if(!finite || !isfinite(o) || !isfinite(s)) o = NAN;
+        uint32_t wl = 0xFFFFFFFFu, wh = 0u;         // empty slots: lo > hi
+        for(int k = 0; k < 4 && !isnan(o); k++)
+        {
+            if(b.child[k] == kInvalid) continue;
+            const double l = double(lo[k]) - m, h = double(hi[k]) + m;
+            int ql = int(floor((l - double(o)) / double(s)));
+            int qh = int(ceil((h - double(o)) / double(s)));
+            ql = max(0, min(255, ql));
+            qh = max(0, min(255, qh));
+            while(ql > 0 && double(o) + double(ql) * double(s) > l) ql--;
+            while(qh < 255 && double(o) + double(qh) * double(s) < h) qh++;
+            wl = (wl & ~(0xFFu << (8 * k))) | (uint32_t(ql) << (8 * k));
+            wh |= uint32_t(qh) << (8 * k);
+        }
+        q.o[a] = o;
+        q.s[a] = s;
+        words[2 * a] = wl;
+        words[2 * a + 1] = wh;
+    }
+    q.qlox = words[0]; q.qhix = words[1]; q.qloy = words[2];
+    q.qhiy = words[3]; q.qloz = words[4]; q.qhiz = words[5];
+    out[i] = q;
+}
+
+int QuantizeNodes(const BNode4* dNodes, uint32_t n, QNode4* dOut, hipStream_t s)
+{
+    if(n == 0) return MRAY_OK;
+    KQuantizeNodes<<<DivUp(n, kTPB), kTPB, 0, s>>>(dNodes, n, dOut);
+    MRAY_HIP_CHECK(hipGetLastError());
+    return MRAY_OK;
+}
+
 int LaunchGatherSoup(const float* dPos, const uint32_t* dIdx, const uint8_t* dCull,
                      const uint32_t* dLeafOrder, uint32_t n, SoupTri* dSoup, hipStream_t s)
 {

@@ -33,7 +33,7 @@ int BuildInstanced(MRayInstScene* sc, const MRayAccel* const* meshes, uint32_t m
                    const MRayInstance* inst, uint32_t n, const MRayInstEnv& env)
 {
     MRayBatchScene& mb = sc->meshes;
-    MRAY_TRY(BuildBatchScene(&mb, meshes, meshCount));
+    MRAY_TRY(BuildBatchScene(&mb, meshes, meshCount, true));
     if(mb.width != 4)
     {
         SetError("instanced_scene_create: meshes need 4-wide trees");

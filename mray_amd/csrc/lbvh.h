@@ -45,6 +45,21 @@ struct alignas(128) BNode4
 };
 static_assert(sizeof(BNode4) == 128, "BNode4 must be one 128-byte line");
 
+// The node the walks read: BNode4 with its boxes quantised to 8 bits per plane
+// on a grid of the node's own (plane p of axis a = o[a] + q * s[a]), half a
+// line.  Boxes only grow: every plane stands at least 8 * 2^-24 times the
+// node's largest coordinate outside the exact one (QuantizeNodes), which
+// covers the rounding of the walk's slab test.  Bytes k of qlo / qhi: child k.
+struct alignas(64) QNode4
+{
+    float o[3], s[3];
+    uint32_t qlox, qhix, qloy, qhiy, qloz, qhiz;
+    uint32_t child[4];
+};
+static_assert(sizeof(QNode4) == 64, "QNode4 must be half a 128-byte line");
+// collapse.hip
+int QuantizeNodes(const BNode4* dNodes, uint32_t n, QNode4* dOut, hipStream_t s);
+
 static constexpr uint32_t kLeafCountShift = 26;
 static constexpr uint32_t kLeafStartMask = (1u << kLeafCountShift) - 1u;
 // Triangles per leaf slot.  One: every triangle gets its own box in its

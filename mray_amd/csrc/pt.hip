@@ -840,11 +840,11 @@ KRefillApply(SlotSoA S, RenderConst rc, const uint4* __restrict__ blockOff,
 // Closest hit
 // ---------------------------------------------------------------------------
 template<int W, bool COUNT, bool BATCH, int TPB = kTraceTPB, bool INST = false>
-__global__ void __launch_bounds__(TPB)
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(INST || W != kNodesQ4 ? 5 : 7, 8)))
 KTrace(TraceCtx ctx, SlotSoA S, const uint32_t* __restrict__ active, Sched* __restrict__ sched,
        const ViewGPU* __restrict__ views, uint32_t* __restrict__ ctr)
 {
-    __shared__ uint2 lstack[kLdsStack * TPB];
+    __shared__ uint2 lstack[(INST ? kLdsStackInst : kLdsStack) * TPB];
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t n = sched->activeCount;
     if(gtid == 0) AdvanceCounter(sched, n);
@@ -1799,12 +1799,12 @@ KShadeQ(SlotSoA S, RenderConst rc, const uint32_t* __restrict__ queues,
 // KCAccumulateShadowRaysPT: a shadow ray that reaches its light point adds
 // its precomputed NEE radiance to the path.
 template<int W, bool BATCH, int TPB = kTraceTPB, bool INST = false, bool COUNT = false>
-__global__ void __launch_bounds__(TPB)
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(INST || W != kNodesQ4 ? 5 : 8, 8)))
 KShadow(TraceCtx ctx, SlotSoA S, const uint32_t* __restrict__ shadowQ, Sched* __restrict__ sched,
         const ViewGPU* __restrict__ views, NrcRenderState nrc, uint32_t* __restrict__ ctr,
         uint32_t N)
 {
-    __shared__ uint2 lstack[kLdsStack * TPB];
+    __shared__ uint2 lstack[(INST ? kLdsStackInst : kLdsStack) * TPB];
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t cap = ShadowShardCap(N);
     Shards g;
@@ -2114,7 +2114,17 @@ static void LaunchTrace(MRayRenderer* r, hipStream_t s)
     if(ctx.width == 8) KTrace<8, COUNT, BATCH><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dActive, r->dSched, r->dViews, r->dCtr);
     else if(r->params.flags & MRAY_RENDER_LANE_REFILL)
         KTraceRefill<COUNT, BATCH><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dActive, r->dSched, r->dViews, r->dCtr);
-    else KTrace<4, COUNT, BATCH><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dActive, r->dSched, r->dViews, r->dCtr);
+    else
+    {
+        // counted walks are the QNode4 ones, like the lane-refill kernel's
+        if constexpr(!BATCH && !COUNT)
+            if(ctx.exact)
+            {
+                KTrace<kNodesB4, false, false><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dActive, r->dSched, r->dViews, r->dCtr);
+                return;
+            }
+        KTrace<4, COUNT, BATCH><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dActive, r->dSched, r->dViews, r->dCtr);
+    }
 }
 
 template<bool COUNT, bool BATCH, bool INST>
@@ -2138,7 +2148,16 @@ static void LaunchShadow(MRayRenderer* r, hipStream_t s)
         }
     }
     if(ctx.width == 8) KShadow<8, BATCH, kTraceTPB, false, COUNT><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dShadowQ, r->dSched, r->dViews, r->rc.nrc, r->dCtr, r->rc.N);
-    else KShadow<4, BATCH, kTraceTPB, false, COUNT><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dShadowQ, r->dSched, r->dViews, r->rc.nrc, r->dCtr, r->rc.N);
+    else
+    {
+        if constexpr(!BATCH && !COUNT)
+            if(ctx.exact)
+            {
+                KShadow<kNodesB4, false><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dShadowQ, r->dSched, r->dViews, r->rc.nrc, r->dCtr, r->rc.N);
+                return;
+            }
+        KShadow<4, BATCH, kTraceTPB, false, COUNT><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dShadowQ, r->dSched, r->dViews, r->rc.nrc, r->dCtr, r->rc.N);
+    }
 }
 
 // Slot blocks up to which a block sums the earlier blocks' counts itself:
@@ -2511,8 +2530,10 @@ static int SizeLaunches(MRayRenderer* r)
     {
         r->traceBlocks = uint32_t(w8 ? resident(KTrace<8, false, false>, tpb, maxTraceBlocks)
                                 : refill ? resident(KTraceRefill<false, false>, tpb, maxTraceBlocks)
+                                : r->ctx.exact ? resident(KTrace<kNodesB4, false, false>, tpb, maxTraceBlocks)
                                          : resident(KTrace<4, false, false>, tpb, maxTraceBlocks));
         r->shadowBlocks = uint32_t(w8 ? resident(KShadow<8, false>, tpb, maxTraceBlocks)
+                                : r->ctx.exact ? resident(KShadow<kNodesB4, false>, tpb, maxTraceBlocks)
                                       : resident(KShadow<4, false>, tpb, maxTraceBlocks));
     }
     else if(tpb == 128)

@@ -87,6 +87,7 @@ struct MRayAccel
     float* dBinBoxes = nullptr;
     uint32_t* dBinRange = nullptr;
     mray::BNode4* dNodes = nullptr;
+    mray::QNode4* dQNodes = nullptr;   // what the walks read (width 4)
     mray::CNode8* dCNodes = nullptr;
     mray::SoupTri* dSoup = nullptr;
     mray::TraceCtx ctx{};
@@ -152,5 +153,6 @@ struct MRayInstScene
 namespace mray
 {
 int UploadSceneData(MRayAccel* a, const MRaySceneDesc* s);
-int BuildBatchScene(MRayBatchScene* b, const MRayAccel* const* accels, uint32_t count);
+// `instanced`: the trees are walked below an instance tree (BNode4 nodes).
+int BuildBatchScene(MRayBatchScene* b, const MRayAccel* const* accels, uint32_t count, bool instanced);
 }

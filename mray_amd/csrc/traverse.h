@@ -1,5 +1,6 @@
-// Closest-hit / any-hit traversal of the wide BVH on gfx950: 4-wide nodes
-// with fp32 boxes (BNode4) or compressed 8-wide nodes (CNode8).
+// Closest-hit / any-hit traversal of the wide BVH on gfx950: 4-wide nodes with
+// boxes quantised to 8 bits (QNode4), 4-wide nodes with fp32 boxes (BNode4:
+// small trees and instance walks) or compressed 8-wide nodes (CNode8).
 //
 // One lane per ray.  The traversal stack holds (node, tNear) pairs: its first
 // kLdsStack entries live in LDS (rows of 64 per wave, conflict-free), deeper ones
@@ -13,11 +14,22 @@
 #include "common.h"
 #include "lbvh.h"
 
+#include <type_traits>
+
 namespace mray
 {
 
 static constexpr uint32_t kTraceTPB = 256;
-static constexpr uint32_t kLdsStack = 12;
+// Stack entries per lane in LDS: 20 KiB a block of 256 let 8 blocks share a CU;
+// the instance walks' two trees run deeper and their registers allow 5.
+static constexpr uint32_t kLdsStack = 10;
+static constexpr uint32_t kLdsStackInst = 12;
+// One-scene trees of at most this many nodes are walked on BNode4: where loads
+// are near (the nodes a CU needs sit in its 32 KiB L1) decoding a QNode4 is the
+// longer way.  Cornell boxes at 128^2 / 512^2 x 4, QNode4 against BNode4:
+// 19 nodes +6 / +6 %, 436 +4 / +2 %, 1394 +3 / +1 %, 6119 +1.5 / -0.3 %,
+// 30573 0 / -1.5 %.
+static constexpr uint32_t kExactNodes = 4096;
 
 // One instance of a mesh in a two-level scene: a TRS transform (rotation
 // quaternion, per-axis scale, translation) object -> world, its inverse as
@@ -37,7 +49,8 @@ struct InstGPU
 
 struct TraceCtx
 {
-    const BNode4* __restrict__ nodes;   // width 4
+    const BNode4* __restrict__ nodes;   // width 4, instance walks
+    const QNode4* __restrict__ qnodes;  // width 4
     const CNode8* __restrict__ cnodes;  // width 8
     const SoupTri* __restrict__ soup;
     uint2* __restrict__ gstack;      // [gstackDepth][gridThreads] (node, tNear bits)
@@ -45,6 +58,7 @@ struct TraceCtx
     uint32_t gridThreads;
     uint32_t maxVisits;              // node count: no correct traversal visits more
     uint32_t width;                  // 4 or 8
+    uint32_t exact;                  // width 4: walk `nodes` (kExactNodes)
     // two-level scenes only: instance tree over world boxes, its leaf
     // positions' instances, the instance table
     const BNode4* __restrict__ tlas;
@@ -108,14 +122,61 @@ __device__ __forceinline__ RayPre MakeRayPre(V3 o, V3 d)
     return r;
 }
 
-// Conservative slab test of the four child boxes (Ize 2013, "Robust BVH Ray
-// Traversal"): near/far planes picked by direction sign, t = (plane - o) * inv
-// with one rounding per operation, and the far bound scaled by 1 + 2*gamma(4).
-// A ray parallel to an axis whose origin lies exactly on a slab plane makes
-// (plane - o) * inv = 0 * inf = NaN; fmaxf/fminf drop the NaN operand, so
-// that plane leaves the interval unbounded -- the ray lies in the box face and
-// must reach its triangles.  tNear[k] = +inf on a miss.
-__device__ __forceinline__ void SlabTest4(const BNode4* __restrict__ np, const RayPre& r,
+// A ray set up for QNode4 trees: t of plane p is fma(p, inv, off), near planes
+// with offN, far with offF.
+struct RayQ : RayPre
+{
+    V3 offN, offF;
+};
+
+// One axis of RayQ: the exact reciprocal, and -o * inv less and plus a bound on
+// its own rounding (SlabTestQ).  A direction component under 1e-30, zero
+// included, takes +-1e30 for its reciprocal: over any distance such a ray
+// stays on its origin's side of a plane, and the finite value keeps the test
+// free of inf - inf.  A plane it starts in bounds it nowhere, so its margin is
+// wider by 1e22 (1e-8 in position).
+__device__ __forceinline__ void MakeAxis(float o, float d, float& inv, float& offN, float& offF, uint32_t& s)
+{
+    const bool parallel = fabsf(d) < 1e-30f;
+    inv = parallel ? copysignf(1e30f, d) : 1.0f / d;
+    const float off = -o * inv;
+    const float e = fabsf(off) * 3e-7f + (parallel ? 1e22f : 0.0f);   // 5 * 2^-24, rounded up
+    offN = off - e;
+    offF = off + e;
+    s = signbit(d) ? 1u : 0u;
+}
+__device__ __forceinline__ RayQ MakeRayQ(V3 o, V3 d)
+{
+    RayQ r;
+    r.o = o;
+    r.d = d;
+    MakeAxis(o.x, d.x, r.inv.x, r.offN.x, r.offF.x, r.sx);
+    MakeAxis(o.y, d.y, r.inv.y, r.offN.y, r.offF.y, r.sy);
+    MakeAxis(o.z, d.z, r.inv.z, r.offN.z, r.offF.z, r.sz);
+    return r;
+}
+
+// Conservative slab test of a BNode4's child boxes, near / far planes picked
+// by direction sign.  With RayPre (instance walks; Ize 2013, "Robust BVH Ray
+// Traversal"): t = (plane - o) * inv with one rounding per operation, and the
+// far bound scaled by 1 + 2*gamma(4).  A ray parallel to an axis whose origin
+// lies exactly on a slab plane makes (plane - o) * inv = 0 * inf = NaN;
+// fmaxf/fminf drop the NaN operand, so that plane leaves the interval
+// unbounded -- the ray lies in the box face and must reach its triangles.
+// With RayQ: one fused multiply-add a plane (the error bound is SlabTestQ's
+// without the node's part; small trees' walks 3 % shorter than with RayPre).
+// tNear[k] = +inf on a miss.
+__device__ __forceinline__ float SlabNear(float tMin, float x, float y, float z)
+{
+    return MaxF(MaxF(tMin, x), MaxF(y, z));
+}
+__device__ __forceinline__ float SlabFar(float tMax, float x, float y, float z)
+{
+    const float grow = 1.0f + 2.0f * 5.96e-8f * 4.0f;
+    return MinF(MinF(tMax, x), MinF(y, z)) * grow;
+}
+template<class RAY>
+__device__ __forceinline__ void SlabTest4(const BNode4* __restrict__ np, const RAY& r,
                                           float tMin, float tMax, float tNear[4], uint4& child)
 {
     const float4* q = reinterpret_cast<const float4*>(np);
@@ -123,20 +184,86 @@ __device__ __forceinline__ void SlabTest4(const BNode4* __restrict__ np, const R
     float4 ny = q[2 + r.sy], fy = q[3 - r.sy];
     float4 nz = q[4 + r.sz], fz = q[5 - r.sz];
     child = reinterpret_cast<const uint4*>(np)[6];
-    const float grow = 1.0f + 2.0f * 5.96e-8f * 4.0f;
     float nX[4] = {nx.x, nx.y, nx.z, nx.w}, fX[4] = {fx.x, fx.y, fx.z, fx.w};
     float nY[4] = {ny.x, ny.y, ny.z, ny.w}, fY[4] = {fy.x, fy.y, fy.z, fy.w};
     float nZ[4] = {nz.x, nz.y, nz.z, nz.w}, fZ[4] = {fz.x, fz.y, fz.z, fz.w};
     #pragma unroll
     for(int k = 0; k < 4; k++)
     {
-        float x0 = (nX[k] - r.o.x) * r.inv.x, x1 = (fX[k] - r.o.x) * r.inv.x;
-        float y0 = (nY[k] - r.o.y) * r.inv.y, y1 = (fY[k] - r.o.y) * r.inv.y;
-        float z0 = (nZ[k] - r.o.z) * r.inv.z, z1 = (fZ[k] - r.o.z) * r.inv.z;
-        float tn = MaxF(MaxF(tMin, x0), MaxF(y0, z0));
-        float tf = MinF(MinF(tMax, x1), MinF(y1, z1)) * grow;
+        float x0, x1, y0, y1, z0, z1;
+        if constexpr(std::is_same_v<RAY, RayQ>)
+        {
+            x0 = Fma(nX[k], r.inv.x, r.offN.x); x1 = Fma(fX[k], r.inv.x, r.offF.x);
+            y0 = Fma(nY[k], r.inv.y, r.offN.y); y1 = Fma(fY[k], r.inv.y, r.offF.y);
+            z0 = Fma(nZ[k], r.inv.z, r.offN.z); z1 = Fma(fZ[k], r.inv.z, r.offF.z);
+        }
+        else
+        {
+            x0 = (nX[k] - r.o.x) * r.inv.x; x1 = (fX[k] - r.o.x) * r.inv.x;
+            y0 = (nY[k] - r.o.y) * r.inv.y; y1 = (fY[k] - r.o.y) * r.inv.y;
+            z0 = (nZ[k] - r.o.z) * r.inv.z; z1 = (fZ[k] - r.o.z) * r.inv.z;
+        }
+        const float tn = SlabNear(tMin, x0, y0, z0), tf = SlabFar(tMax, x1, y1, z1);
         // empty slots store lo = +inf, hi = -inf: their near bound is +inf
         // and far bound -inf for every direction sign, so they always miss
+        tNear[k] = (tn <= tf) ? tn : INFINITY;
+    }
+}
+
+// The node types a walk is compiled for (template parameter W).
+constexpr int kNodesQ4 = 4;      // QNode4
+constexpr int kNodesB4 = 5;      // BNode4
+constexpr int kNodesC8 = 8;      // CNode8
+constexpr int WidthOf(int W) { return (W == kNodesC8) ? 8 : 4; }
+
+// The ray of such a walk.
+template<int W>
+__device__ __forceinline__ auto MakeRay(V3 o, V3 d)
+{
+    if constexpr(W == kNodesC8) return MakeRayPre(o, d);
+    else return MakeRayQ(o, d);
+}
+
+// Conservative slab test of a QNode4's child boxes: four 16-byte loads where a
+// BNode4 takes seven, a convert and a fused multiply-add per plane.  Plane
+// o + q s in t is q a + b with a = s inv, b = o inv + off.  With u = 2^-24,
+// inv, a and the final fma carry relative errors of u, off and b absolute ones
+// of u |ray.o inv| and u |o inv|: the ray's offsets cover five u |ray.o inv|,
+// the node's planes stand 8 u of the node's largest coordinate outside the
+// exact box, and the far bound's factor 1 + 8 u covers the relative part of
+// both bounds as in SlabTest4.  Values that overflow are NaN, which
+// fmaxf/fminf drop: that plane leaves the interval unbounded.
+// tNear[k] = +inf on a miss.
+// Closest-hit walks are bound by the rate of these loads and of VALU issue
+// together; 64-byte nodes also leave 64-72 VGPRs, so 7 waves per SIMD run
+// instead of 6, on 10 LDS stack entries.  1080p terrain: trace 34.9 -> 32.4 ms,
+// shadow 9.6 -> 9.0 ms; 2.8 M rays of a caller 893 -> 690 us; six Cornell
+// scenes' trace 21.7 -> 20.9 ms.  Instance walks run on BNode4: their object-space rays are
+// set up again at every instance, and the wider ray state costs them a wave
+// (trace 5.35 -> 5.55 ms).
+__device__ __forceinline__ float ByteF(uint32_t w, int k) { return float((w >> (8 * k)) & 0xFFu); }
+__device__ __forceinline__ void SlabTestQ(const QNode4* __restrict__ np, const RayQ& r,
+                                          float tMin, float tMax, float tNear[4], uint4& child)
+{
+    const uint4* q = reinterpret_cast<const uint4*>(np);
+    const uint4 h0 = q[0], h1 = q[1], h2 = q[2];
+    child = q[3];
+    const float ox = __uint_as_float(h0.x), oy = __uint_as_float(h0.y), oz = __uint_as_float(h0.z);
+    const float ax = __uint_as_float(h0.w) * r.inv.x, ay = __uint_as_float(h1.x) * r.inv.y,
+                az = __uint_as_float(h1.y) * r.inv.z;
+    const float nbx = Fma(ox, r.inv.x, r.offN.x), fbx = Fma(ox, r.inv.x, r.offF.x);
+    const float nby = Fma(oy, r.inv.y, r.offN.y), fby = Fma(oy, r.inv.y, r.offF.y);
+    const float nbz = Fma(oz, r.inv.z, r.offN.z), fbz = Fma(oz, r.inv.z, r.offF.z);
+    const uint32_t nx = r.sx ? h1.w : h1.z, fx = r.sx ? h1.z : h1.w;
+    const uint32_t ny = r.sy ? h2.y : h2.x, fy = r.sy ? h2.x : h2.y;
+    const uint32_t nz = r.sz ? h2.w : h2.z, fz = r.sz ? h2.z : h2.w;
+    #pragma unroll
+    for(int k = 0; k < 4; k++)
+    {
+        const float tn = SlabNear(tMin, Fma(ByteF(nx, k), ax, nbx), Fma(ByteF(ny, k), ay, nby),
+                                  Fma(ByteF(nz, k), az, nbz));
+        const float tf = SlabFar(tMax, Fma(ByteF(fx, k), ax, fbx), Fma(ByteF(fy, k), ay, fby),
+                                 Fma(ByteF(fz, k), az, fbz));
         tNear[k] = (tn <= tf) ? tn : INFINITY;
     }
 }
@@ -191,9 +318,10 @@ __device__ __forceinline__ void SlabTest8(const CNode8* __restrict__ np, const R
 // LDS stack layout: each wave owns kLdsStack rows of 64 entries, entry sp
 // of a lane at sp * 64 + StackLane() (a shift, no multiply by the block
 // size; a row is 64 consecutive 8-byte entries, conflict-free).
+template<uint32_t LDS>
 __device__ __forceinline__ uint32_t StackLane()
 {
-    return (threadIdx.x >> 6) * (kLdsStack * 64u) + (threadIdx.x & 63u);
+    return (threadIdx.x >> 6) * (LDS * 64u) + (threadIdx.x & 63u);
 }
 
 // One traversal-stack entry: the first kLdsStack levels in LDS, deeper ones
@@ -203,27 +331,29 @@ __device__ __forceinline__ uint32_t StackLane()
 // each lane picks its memory.  The empty asm statement (a compiler barrier;
 // it emits nothing) keeps that slow path's LDS and global accesses apart:
 // merged, they would become one access through a generic pointer.
+template<uint32_t LDS>
 __device__ __forceinline__ void StackPut(const TraceCtx& ctx, uint2* lstack, uint32_t sp,
                                          uint32_t lb, uint32_t gtid, uint2 v)
 {
-    if(__builtin_expect(__ballot(sp >= kLdsStack) == 0ull, 1)) lstack[sp * 64u + lb] = v;
-    else if(sp < kLdsStack) lstack[sp * 64u + lb] = v;
+    if(__builtin_expect(__ballot(sp >= LDS) == 0ull, 1)) lstack[sp * 64u + lb] = v;
+    else if(sp < LDS) lstack[sp * 64u + lb] = v;
     else
     {
-        ctx.gstack[size_t(sp - kLdsStack) * ctx.gridThreads + gtid] = v;
+        ctx.gstack[size_t(sp - LDS) * ctx.gridThreads + gtid] = v;
         asm volatile("" ::: "memory");
     }
 }
 
+template<uint32_t LDS>
 __device__ __forceinline__ uint2 StackGet(const TraceCtx& ctx, const uint2* lstack, uint32_t sp,
                                           uint32_t lb, uint32_t gtid)
 {
     uint2 v;
-    if(__builtin_expect(__ballot(sp >= kLdsStack) == 0ull, 1)) v = lstack[sp * 64u + lb];
-    else if(sp < kLdsStack) v = lstack[sp * 64u + lb];
+    if(__builtin_expect(__ballot(sp >= LDS) == 0ull, 1)) v = lstack[sp * 64u + lb];
+    else if(sp < LDS) v = lstack[sp * 64u + lb];
     else
     {
-        v = ctx.gstack[size_t(sp - kLdsStack) * ctx.gridThreads + gtid];
+        v = ctx.gstack[size_t(sp - LDS) * ctx.gridThreads + gtid];
         asm volatile("" ::: "memory");
     }
     return v;
@@ -237,7 +367,7 @@ __device__ __forceinline__ uint2 StackGet(const TraceCtx& ctx, const uint2* lsta
 // stack grows only on a real push (a write above the top is dead).  The
 // 8-wide walk and the two-level walk use the guarded pushes only (their
 // branch-free form spilled SGPRs, and measured slower, respectively).
-template<int W, bool BRANCH_FREE = true>
+template<int W, uint32_t LDS, bool BRANCH_FREE>
 __device__ __forceinline__ void PushFarFirst(const TraceCtx& ctx, uint2* lstack, uint32_t& sp,
                                              uint32_t spMax, uint32_t lb, uint32_t gtid, const float (&tn)[W],
                                              const uint32_t (&c)[W], uint32_t cand,
@@ -245,7 +375,7 @@ __device__ __forceinline__ void PushFarFirst(const TraceCtx& ctx, uint2* lstack,
 {
     next = kInvalid;
     nextT = 0.0f;
-    if(BRANCH_FREE && __builtin_expect(__ballot(sp + uint32_t(W - 1) > kLdsStack) == 0ull, 1))
+    if(BRANCH_FREE && __builtin_expect(__ballot(sp + uint32_t(W - 1) > LDS) == 0ull, 1))
     {
         #pragma unroll
         for(int k = W - 1; k >= 0; k--)
@@ -268,7 +398,7 @@ __device__ __forceinline__ void PushFarFirst(const TraceCtx& ctx, uint2* lstack,
             if(!((cand >> k) & 1u)) continue;
             if(next != kInvalid && sp < spMax)   // sp < spMax: sized for every level
             {
-                StackPut(ctx, lstack, sp, lb, gtid, make_uint2(next, __float_as_uint(nextT)));
+                StackPut<LDS>(ctx, lstack, sp, lb, gtid, make_uint2(next, __float_as_uint(nextT)));
                 sp++;
             }
             next = c[k];
@@ -311,6 +441,9 @@ __device__ __forceinline__ bool TestLeafRange(const SoupTri* __restrict__ soup, 
                                               const RayPre& r, float tMin, float tMax,
                                               HitRec& best, uint32_t* triTests)
 {
+    // an empty slot of a node whose extent is lost in the slab test's margins
+    // (255 / 0 bytes do not decode to an empty box there)
+    if(leaf == kInvalid) return false;
     uint32_t first = leaf & kLeafStartMask;
     // every tree is collapsed with kLeafMax triangles per leaf at most
     uint32_t cnt = (kLeafMax == 1u) ? 1u : ((leaf & ~kLeafFlag) >> kLeafCountShift) + 1u;
@@ -345,7 +478,7 @@ __device__ __forceinline__ bool TestLeafRange(const SoupTri* __restrict__ soup, 
 // TraceW's loop does, so a walk finds TraceW's hit.
 struct Walk
 {
-    RayPre r;
+    RayQ r;
     float tMin, tMax;
     HitRec best;
     uint32_t node;       // the node the next step visits
@@ -355,7 +488,7 @@ struct Walk
 __device__ __forceinline__ void WalkInit(Walk& w, V3 o, V3 d, float tMin, float tMax, uint32_t root,
                                          uint32_t sp0)
 {
-    w.r = MakeRayPre(o, d);
+    w.r = MakeRayQ(o, d);
     w.tMin = tMin;
     w.tMax = tMax;
     w.best = HitRec{kInvalid, INFINITY, 0.0f, 0.0f};
@@ -373,7 +506,8 @@ template<int W, bool ANY_HIT, bool COUNT>
 __device__ __forceinline__ bool WalkStep(const TraceCtx& ctx, uint2* lstack, uint32_t gtid, Walk& w,
                                          uint32_t sp0, uint32_t* nodeVisits, uint32_t* triTests)
 {
-    const uint32_t lb = StackLane();
+    static_assert(W == 4, "the walk's ray is a QNode4 tree's");
+    const uint32_t lb = StackLane<kLdsStack>();
     const uint32_t spMax = kLdsStack + ctx.gstackDepth;
     const float kGrow = 1.0000005f;
     if(COUNT) (*nodeVisits)++;
@@ -381,13 +515,9 @@ __device__ __forceinline__ bool WalkStep(const TraceCtx& ctx, uint2* lstack, uin
     float curMax = (best.prim == kInvalid) ? w.tMax : best.t;
     float tn[W];
     uint32_t c[W];
-    if constexpr(W == 8) SlabTest8(ctx.cnodes + w.node, w.r, w.tMin, curMax, tn, c);
-    else
-    {
-        uint4 ch;
-        SlabTest4(ctx.nodes + w.node, w.r, w.tMin, curMax, tn, ch);
-        c[0] = ch.x; c[1] = ch.y; c[2] = ch.z; c[3] = ch.w;
-    }
+    uint4 ch;
+    SlabTestQ(ctx.qnodes + w.node, w.r, w.tMin, curMax, tn, ch);
+    c[0] = ch.x; c[1] = ch.y; c[2] = ch.z; c[3] = ch.w;
     SortNear<W>(tn, c);
     // as in TraceW: inner children farthest first, each pushing the one
     // found before it; then the leaves nearest first
@@ -401,7 +531,7 @@ __device__ __forceinline__ bool WalkStep(const TraceCtx& ctx, uint2* lstack, uin
         if(next != kInvalid && sp < spMax)   // sp < spMax: sized (W-1) per level
         {
             const uint2 v = make_uint2(next, __float_as_uint(nextT));
-            StackPut(ctx, lstack, sp, lb, gtid, v);
+            StackPut<kLdsStack>(ctx, lstack, sp, lb, gtid, v);
             sp++;
         }
         next = c[k];
@@ -426,7 +556,7 @@ __device__ __forceinline__ bool WalkStep(const TraceCtx& ctx, uint2* lstack, uin
     {
         sp--;
         uint2 v;
-        v = StackGet(ctx, lstack, sp, lb, gtid);
+        v = StackGet<kLdsStack>(ctx, lstack, sp, lb, gtid);
         // drop subtrees that start beyond the closest hit so far
         if(!ANY_HIT && best.prim != kInvalid && __uint_as_float(v.y) > best.t * kGrow) continue;
         next = v.x;
@@ -447,30 +577,32 @@ __device__ __forceinline__ HitRec TraceW(const TraceCtx& ctx, uint2* lstack, uin
                                          uint32_t* triTests = nullptr, uint32_t sp0 = 0)
 {
     HitRec best{kInvalid, INFINITY, 0.0f, 0.0f};
-    RayPre r = MakeRayPre(o, d);
+    const auto r = MakeRay<W>(o, d);
     uint32_t sp = sp0;
     uint32_t node = root;
-    const uint32_t lb = StackLane();
+    const uint32_t lb = StackLane<kLdsStack>();
     const uint32_t spMax = kLdsStack + ctx.gstackDepth;
     const float kGrow = 1.0000005f;
     for(uint32_t visits = 0; visits < ctx.maxVisits; visits++)
     {
         if(COUNT) (*nodeVisits)++;
         float curMax = (best.prim == kInvalid) ? tMax : best.t;
-        float tn[W];
-        uint32_t c[W];
-        if constexpr(W == 8) SlabTest8(ctx.cnodes + node, r, tMin, curMax, tn, c);
+        constexpr int N = WidthOf(W);
+        float tn[N];
+        uint32_t c[N];
+        if constexpr(W == kNodesC8) SlabTest8(ctx.cnodes + node, r, tMin, curMax, tn, c);
         else
         {
             uint4 ch;
-            SlabTest4(ctx.nodes + node, r, tMin, curMax, tn, ch);
+            if constexpr(W == kNodesQ4) SlabTestQ(ctx.qnodes + node, r, tMin, curMax, tn, ch);
+            else SlabTest4(ctx.nodes + node, r, tMin, curMax, tn, ch);
             c[0] = ch.x; c[1] = ch.y; c[2] = ch.z; c[3] = ch.w;
         }
-        SortNear<W>(tn, c);
+        SortNear<N>(tn, c);
         // hit children: leaves are tested below, inner ones go on the stack
         uint32_t leafMask = 0, cand = 0;
         #pragma unroll
-        for(int k = 0; k < W; k++)
+        for(int k = 0; k < N; k++)
         {
             const bool hit = tn[k] != INFINITY, leaf = (c[k] & kLeafFlag) != 0u;
             leafMask |= (hit && leaf) ? (1u << k) : 0u;
@@ -478,7 +610,7 @@ __device__ __forceinline__ HitRec TraceW(const TraceCtx& ctx, uint2* lstack, uin
         }
         uint32_t next;
         float nextT;
-        PushFarFirst<W, W == 4>(ctx, lstack, sp, spMax, lb, gtid, tn, c, cand, next, nextT);
+        PushFarFirst<N, kLdsStack, N == 4>(ctx, lstack, sp, spMax, lb, gtid, tn, c, cand, next, nextT);
         // the node's leaves, nearest first: a wave runs as many triangle
         // tests as its lane with the most leaves here, not one per child
         // position that any lane has a leaf in
@@ -489,7 +621,7 @@ __device__ __forceinline__ HitRec TraceW(const TraceCtx& ctx, uint2* lstack, uin
             uint32_t ck = c[0];
             float tk = tn[0];
             #pragma unroll
-            for(int j = 1; j < W; j++)
+            for(int j = 1; j < N; j++)
             {
                 ck = (k == j) ? c[j] : ck;
                 tk = (k == j) ? tn[j] : tk;
@@ -507,7 +639,7 @@ __device__ __forceinline__ HitRec TraceW(const TraceCtx& ctx, uint2* lstack, uin
         while(next == kInvalid && sp > sp0)
         {
             sp--;
-            uint2 v = StackGet(ctx, lstack, sp, lb, gtid);
+            uint2 v = StackGet<kLdsStack>(ctx, lstack, sp, lb, gtid);
             // drop subtrees that start beyond the closest hit so far
             if(!ANY_HIT && best.prim != kInvalid && __uint_as_float(v.y) > best.t * kGrow) continue;
             next = v.x;
@@ -548,8 +680,8 @@ __device__ __forceinline__ HitRec TraceInstFlat(const TraceCtx& ctx, uint2* lsta
     const BNode4* tree = ctx.tlas;
     uint32_t sp = 0;
     uint32_t node = 0;
-    const uint32_t lb = StackLane();
-    const uint32_t spMax = kLdsStack + ctx.gstackDepth;
+    const uint32_t lb = StackLane<kLdsStackInst>();
+    const uint32_t spMax = kLdsStackInst + ctx.gstackDepth;
     const float kGrow = 1.0000005f;
     for(uint32_t visits = 0; visits < ctx.instWalkVisits; visits++)
     {
@@ -572,7 +704,7 @@ __device__ __forceinline__ HitRec TraceInstFlat(const TraceCtx& ctx, uint2* lsta
         }
         uint32_t next;
         float nextT;
-        PushFarFirst<4, false>(ctx, lstack, sp, spMax, lb, gtid, tn, c, cand, next, nextT);
+        PushFarFirst<4, kLdsStackInst, false>(ctx, lstack, sp, spMax, lb, gtid, tn, c, cand, next, nextT);
         #pragma unroll
         for(int k = 0; k < 4; k++)
         {
@@ -599,7 +731,7 @@ __device__ __forceinline__ HitRec TraceInstFlat(const TraceCtx& ctx, uint2* lsta
         {
             sp--;
             uint2 v;
-            v = StackGet(ctx, lstack, sp, lb, gtid);
+            v = StackGet<kLdsStackInst>(ctx, lstack, sp, lb, gtid);
             if(v.x == kInstReturn)
             {
                 // back from an instance: world ray, instance tree
@@ -620,7 +752,7 @@ __device__ __forceinline__ HitRec TraceInstFlat(const TraceCtx& ctx, uint2* lsta
             const InstGPU& I = ctx.inst[id];
             if(sp >= spMax) break;       // unreachable: the mark has its slot
             const uint2 mark = make_uint2(kInstReturn, 0u);
-            StackPut(ctx, lstack, sp, lb, gtid, mark);
+            StackPut<kLdsStackInst>(ctx, lstack, sp, lb, gtid, mark);
             sp++;
             const float4 a = I.inv[0], b = I.inv[1], e = I.inv[2];
             const V3 lo = {a.x * o.x + a.y * o.y + a.z * o.z + a.w,

@@ -67,6 +67,7 @@ int LaunchCastClosest(const TraceCtx& ctx, const float* dRays, uint32_t n, uint3
     else
     {
         if(w8) KCCastClosest<8, false><<<blocks, kTraceTPB, 0, s>>>(ctx, r, n, dPrim, dT, dBary, nullptr);
+        else if(ctx.exact) KCCastClosest<kNodesB4, false><<<blocks, kTraceTPB, 0, s>>>(ctx, r, n, dPrim, dT, dBary, nullptr);
         else KCCastClosest<4, false><<<blocks, kTraceTPB, 0, s>>>(ctx, r, n, dPrim, dT, dBary, nullptr);
     }
     MRAY_HIP_CHECK(hipGetLastError());
@@ -80,6 +81,7 @@ int LaunchCastVisibility(const TraceCtx& ctx, const float* dRays, uint32_t n, ui
     uint32_t blocks = std::min(ctx.gridThreads / kTraceTPB, DivUp(n, kTraceTPB));
     const float4* r = reinterpret_cast<const float4*>(dRays);
     if(ctx.width == 8) KCCastVisibility<8><<<blocks, kTraceTPB, 0, s>>>(ctx, r, n, dVisible);
+    else if(ctx.exact) KCCastVisibility<kNodesB4><<<blocks, kTraceTPB, 0, s>>>(ctx, r, n, dVisible);
     else KCCastVisibility<4><<<blocks, kTraceTPB, 0, s>>>(ctx, r, n, dVisible);
     MRAY_HIP_CHECK(hipGetLastError());
     return MRAY_OK;

@@ -227,3 +227,54 @@ def test_deep_stack_spills_past_lds(torch_gpu, builder):
     rays[:, 3] = 1e-4
     rays[:, 7] = 3.4e38
     _compare(acc, refcpu.OracleScene(s), rays, brute=True)
+
+
+@pytest.mark.parametrize("cells,offset,flat", [(24, 0.0, True), (96, 0.0, True), (96, 1000.0, False), (96, -3e4, True),
+                                               (200, 0.0, False)])
+def test_node_kinds_equal_brute_force(torch_gpu, cells, offset, flat):
+    """Small trees are walked on exact boxes, larger ones (over 4096 nodes) on
+    boxes quantised to 8 bits: both equal brute force for axis-parallel rays
+    (+0 and -0) that start on box planes, rays along edges and random rays, on
+    flat and bumpy grids, near the origin and far from it."""
+    from mray_amd import native
+    rng = np.random.default_rng(cells)
+    g = np.arange(cells + 1, dtype=np.float32) / cells + np.float32(offset)
+    x, y = np.meshgrid(g, g, indexing="ij")
+    z = np.zeros_like(x) if flat else (0.05 * rng.random(x.shape)).astype(np.float32)
+    pos = np.stack([x, y, z], -1).reshape(-1, 3).astype(np.float32)
+    i, j = np.meshgrid(np.arange(cells), np.arange(cells), indexing="ij")
+    v = (i * (cells + 1) + j).reshape(-1)
+    idx = np.concatenate([np.stack([v, v + cells + 1, v + cells + 2], 1),
+                          np.stack([v, v + cells + 2, v + 1], 1)]).astype(np.uint32)
+    n = len(idx)
+    s = scenes.Scene(positions=pos, tbn=np.tile(np.array([[1, 0, 0, 0]], np.float32), (len(pos), 1)),
+                     indices=idx, surface_keys=np.zeros(n, np.uint32), cull=np.zeros(n, np.uint8),
+                     materials=[{"type": abi.MAT_LAMBERT, "albedo": (1, 1, 1)}],
+                     light_tris=np.zeros(0, np.uint32), light_radiance=np.zeros((0, 3), np.float32),
+                     light_two_sided=np.zeros(0, np.uint8),
+                     camera={"position": (0, 0, 1), "gaze": (0, 0, 0), "up": (0, 1, 0),
+                             "fov": (1.0, 1.0), "nearFar": (0.1, 10.0)})
+    acc = native.Accel(s)
+    print(f"{n} triangles, {acc.info()['wide_nodes']} nodes, offset {offset}", flush=True)
+    assert (acc.info()["wide_nodes"] > 4096) == (cells > 24)
+    down = np.zeros((400, 8), np.float32)
+    down[:, 0:2] = g[rng.integers(0, cells + 1, (400, 2))]     # on vertices and planes
+    down[200:, 0] += np.float32(0.3 / cells)
+    down[:, 2] = 1.0
+    down[:, 6] = -1.0
+    down[:, 7] = 10.0
+    down[::2, 4:6] = -0.0
+    slant = np.zeros((400, 8), np.float32)
+    slant[:, 0:3] = rng.uniform(-0.5, 1.5, (400, 3)) + [offset, offset, 0.6]
+    to = np.stack([g[rng.integers(0, cells + 1, 400)], g[rng.integers(0, cells + 1, 400)], np.zeros(400)], 1)
+    slant[:, 4:7] = to - slant[:, 0:3]                         # through vertices
+    slant[::3, 5] = 0.0
+    slant[::7, 4] = 1e-35
+    slant[:, 7] = 1e6
+    along = np.zeros((100, 8), np.float32)                     # in the grid's plane
+    along[:, 0:3] = np.stack([np.full(100, offset - 0.25), g[rng.integers(0, cells + 1, 100)],
+                              rng.choice([0.0, 0.01], 100)], 1)
+    along[:, 4] = 1.0
+    along[:, 7] = 100.0
+    _compare(acc, refcpu.OracleScene(s), np.concatenate([down, slant, along]).astype(np.float32), brute=True)
+    acc.close()
