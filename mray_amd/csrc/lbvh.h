@@ -30,6 +30,9 @@ int    LaunchLbvhBuild(const uint64_t* dSortedCodes, const uint32_t* dLeafOrder,
 // root and each node's two children split its leaf range at one point.
 bool ValidateBinaryTree(const std::vector<uint32_t>& nodes, const std::vector<uint32_t>& range,
                         uint32_t n);
+// The same of a tree in device memory (dFlag: 4 bytes of scratch); waits for s.
+int    ValidateTreeDevice(const uint32_t* dNodes, const uint32_t* dRange, const uint32_t* dLeafOrder,
+                          uint32_t n, uint32_t* dFlag, hipStream_t s, bool* ok);
 
 // ---------------------------------------------------------------------------
 // 4-wide BVH node: one 128-byte line, child boxes as SoA lanes so a node is

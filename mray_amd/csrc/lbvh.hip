@@ -707,6 +707,41 @@ KCKarras(const uint64_t* __restrict__ codes, const uint32_t* __restrict__ leafOr
     StoreBox(boxes + 6 * size_t(i), RangeBox(lv, uint32_t(lo), uint32_t(hi)));
 }
 
+// ---------------------------------------------------------------------------
+// ValidateBinaryTree on the device, one thread per node: a node's children
+// split its range at one point and name it as their parent.  With the root
+// over all leaves that is the whole tree: a node has one stored parent, so
+// nothing is reached twice, and a walk from the root splits n positions into
+// single leaves, which takes all n - 1 nodes.
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(kTPB)
+KCValidate(const uint32_t* __restrict__ nodes, const uint32_t* __restrict__ range,
+           const uint32_t* __restrict__ leafOrder, uint32_t n, uint32_t* __restrict__ bad)
+{
+    const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+    if(v >= n - 1u) return;
+    const uint32_t lo = range[2 * size_t(v)], hi = range[2 * size_t(v) + 1];
+    bool ok = lo < hi && hi < n && (v != 0u || (lo == 0u && hi == n - 1u));
+    uint32_t mid = lo;
+    for(uint32_t side = 0; side < 2 && ok; side++)
+    {
+        const uint32_t c = nodes[size_t(v) * 3 + side];
+        const uint32_t first = side ? mid + 1u : lo;
+        if(c & kLeafFlag)
+        {
+            ok = (!side || first == hi) && c == (kLeafFlag | leafOrder[first]);
+            mid = first;
+        }
+        else
+        {
+            ok = c != 0u && c < n - 1u && nodes[size_t(c) * 3 + 2] == v && range[2 * size_t(c)] == first;
+            mid = ok ? range[2 * size_t(c) + 1] : 0u;
+            ok = ok && (side ? mid == hi : mid < hi);
+        }
+    }
+    if(!ok) *bad = 1u;
+}
+
 __global__ void __launch_bounds__(kTPB) KCIota(uint32_t* __restrict__ out, uint32_t n)
 {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -901,6 +936,30 @@ int LaunchLbvhBuild(const uint64_t* dSortedCodes, const uint32_t* dLeafOrder,
     KCKarras<<<DivUp(std::max(n - 1, 1u), kTPB), kTPB, 0, s>>>(dSortedCodes, dLeafOrder, int32_t(n), dNodes,
                                                                dNodeRange, lv, dBoxes, strictTie);
     MRAY_HIP_CHECK(hipGetLastError());
+    return MRAY_OK;
+}
+
+int ValidateTreeDevice(const uint32_t* dNodes, const uint32_t* dRange, const uint32_t* dLeafOrder,
+                       uint32_t n, uint32_t* dFlag, hipStream_t s, bool* ok)
+{
+    *ok = false;
+    uint32_t bad = 1u;
+    if(n == 1)
+    {
+        uint32_t node0 = 0;
+        MRAY_HIP_CHECK(hipMemcpyAsync(&node0, dNodes, 4, hipMemcpyDeviceToHost, s));
+        MRAY_HIP_CHECK(hipStreamSynchronize(s));
+        bad = (node0 != (kLeafFlag | 0u)) ? 1u : 0u;
+    }
+    else
+    {
+        MRAY_HIP_CHECK(hipMemsetAsync(dFlag, 0, 4, s));
+        KCValidate<<<DivUp(n - 1u, kTPB), kTPB, 0, s>>>(dNodes, dRange, dLeafOrder, n, dFlag);
+        MRAY_HIP_CHECK(hipGetLastError());
+        MRAY_HIP_CHECK(hipMemcpyAsync(&bad, dFlag, 4, hipMemcpyDeviceToHost, s));
+        MRAY_HIP_CHECK(hipStreamSynchronize(s));
+    }
+    *ok = bad == 0u;
     return MRAY_OK;
 }
 

@@ -218,3 +218,45 @@ def test_stage_lbvh_boxes_at_level_edges(torch_gpu, n):
     rnodes, rboxes = refcpu.lbvh_from_sorted(codes, order, aabbs)
     assert np.array_equal(nodes, rnodes)
     assert np.array_equal(boxes.view(np.uint32), rboxes.view(np.uint32))
+
+
+def test_malformed_reference_tree_is_rebuilt(torch_gpu):
+    """A scene whose triangle centres share few Morton codes in long runs (the
+    reference's Delta gives a malformed tree for them) builds with the strict
+    tie-break, as the device-side check of the first tree demands; hits equal
+    brute force."""
+    from mray_amd import abi, native
+    rng = np.random.default_rng(8)
+    n = 3000
+    # centres on 64 neighbouring cells of the 2^21 grid, spread by two far triangles
+    cell = rng.integers(0, 4, size=(n, 3)).astype(np.float64) * 2.0 ** -21 * 1.00000001
+    tri = rng.uniform(-1e-3, 1e-3, size=(n, 3, 3))
+    tri -= tri.mean(axis=1, keepdims=True)
+    tri += cell[:, None, :]
+    tri[0] += 0.999
+    pos = tri.reshape(-1, 3).astype(np.float32)
+    s = scenes.random_triangles(n, seed=4)
+    s.positions, s.indices = pos, np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+    s.tbn = np.tile(np.array([[1, 0, 0, 0]], np.float32), (3 * n, 1))
+    o = refcpu.OracleScene(s)
+    codes, order, nodes, _, _ = o.lbvh()
+    print("distinct codes", len(np.unique(codes)), "reference tree valid",
+          refcpu.lbvh_tree_valid(np.sort(codes), order), flush=True)
+    assert not refcpu.lbvh_tree_valid(np.sort(codes), order)
+    acc = native.Accel(s, builder="lbvh")
+    _, gorder, gnodes, gboxes = acc.read_lbvh()
+    rays = np.zeros((500, 8), np.float32)
+    rays[:, 0:3] = rng.uniform(-2e-3, 2e-3, size=(500, 3)) + [0, 0, 1]
+    rays[:, 6] = -1.0
+    rays[:, 7] = 10.0
+    prim, t, _ = acc.cast_closest(torch_gpu.from_numpy(rays).cuda())
+    rp, rt, _ = o.cast_closest(rays, brute=True)
+    assert (rp != abi.INVALID_PRIM).sum() > 100
+    assert np.array_equal(prim.cpu().numpy().view(np.uint32), rp)
+    assert np.array_equal(t.cpu().numpy(), rt)
+    # the tree handed out is well formed: each node's children name it as parent
+    inner = gnodes[:, :2][gnodes[:, :2] < 0x80000000]
+    assert np.array_equal(np.sort(inner), np.arange(1, n - 1))
+    leaves = gnodes[:, :2][gnodes[:, :2] >= 0x80000000] & 0x7FFFFFFF
+    assert np.array_equal(np.sort(leaves), np.arange(n))
+    acc.close()
