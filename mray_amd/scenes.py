@@ -111,8 +111,13 @@ class Scene:
         AABB (TracerBase.cpp:1651-1664)."""
         if self.scene_diameter is not None:
             return float(self.scene_diameter)
-        p = np.asarray(self.positions, np.float32)[np.asarray(self.indices).reshape(-1)]
-        span = p.max(axis=0) - p.min(axis=0)
+        # the referenced vertices once each: gathering every corner of 200 K
+        # triangles and reducing its rows took 25 of a 30 ms accelerator build
+        p = np.asarray(self.positions, np.float32)
+        used = np.zeros(len(p), bool)
+        used[np.asarray(self.indices).reshape(-1)] = True
+        q = p[used].T.copy()
+        span = q.max(axis=1) - q.min(axis=1)
         return float(np.float32(np.sqrt(np.float32(span[0] * span[0] + span[2] * span[2]))))
 
     def desc(self):
