@@ -173,7 +173,7 @@ KCMorton30(const float* __restrict__ centers, uint32_t n, const float* __restric
 //                   so that a digit's keys leave in one run: bound by HBM
 //                   (24 B per pair and pass)
 // The scan was one workgroup walking all 256 x tiles counts: 247 us a pass
-// at 2.25 M pairs, now 4.8 us; the scatter 40.1 -> 22.2 us.
+// at 2.25 M pairs, now 4.8 us; the scatter 40.1 -> 16.0 us.
 //
 // Ranking (both forms): a wave owns 64 R consecutive pairs and takes them 64
 // at a time; 8 ballots give each lane the lanes with its digit (its peers),
@@ -184,15 +184,15 @@ static constexpr uint32_t kRsThreads = 256;
 static constexpr uint32_t kRsWaves = kRsThreads / 64;
 static constexpr uint32_t kRsOneThreads = 1024;
 static constexpr uint32_t kRsOneMax = kRsOneThreads * 12u;
-// Rounds per wave of a tile: small tiles until they fill the 256 CUs about
-// twice over (a tile's rounds are serial), then large ones, whose digit runs
-// are longer (64 B at 2048 pairs, 128 B at 4096).
-static constexpr uint32_t kRsSmallRounds = 4, kRsLargeRounds = 16;
-static constexpr uint32_t kRsLargeFrom = 1u << 19;
-static constexpr uint32_t RsTile(uint32_t n)
-{
-    return kRsThreads * ((n < kRsLargeFrom) ? kRsSmallRounds : kRsLargeRounds);
-}
+// Rounds per wave of a tile (256 pairs each).  A tile's rounds are serial and
+// its pairs fill LDS (8 workgroups of 4 rounds share a CU, 4 of 8, 3 of 12,
+// 2 of 16), so tiles grow only as the count fills the 256 CUs; larger tiles
+// have longer digit runs and fewer histogram rows.  Whole sorts with 8 / 12 /
+// 16 rounds: 2^19 pairs 123 / 142 / 163 us, 10^6 149 / 163 / 167, 2.25 M 229 /
+// 212 / 270, 8 M 688 / 614 / 611; 4 rounds below 2^19: 300 K 111 us.
+static constexpr uint32_t kRsMidFrom = 1u << 19, kRsLargeFrom = 1u << 21;
+static constexpr uint32_t RsRounds(uint32_t n) { return (n < kRsMidFrom) ? 4u : (n < kRsLargeFrom) ? 8u : 12u; }
+static constexpr uint32_t RsTile(uint32_t n) { return kRsThreads * RsRounds(n); }
 
 // Lanes of the wave whose key has this lane's digit (valid lanes only).
 __device__ __forceinline__ uint64_t DigitPeers(uint32_t digit, bool valid)
@@ -848,9 +848,12 @@ int LaunchRadixSort(uint64_t* dKeys, uint32_t* dVals, uint32_t n, void* dTemp, s
     uint32_t* dstV = altV;
     for(uint32_t pass = 0; pass < 8; pass++)
     {
-        if(RsTile(n) == kRsThreads * kRsSmallRounds)
-            LaunchRadixPass<kRsSmallRounds>(srcK, srcV, dstK, dstV, n, pass * 8u, hist, s);
-        else LaunchRadixPass<kRsLargeRounds>(srcK, srcV, dstK, dstV, n, pass * 8u, hist, s);
+        switch(RsRounds(n))
+        {
+            case 4: LaunchRadixPass<4>(srcK, srcV, dstK, dstV, n, pass * 8u, hist, s); break;
+            case 8: LaunchRadixPass<8>(srcK, srcV, dstK, dstV, n, pass * 8u, hist, s); break;
+            default: LaunchRadixPass<12>(srcK, srcV, dstK, dstV, n, pass * 8u, hist, s); break;
+        }
         MRAY_HIP_CHECK(hipGetLastError());
         std::swap(srcK, dstK);
         std::swap(srcV, dstV);
@@ -867,7 +870,7 @@ int LaunchRadixSort(uint64_t* dKeys, uint32_t* dVals, uint32_t n, void* dTemp, s
 constexpr uint32_t kNoAllocSortMax = MRAY_NOALLOC_SORT_MAX;
 static_assert(kNoAllocSortMax == (1u << 20), "scratch size is stated as 2^20 pairs");
 // the histograms are largest just below the count where tiles grow
-constexpr size_t kNoAllocSortHistBytes = std::max(RsHistBytes(kNoAllocSortMax), RsHistBytes(kRsLargeFrom - 1u));
+constexpr size_t kNoAllocSortHistBytes = std::max(RsHistBytes(kNoAllocSortMax), RsHistBytes(kRsMidFrom - 1u));
 constexpr size_t kNoAllocSortBytes =
     kNoAllocSortHistBytes + size_t(kNoAllocSortMax) * (sizeof(uint64_t) + sizeof(uint32_t)) + 256;
 static __device__ __align__(256) unsigned char scratch[kNoAllocSortBytes];

@@ -186,12 +186,13 @@ def test_device_collapse_is_host_collapse(torch_gpu, idx):
     assert cd == ch
 
 
-@pytest.mark.parametrize("n", [63, 64, 65, 1023, 4097, 12287, 12288, 12289, 16385, 524287, 524288, 600001])
-@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("noalloc,n", [(a, n) for a in (False, True) for n in
+                                       (63, 64, 65, 1023, 4097, 12287, 12288, 12289, 16385, 524287, 524288, 600001,
+                                        1048576)] + [(False, 2097151), (False, 2097152), (False, 2100001)])
 def test_stage_radix_sort_forms(torch_gpu, n, noalloc):
     """Both sort forms around their limits: one workgroup up to 12288 pairs,
-    small tiles below 2^19, large tiles from there; ties everywhere, keys with
-    the top bit set."""
+    then tiles of 1024, from 2^19 of 2048 and from 2^21 of 3072; ties
+    everywhere, keys with the top bit set."""
     from mray_amd import native
     torch = torch_gpu
     rng = np.random.default_rng(n)
