@@ -23,7 +23,7 @@ METRIC = "Mpaths/s at 1080p; equal-time relMSE: radiance-cache PT vs plain PT, 1
 HBM_PEAK_GBS = 8000.0
 # bytes a node visit loads: BNode4 = six float4 boxes + uint4 children (112 B);
 # CNode8 = origin/exponent header + 48 B of 8-bit boxes + 32 B children (96 B)
-NODE_BYTES = {4: 112, 8: 96}
+NODE_BYTES = {4: 64, 8: 96, "instanced": 112}   # QNode4, CNode8, BNode4
 TRI_BYTES = 48            # SoupTri
 RAY_BYTES = 32 + 28       # RayGMem in, hit record out (prim/t/bary + keys)
 
@@ -723,14 +723,14 @@ def bench_instanced(args):
         "host_waits_per_step": totals["host_waits"] / args.steps,
         "device_drains_per_step": totals["device_drains"] / args.steps,
         "profiled_ms_per_step": round(m["prof_elapsed"] * 1e3 / args.steps, 2),
-        "roofline": _trace_roofline(m, 4, "KTrace (closest hit, instance tree + 4-wide mesh trees)"),
-        "kernel_rooflines": kernel_rooflines(m["cst"], m["ptotals"], phases, 4, spectral, False),
+        "roofline": _trace_roofline(m, "instanced", "KTrace (closest hit, instance tree + 4-wide mesh trees)"),
+        "kernel_rooflines": kernel_rooflines(m["cst"], m["ptotals"], phases, "instanced", spectral, False),
         "single_view": {
             "resolution": [args.width, args.height],
             "mpaths_per_s": round(single_paths * args.steps / el1 / 1e6, 3),
             "ms_per_step": round(el1 * 1e3 / args.steps, 2),
             "phase_ms_per_step": {k: round(v[0] / args.steps, 3) for k, v in ph1.items()},
-            "roofline": _trace_roofline(m1, 4, "KTrace (instanced)"),
+            "roofline": _trace_roofline(m1, "instanced", "KTrace (instanced)"),
         },
     }
     return result
@@ -833,7 +833,7 @@ def main():
         "bounces_per_step": totals["iterations"] // args.steps,
         "host_waits_per_step": totals["host_waits"] / args.steps,
         "device_drains_per_step": totals["device_drains"] / args.steps,
-        "timed_path": "hipGraph bursts of 8 bounces, scheduler snapshots read 2 bursts behind, "
+        "timed_path": "hipGraph bursts of 4 bounces, scheduler snapshots read 1 burst behind, "
                       "one device drain per frame",
         "lane_refill": bool(args.lane_refill),
         "profiled_ms_per_step": round(prof_elapsed * 1e3 / args.steps, 2),

@@ -130,7 +130,7 @@ typedef struct MRayRenderParams
  * on the measured scenes.                                                  */
 #define MRAY_RENDER_MATERIAL_QUEUES 1u
 /* Launch every bounce directly instead of replaying a captured hipGraph of
- * 8 bounces (mray_renderer_iterate on the renderer's own stream).          */
+ * 4 bounces (mray_renderer_iterate on the renderer's own stream).          */
 #define MRAY_RENDER_NO_GRAPH 2u
 /* NEE picks triangle lights in proportion to emitted power (luminance x
  * area, x2 if two-sided) through an alias table, instead of uniformly

@@ -12,6 +12,7 @@
 //        Device/CPU/AlgBinaryPartitionCPU.h:31-48).  Live slots form the
 //        active list in ascending slot order; every position comes from the
 //        per-block scan, so no atomics and a deterministic order.
+//        Small renderers have no scan launch (kFusedRefillBlocks).
 //   KTrace    closest hit of every active slot (CastRays)
 //   KShade    boundary/light work or NEE (work 1) + BxDF scatter (work 0)
 //             (PathTracerRendererShaders.h:201-520); slots with a shadow ray
