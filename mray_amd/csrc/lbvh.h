@@ -49,9 +49,10 @@ struct alignas(128) BNode4
 static_assert(sizeof(BNode4) == 128, "BNode4 must be one 128-byte line");
 
 // The node the walks read: BNode4 with its boxes quantised to 8 bits per plane
-// on a grid of the node's own (plane p of axis a = o[a] + q * s[a]), half a
-// line.  Boxes only grow: every plane stands at least 8 * 2^-24 times the
-// node's largest coordinate outside the exact one (QuantizeNodes), which
+// on a grid of the node's own (plane p of axis a = o[a] + (1024 + q) * s[a]:
+// the walk reads a byte as the half 1024 + q), half a line.  Boxes only grow:
+// every plane stands at least 8 * 2^-24 times the node's largest coordinate
+// and 12 * 2^-24 times its extent outside the exact one (QuantizeNodes), which
 // covers the rounding of the walk's slab test.  Bytes k of qlo / qhi: child k.
 struct alignas(64) QNode4
 {

@@ -225,12 +225,14 @@ __device__ __forceinline__ auto MakeRay(V3 o, V3 d)
 }
 
 // Conservative slab test of a QNode4's child boxes: four 16-byte loads where a
-// BNode4 takes seven, a convert and a fused multiply-add per plane.  Plane
-// o + q s in t is q a + b with a = s inv, b = o inv + off.  With u = 2^-24,
+// BNode4 takes seven, half a byte permute and a fused multiply-add per plane.
+// Plane o + (1024 + q) s in t is (1024 + q) a + b with a = s inv,
+// b = o inv + off; the halves 1024 + q are exact.  With u = 2^-24,
 // inv, a and the final fma carry relative errors of u, off and b absolute ones
 // of u |ray.o inv| and u |o inv|: the ray's offsets cover five u |ray.o inv|,
-// the node's planes stand 8 u of the node's largest coordinate outside the
-// exact box, and the far bound's factor 1 + 8 u covers the relative part of
+// the node's planes stand 8 u of the node's largest coordinate and 12 u of its
+// extent outside the exact box (|o| is at most the coordinate and 4.02
+// extents, 1279 s 5.02 extents), and the far bound's factor 1 + 8 u covers the relative part of
 // both bounds as in SlabTest4.  Values that overflow are NaN, which
 // fmaxf/fminf drop: that plane leaves the interval unbounded.
 // tNear[k] = +inf on a miss.
@@ -238,10 +240,20 @@ __device__ __forceinline__ auto MakeRay(V3 o, V3 d)
 // together; 64-byte nodes also leave 64-72 VGPRs, so 7 waves per SIMD run
 // instead of 6, on 10 LDS stack entries.  1080p terrain: trace 34.9 -> 32.4 ms,
 // shadow 9.6 -> 9.0 ms; 2.8 M rays of a caller 893 -> 690 us; six Cornell
-// scenes' trace 21.7 -> 20.9 ms.  Instance walks run on BNode4: their object-space rays are
+// scenes' trace 21.7 -> 20.9 ms (these with a convert per byte).  Permutes
+// against converts: 32 Cornell scenes of 9.7 M triangles, trace 635 -> 598 ms,
+// shadow 343 -> 333 (BNode4 with the fused test 638, 358; with SlabTest4's
+// subtract and multiply 598, 336); 1080p terrain the same; a caller's rays
+// 679 -> 709 us.  Instance walks run on BNode4: their object-space rays are
 // set up again at every instance, and the wider ray state costs them a wave
 // (trace 5.35 -> 5.55 ms).
-__device__ __forceinline__ float ByteF(uint32_t w, int k) { return float((w >> (8 * k)) & 0xFFu); }
+// Bytes (SEL: two of them) of w as a pair of halves of value 1024 + q: one byte
+// permute for two planes, and the fused multiply-add reads a half at no cost.
+typedef _Float16 Half2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ Half2 BytePair(uint32_t w, uint32_t sel)
+{
+    return __builtin_bit_cast(Half2, __builtin_amdgcn_perm(0x64646464u, w, sel));
+}
 __device__ __forceinline__ void SlabTestQ(const QNode4* __restrict__ np, const RayQ& r,
                                           float tMin, float tMax, float tNear[4], uint4& child)
 {
@@ -258,13 +270,20 @@ __device__ __forceinline__ void SlabTestQ(const QNode4* __restrict__ np, const R
     const uint32_t ny = r.sy ? h2.y : h2.x, fy = r.sy ? h2.x : h2.y;
     const uint32_t nz = r.sz ? h2.w : h2.z, fz = r.sz ? h2.z : h2.w;
     #pragma unroll
-    for(int k = 0; k < 4; k++)
+    for(int p = 0; p < 2; p++)
     {
-        const float tn = SlabNear(tMin, Fma(ByteF(nx, k), ax, nbx), Fma(ByteF(ny, k), ay, nby),
-                                  Fma(ByteF(nz, k), az, nbz));
-        const float tf = SlabFar(tMax, Fma(ByteF(fx, k), ax, fbx), Fma(ByteF(fy, k), ay, fby),
-                                 Fma(ByteF(fz, k), az, fbz));
-        tNear[k] = (tn <= tf) ? tn : INFINITY;
+        const uint32_t sel = p ? 0x04030402u : 0x04010400u;
+        const Half2 hnx = BytePair(nx, sel), hny = BytePair(ny, sel), hnz = BytePair(nz, sel);
+        const Half2 hfx = BytePair(fx, sel), hfy = BytePair(fy, sel), hfz = BytePair(fz, sel);
+        #pragma unroll
+        for(int k = 0; k < 2; k++)
+        {
+            const float tn = SlabNear(tMin, Fma(float(hnx[k]), ax, nbx), Fma(float(hny[k]), ay, nby),
+                                      Fma(float(hnz[k]), az, nbz));
+            const float tf = SlabFar(tMax, Fma(float(hfx[k]), ax, fbx), Fma(float(hfy[k]), ay, fby),
+                                     Fma(float(hfz[k]), az, fbz));
+            tNear[2 * p + k] = (tn <= tf) ? tn : INFINITY;
+        }
     }
 }
 
