@@ -300,60 +300,11 @@ int CollapseToBvh4Device(const uint32_t* dBinNodes, const float* dBinBoxes, cons
     return rc;
 }
 
-// One thread per node; sums in double (the products, 11 bits times 24, are exact).
 __global__ void __launch_bounds__(kTPB)
 KQuantizeNodes(const BNode4* __restrict__ in, uint32_t n, QNode4* __restrict__ out)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= n) return;
-    const BNode4 b = in[i];
-    QNode4 q;
-    for(int k = 0; k < 4; k++) q.child[k] = b.child[k];
-    uint32_t words[6];
-    for(int a = 0; a < 3; a++)
-    {
-        const float* lo = (a == 0) ? b.lox : (a == 1) ? b.loy : b.loz;
-        const float* hi = (a == 0) ? b.hix : (a == 1) ? b.hiy : b.hiz;
-        float L = INFINITY, H = -INFINITY;
-        bool finite = true;
-        for(int k = 0; k < 4; k++)
-        {
-            if(b.child[k] == kInvalid) continue;
-            L = MinF(L, lo[k]);
-            H = MaxF(H, hi[k]);
-            finite = finite && isfinite(lo[k]) && isfinite(hi[k]);
-        }
-        const double m = 4.8e-7 * double(MaxF(fabsf(L), fabsf(H))) + 7.2e-7 * (double(H) - double(L));
-        // 8 u of the coordinates and 12 u of the extent (SlabTestQ), u = 2^-24;
-        // s spans the grown box with a little to spare; o lies 1024 steps below it
-        float s = MaxF(float((double(H) - double(L) + 4.0 * m) * (1.000001 / 255.0)), 1e-30f);
-        float o = float(double(L) - 1.5 * m - 1024.0 * double(s));
-        while(finite && double(o) + 1024.0 * double(s) > double(L) - m) o = nextafterf(o, -INFINITY);
-        const double base = double(o) + 1024.0 * double(s);
-        // a plane that is not finite: NaN leaves the walk's interval unbounded
-        if(!finite || !isfinite(o) || !isfinite(s) || !(base + 255.0 * double(s) >= double(H) + m)) o = NAN;
-        uint32_t wl = 0xFFFFFFFFu, wh = 0u;         // empty slots: lo > hi
-        for(int k = 0; k < 4 && !isnan(o); k++)
-        {
-            if(b.child[k] == kInvalid) continue;
-            const double l = double(lo[k]) - m, h = double(hi[k]) + m;
-            int ql = int(floor((l - base) / double(s)));
-            int qh = int(ceil((h - base) / double(s)));
-            ql = max(0, min(255, ql));
-            qh = max(0, min(255, qh));
-            while(ql > 0 && base + double(ql) * double(s) > l) ql--;
-            while(qh < 255 && base + double(qh) * double(s) < h) qh++;
-            wl = (wl & ~(0xFFu << (8 * k))) | (uint32_t(ql) << (8 * k));
-            wh |= uint32_t(qh) << (8 * k);
-        }
-        q.o[a] = o;
-        q.s[a] = s;
-        words[2 * a] = wl;
-        words[2 * a + 1] = wh;
-    }
-    q.qlox = words[0]; q.qhix = words[1]; q.qloy = words[2];
-    q.qhiy = words[3]; q.qloz = words[4]; q.qhiz = words[5];
-    out[i] = q;
+    if(i < n) out[i] = QuantizeNode(in[i]);
 }
 
 int QuantizeNodes(const BNode4* dNodes, uint32_t n, QNode4* dOut, hipStream_t s)

@@ -109,16 +109,16 @@ struct RayPre
     uint32_t sx, sy, sz;
 };
 
-__device__ __forceinline__ RayPre MakeRayPre(V3 o, V3 d)
+MRAY_HD RayPre MakeRayPre(V3 o, V3 d)
 {
     RayPre r;
     r.o = o;
     r.d = d;
     // exact IEEE reciprocals; a zero component gives +-inf
     r.inv = {1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
-    r.sx = signbit(r.inv.x) ? 1u : 0u;
-    r.sy = signbit(r.inv.y) ? 1u : 0u;
-    r.sz = signbit(r.inv.z) ? 1u : 0u;
+    r.sx = __builtin_signbit(r.inv.x) ? 1u : 0u;
+    r.sy = __builtin_signbit(r.inv.y) ? 1u : 0u;
+    r.sz = __builtin_signbit(r.inv.z) ? 1u : 0u;
     return r;
 }
 
@@ -130,29 +130,45 @@ struct RayQ : RayPre
 };
 
 // One axis of RayQ: the exact reciprocal, and -o * inv less and plus a bound on
-// its own rounding (SlabTestQ).  A direction component under 1e-30, zero
-// included, takes +-1e30 for its reciprocal: over any distance such a ray
-// stays on its origin's side of a plane, and the finite value keeps the test
-// free of inf - inf.  A plane it starts in bounds it nowhere, so its margin is
-// wider by 1e22 (1e-8 in position).
-__device__ __forceinline__ void MakeAxis(float o, float d, float& inv, float& offN, float& offF, uint32_t& s)
+// its own rounding (SlabTestQ).  A direction component under 1e-20, zero
+// included, takes +-1e20 for its reciprocal: up to a distance of `reach` such a
+// ray moves less than 1e-20 reach on the axis, so with a margin of `reach` it is
+// never taken off its origin's side of a plane, nor out of a plane it starts in.
+// 1e20 and not more: a node's planes are reached from an origin that lies up to
+// four extents below its box, and every product with it has to stay finite
+// (QuantizeNode keeps origins and extents under 1.5e18, and a ray's origin past
+// 3.4e18 leaves the axis unbounded).
+MRAY_HD void MakeAxis(float o, float d, float reach, float& inv, float& offN, float& offF, uint32_t& s)
 {
-    const bool parallel = fabsf(d) < 1e-30f;
-    inv = parallel ? copysignf(1e30f, d) : 1.0f / d;
+    const bool parallel = fabsf(d) < 1e-20f;
+    inv = parallel ? copysignf(1e20f, d) : 1.0f / d;
     const float off = -o * inv;
-    const float e = fabsf(off) * 3e-7f + (parallel ? 1e22f : 0.0f);   // 5 * 2^-24, rounded up
+    const float e = fabsf(off) * 3e-7f + (parallel ? reach : 0.0f);   // 5 * 2^-24, rounded up
     offN = off - e;
     offF = off + e;
-    s = signbit(d) ? 1u : 0u;
+    s = __builtin_signbit(d) ? 1u : 0u;
 }
-__device__ __forceinline__ RayQ MakeRayQ(V3 o, V3 d)
+// Reach of a unit vector (a renderer's rays): no hit lies past 1e14 units of
+// length; a margin of 1e-6 in position.
+constexpr float kUnitReach = 1e14f;
+// Reach of a caller's ray: a direction that is no unit vector counts that
+// length in units of its own, here down to a power of two, and no hit lies
+// beyond tMax.  (Taken for every ray, renders of small closed scenes were 1 %
+// slower, with a division 3 %.)
+MRAY_HD float Reach(V3 d, float tMax)
+{
+    int e = 0;
+    (void)frexpf(MaxF(fabsf(d.x), MaxF(fabsf(d.y), fabsf(d.z))), &e);
+    return MaxF(MinF(ldexpf(2.0f * kUnitReach, -e), tMax), kUnitReach);
+}
+MRAY_HD RayQ MakeRayQ(V3 o, V3 d, float reach)
 {
     RayQ r;
     r.o = o;
     r.d = d;
-    MakeAxis(o.x, d.x, r.inv.x, r.offN.x, r.offF.x, r.sx);
-    MakeAxis(o.y, d.y, r.inv.y, r.offN.y, r.offF.y, r.sy);
-    MakeAxis(o.z, d.z, r.inv.z, r.offN.z, r.offF.z, r.sz);
+    MakeAxis(o.x, d.x, reach, r.inv.x, r.offN.x, r.offF.x, r.sx);
+    MakeAxis(o.y, d.y, reach, r.inv.y, r.offN.y, r.offF.y, r.sy);
+    MakeAxis(o.z, d.z, reach, r.inv.z, r.offN.z, r.offF.z, r.sz);
     return r;
 }
 
@@ -166,17 +182,17 @@ __device__ __forceinline__ RayQ MakeRayQ(V3 o, V3 d)
 // With RayQ: one fused multiply-add a plane (the error bound is SlabTestQ's
 // without the node's part; small trees' walks 3 % shorter than with RayPre).
 // tNear[k] = +inf on a miss.
-__device__ __forceinline__ float SlabNear(float tMin, float x, float y, float z)
+MRAY_HD float SlabNear(float tMin, float x, float y, float z)
 {
     return MaxF(MaxF(tMin, x), MaxF(y, z));
 }
-__device__ __forceinline__ float SlabFar(float tMax, float x, float y, float z)
+MRAY_HD float SlabFar(float tMax, float x, float y, float z)
 {
     const float grow = 1.0f + 2.0f * 5.96e-8f * 4.0f;
     return MinF(MinF(tMax, x), MinF(y, z)) * grow;
 }
 template<class RAY>
-__device__ __forceinline__ void SlabTest4(const BNode4* __restrict__ np, const RAY& r,
+MRAY_HD void SlabTest4(const BNode4* __restrict__ np, const RAY& r,
                                           float tMin, float tMax, float tNear[4], uint4& child)
 {
     const float4* q = reinterpret_cast<const float4*>(np);
@@ -218,12 +234,41 @@ constexpr int WidthOf(int W) { return (W == kNodesC8) ? 8 : 4; }
 
 // The ray of such a walk.
 template<int W>
-__device__ __forceinline__ auto MakeRay(V3 o, V3 d)
+__device__ __forceinline__ auto MakeRay(V3 o, V3 d, float reach)
 {
     if constexpr(W == kNodesC8) return MakeRayPre(o, d);
-    else return MakeRayQ(o, d);
+    else return MakeRayQ(o, d, reach);
 }
 
+// Bytes 2 P and 2 P + 1 of w as a pair of halves of value 1024 + q: one byte
+// permute for two planes, and the fused multiply-add reads a half at no cost.
+typedef _Float16 Half2 __attribute__((ext_vector_type(2)));
+template<uint32_t P>
+MRAY_HD Half2 BytePair(uint32_t w)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_bit_cast(Half2, __builtin_amdgcn_perm(0x64646464u, w, P ? 0x04030402u : 0x04010400u));
+#else
+    const uint32_t b = w >> (16u * P);       // the host's tests of the walk's arithmetic
+    return __builtin_bit_cast(Half2, 0x64006400u | (b & 0xFFu) | ((b & 0xFF00u) << 8));
+#endif
+}
+template<uint32_t P>
+MRAY_HD void SlabPairQ(const uint32_t (&words)[6], const float (&a)[3], const float (&nb)[3], const float (&fb)[3],
+                       float tMin, float tMax, float (&tNear)[4])
+{
+    const Half2 hnx = BytePair<P>(words[0]), hny = BytePair<P>(words[1]), hnz = BytePair<P>(words[2]);
+    const Half2 hfx = BytePair<P>(words[3]), hfy = BytePair<P>(words[4]), hfz = BytePair<P>(words[5]);
+    #pragma unroll
+    for(int k = 0; k < 2; k++)
+    {
+        const float tn = SlabNear(tMin, Fma(float(hnx[k]), a[0], nb[0]), Fma(float(hny[k]), a[1], nb[1]),
+                                  Fma(float(hnz[k]), a[2], nb[2]));
+        const float tf = SlabFar(tMax, Fma(float(hfx[k]), a[0], fb[0]), Fma(float(hfy[k]), a[1], fb[1]),
+                                 Fma(float(hfz[k]), a[2], fb[2]));
+        tNear[2 * P + k] = (tn <= tf) ? tn : INFINITY;
+    }
+}
 // Conservative slab test of a QNode4's child boxes: four 16-byte loads where a
 // BNode4 takes seven, half a byte permute and a fused multiply-add per plane.
 // Plane o + (1024 + q) s in t is (1024 + q) a + b with a = s inv,
@@ -232,9 +277,12 @@ __device__ __forceinline__ auto MakeRay(V3 o, V3 d)
 // of u |ray.o inv| and u |o inv|: the ray's offsets cover five u |ray.o inv|,
 // the node's planes stand 8 u of the node's largest coordinate and 12 u of its
 // extent outside the exact box (|o| is at most the coordinate and 4.02
-// extents, 1279 s 5.02 extents), and the far bound's factor 1 + 8 u covers the relative part of
-// both bounds as in SlabTest4.  Values that overflow are NaN, which
-// fmaxf/fminf drop: that plane leaves the interval unbounded.
+// extents, 1279 s 5.02 extents), and the far bound's factor 1 + 8 u covers the
+// relative part of both bounds as in SlabTest4.
+// Range: |o| + 1279 s <= 1.5e18 (QuantizeNode) and |inv| <= 1e20 (MakeAxis)
+// keep a and o inv finite, and b overflows only where every plane of the node
+// lies on one side of the ray's origin, to the infinity of that side.  An axis
+// past that range has o = NaN, which fmaxf/fminf drop: it bounds nothing.
 // tNear[k] = +inf on a miss.
 // Closest-hit walks are bound by the rate of these loads and of VALU issue
 // together; 64-byte nodes also leave 64-72 VGPRs, so 7 waves per SIMD run
@@ -247,44 +295,21 @@ __device__ __forceinline__ auto MakeRay(V3 o, V3 d)
 // 679 -> 709 us.  Instance walks run on BNode4: their object-space rays are
 // set up again at every instance, and the wider ray state costs them a wave
 // (trace 5.35 -> 5.55 ms).
-// Bytes (SEL: two of them) of w as a pair of halves of value 1024 + q: one byte
-// permute for two planes, and the fused multiply-add reads a half at no cost.
-typedef _Float16 Half2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ Half2 BytePair(uint32_t w, uint32_t sel)
-{
-    return __builtin_bit_cast(Half2, __builtin_amdgcn_perm(0x64646464u, w, sel));
-}
-__device__ __forceinline__ void SlabTestQ(const QNode4* __restrict__ np, const RayQ& r,
-                                          float tMin, float tMax, float tNear[4], uint4& child)
+MRAY_HD void SlabTestQ(const QNode4* __restrict__ np, const RayQ& r, float tMin, float tMax, float (&tNear)[4],
+                       uint4& child)
 {
     const uint4* q = reinterpret_cast<const uint4*>(np);
     const uint4 h0 = q[0], h1 = q[1], h2 = q[2];
     child = q[3];
-    const float ox = __uint_as_float(h0.x), oy = __uint_as_float(h0.y), oz = __uint_as_float(h0.z);
-    const float ax = __uint_as_float(h0.w) * r.inv.x, ay = __uint_as_float(h1.x) * r.inv.y,
-                az = __uint_as_float(h1.y) * r.inv.z;
-    const float nbx = Fma(ox, r.inv.x, r.offN.x), fbx = Fma(ox, r.inv.x, r.offF.x);
-    const float nby = Fma(oy, r.inv.y, r.offN.y), fby = Fma(oy, r.inv.y, r.offF.y);
-    const float nbz = Fma(oz, r.inv.z, r.offN.z), fbz = Fma(oz, r.inv.z, r.offF.z);
-    const uint32_t nx = r.sx ? h1.w : h1.z, fx = r.sx ? h1.z : h1.w;
-    const uint32_t ny = r.sy ? h2.y : h2.x, fy = r.sy ? h2.x : h2.y;
-    const uint32_t nz = r.sz ? h2.w : h2.z, fz = r.sz ? h2.z : h2.w;
-    #pragma unroll
-    for(int p = 0; p < 2; p++)
-    {
-        const uint32_t sel = p ? 0x04030402u : 0x04010400u;
-        const Half2 hnx = BytePair(nx, sel), hny = BytePair(ny, sel), hnz = BytePair(nz, sel);
-        const Half2 hfx = BytePair(fx, sel), hfy = BytePair(fy, sel), hfz = BytePair(fz, sel);
-        #pragma unroll
-        for(int k = 0; k < 2; k++)
-        {
-            const float tn = SlabNear(tMin, Fma(float(hnx[k]), ax, nbx), Fma(float(hny[k]), ay, nby),
-                                      Fma(float(hnz[k]), az, nbz));
-            const float tf = SlabFar(tMax, Fma(float(hfx[k]), ax, fbx), Fma(float(hfy[k]), ay, fby),
-                                     Fma(float(hfz[k]), az, fbz));
-            tNear[2 * p + k] = (tn <= tf) ? tn : INFINITY;
-        }
-    }
+    auto f = [](uint32_t w) { return __builtin_bit_cast(float, w); };
+    const float o[3] = {f(h0.x), f(h0.y), f(h0.z)};
+    const float a[3] = {f(h0.w) * r.inv.x, f(h1.x) * r.inv.y, f(h1.y) * r.inv.z};
+    const float nb[3] = {Fma(o[0], r.inv.x, r.offN.x), Fma(o[1], r.inv.y, r.offN.y), Fma(o[2], r.inv.z, r.offN.z)};
+    const float fb[3] = {Fma(o[0], r.inv.x, r.offF.x), Fma(o[1], r.inv.y, r.offF.y), Fma(o[2], r.inv.z, r.offF.z)};
+    const uint32_t words[6] = {r.sx ? h1.w : h1.z, r.sy ? h2.y : h2.x, r.sz ? h2.w : h2.z,
+                               r.sx ? h1.z : h1.w, r.sy ? h2.x : h2.y, r.sz ? h2.z : h2.w};
+    SlabPairQ<0>(words, a, nb, fb, tMin, tMax, tNear);
+    SlabPairQ<1>(words, a, nb, fb, tMin, tMax, tNear);
 }
 
 // Compressed 8-wide node: decode each child box exactly as the builder
@@ -507,7 +532,7 @@ struct Walk
 __device__ __forceinline__ void WalkInit(Walk& w, V3 o, V3 d, float tMin, float tMax, uint32_t root,
                                          uint32_t sp0)
 {
-    w.r = MakeRayQ(o, d);
+    w.r = MakeRayQ(o, d, kUnitReach);
     w.tMin = tMin;
     w.tMax = tMax;
     w.best = HitRec{kInvalid, INFINITY, 0.0f, 0.0f};
@@ -593,10 +618,11 @@ template<int W, bool ANY_HIT, bool COUNT>
 __device__ __forceinline__ HitRec TraceW(const TraceCtx& ctx, uint2* lstack, uint32_t gtid,
                                          V3 o, V3 d, float tMin, float tMax, uint32_t root,
                                          uint32_t* nodeVisits = nullptr,
-                                         uint32_t* triTests = nullptr, uint32_t sp0 = 0)
+                                         uint32_t* triTests = nullptr, uint32_t sp0 = 0,
+                                         float reach = kUnitReach)
 {
     HitRec best{kInvalid, INFINITY, 0.0f, 0.0f};
-    const auto r = MakeRay<W>(o, d);
+    const auto r = MakeRay<W>(o, d, reach);
     uint32_t sp = sp0;
     uint32_t node = root;
     const uint32_t lb = StackLane<kLdsStack>();

@@ -278,3 +278,87 @@ def test_node_kinds_equal_brute_force(torch_gpu, cells, offset, flat):
     along[:, 7] = 100.0
     _compare(acc, refcpu.OracleScene(s), np.concatenate([down, slant, along]).astype(np.float32), brute=True)
     acc.close()
+
+
+def _lit_grid(cells, extent):
+    """A flat grid over [-extent, extent]^2 at z = 0, every triangle a
+    two-sided light of its own, and a camera straight above it whose opening
+    angle is so small that all its rays are exactly axis-parallel."""
+    g = (np.arange(cells + 1, dtype=np.float64) / cells * 2 - 1) * extent
+    x, y = np.meshgrid(g, g, indexing="ij")
+    pos = np.stack([x, y, np.zeros_like(x)], -1).reshape(-1, 3).astype(np.float32)
+    i, j = np.meshgrid(np.arange(cells), np.arange(cells), indexing="ij")
+    v = (i * (cells + 1) + j).reshape(-1)
+    idx = np.concatenate([np.stack([v, v + cells + 1, v + cells + 2], 1),
+                          np.stack([v, v + cells + 2, v + 1], 1)]).astype(np.uint32)
+    n = len(idx)
+    key = (np.arange(n) | abi.LIGHT_FLAG).astype(np.uint32)
+    rad = np.random.default_rng(n).uniform(0.5, 2.0, size=(n, 3)).astype(np.float32)
+    at = (0.1 * extent, -0.23 * extent)
+    return scenes.Scene(positions=pos, tbn=np.tile(np.array([[1, 0, 0, 0]], np.float32), (len(pos), 1)),
+                        indices=idx, surface_keys=key, cull=np.zeros(n, np.uint8),
+                        materials=[{"type": abi.MAT_LAMBERT, "albedo": (1, 1, 1)}],
+                        light_tris=np.arange(n, dtype=np.uint32), light_radiance=rad,
+                        light_two_sided=np.ones(n, np.uint8),
+                        camera={"position": at + (0.5 * extent,), "gaze": at + (0.0,), "up": (0, 1, 0),
+                                "fov": (1e-25, 1e-25), "nearFar": (0.01 * extent, 10.0 * extent)})
+
+
+@pytest.mark.parametrize("cells", [24, 96])
+@pytest.mark.parametrize("extent", [1e3, 4e7, 1e8, 1e10])
+def test_axis_parallel_rays_in_large_scenes(torch_gpu, extent, cells):
+    """Axis-parallel rays (+0, -0 and tiny components) and directions that are
+    far from unit length over scenes of large extent, on exact and on quantised
+    nodes: equal to brute force."""
+    from mray_amd import native
+    s = _lit_grid(cells, extent)
+    acc = native.Accel(s)
+    assert (acc.info()["wide_nodes"] > 4096) == (cells > 24)
+    rng = np.random.default_rng(cells)
+    g = s.positions[:, 0]
+    rays = np.zeros((600, 8), np.float32)
+    rays[:, 0:2] = rng.choice(g, (600, 2))                       # on vertices and planes
+    rays[200:, 0:2] = rng.uniform(-1.2 * extent, 1.2 * extent, (400, 2))
+    rays[:, 2] = 0.5 * extent
+    rays[:, 6] = -1.0
+    rays[:, 7] = 3.4e38
+    rays[::2, 4:6] = -0.0
+    rays[1::5, 4] = 1e-36
+    # direction lengths of 1e-9 and 1e9: t grows and shrinks with them
+    rays[100:150, 4:7] *= np.float32(1e-9)
+    rays[150:200, 4:7] *= np.float32(1e9)
+    along = rays[:100].copy()                                    # across the grid, above and in its plane
+    along[:, 0] = -1.5 * extent
+    along[:, 2] = 0.0
+    along[:, 4:7] = (1.0, 0.0, -0.0)
+    _compare(acc, refcpu.OracleScene(s), np.concatenate([rays, along]), brute=True)
+    acc.close()
+
+
+@pytest.mark.parametrize("kind", ["one", "lane_refill", "batch"])
+@pytest.mark.parametrize("extent", [1e3, 1e9])
+def test_renders_of_large_scenes(torch_gpu, extent, kind):
+    """Renders whose camera rays are exactly axis-parallel, over a small tree
+    of large extent: every path reaches the light below the camera, as in the
+    oracle (batch and lane-refill walks take quantised nodes at any size)."""
+    from mray_amd import native
+    s = _lit_grid(16, extent)
+    params = abi.render_params(8, 8, 4, rr=(4, 4), mode=abi.SAMPLE_PURE, seed=3,
+                               flags=abi.RENDER_LANE_REFILL if kind == "lane_refill" else 0)
+    acc = native.Accel(s)
+    if kind == "batch":
+        b = native.BatchScene([acc])
+        r = native.BatchRenderer(b, [{"scene": 0, "width": 8, "height": 8, "spp": 4}], params)
+    else:
+        r = native.Renderer(acc, params)
+    st = r.render_all()
+    film = r.film()
+    film = film[0] if kind == "batch" else film
+    r.close()
+    ref, rst = refcpu.OracleScene(s).render(params)
+    img, rimg = film[:3] / film[3], ref[:3] / ref[3]
+    print(f"{kind} extent {extent:g}: {st['dead_paths']} paths, image {img.min():.3f}..{img.max():.3f}", flush=True)
+    assert st["dead_paths"] == rst["dead_paths"] == 256
+    assert rimg.min() >= 0.49
+    assert np.allclose(img, rimg, rtol=1e-5)
+    acc.close()
