@@ -200,7 +200,8 @@ int mray_morton30(const float* dCenters, uint32_t count, const float* dSceneAabb
                   uint32_t* dCodes, void* stream);
 /* Stable ascending sort of (code, index) pairs over all 64 key bits
  * (AlgRadixSortCUDA.h, used at AcceleratorLBVH.hpp:828-838).  dTemp needs
- * mray_radix_sort_temp_bytes(count) bytes.                                 */
+ * mray_radix_sort_temp_bytes(count) bytes; a buffer of that size also serves
+ * every smaller count.                                                     */
 size_t mray_radix_sort_temp_bytes(uint32_t count);
 int mray_radix_sort_u64_u32(uint64_t* dKeys, uint32_t* dValues, uint32_t count,
                             void* dTemp, size_t tempBytes, void* stream);

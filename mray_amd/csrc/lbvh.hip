@@ -806,10 +806,22 @@ static constexpr size_t RsHistBytes(uint32_t n)
     return ((256u * (tiles ? tiles : 1u) + 256u) * sizeof(uint32_t) + 255) / 256 * 256;
 }
 
-size_t RadixSortTempBytes(uint32_t n)
+// What a sort of n pairs uses.
+static constexpr size_t RsNeed(size_t histBytes, uint32_t n)
 {
-    return RsHistBytes(n) + size_t(n) * (sizeof(uint64_t) + sizeof(uint32_t)) + 256;
+    return histBytes + size_t(n) * (sizeof(uint64_t) + sizeof(uint32_t)) + 256;
 }
+
+// A workspace for n pairs serves every smaller count too: where tiles grow,
+// the count just below has more histogram rows.
+static constexpr size_t RsHistBytesUpTo(uint32_t n)
+{
+    size_t b = RsHistBytes(n);
+    if(n >= kRsMidFrom) b = std::max(b, RsHistBytes(kRsMidFrom - 1u));
+    if(n >= kRsLargeFrom) b = std::max(b, RsHistBytes(kRsLargeFrom - 1u));
+    return b;
+}
+size_t RadixSortTempBytes(uint32_t n) { return RsNeed(RsHistBytesUpTo(n), n); }
 
 template<uint32_t R>
 static void LaunchRadixPass(const uint64_t* srcK, const uint32_t* srcV, uint64_t* dstK, uint32_t* dstV,
@@ -826,7 +838,7 @@ int LaunchRadixSort(uint64_t* dKeys, uint32_t* dVals, uint32_t n, void* dTemp, s
                     hipStream_t s)
 {
     if(n <= 1) return MRAY_OK;
-    if(tempBytes < RadixSortTempBytes(n))
+    if(tempBytes < RsNeed(RsHistBytes(n), n))
     {
         SetError("radix sort: temporary buffer too small");
         return MRAY_ERR_INVALID;
@@ -869,10 +881,7 @@ int LaunchRadixSort(uint64_t* dKeys, uint32_t* dVals, uint32_t n, void* dTemp, s
 // ---------------------------------------------------------------------------
 constexpr uint32_t kNoAllocSortMax = MRAY_NOALLOC_SORT_MAX;
 static_assert(kNoAllocSortMax == (1u << 20), "scratch size is stated as 2^20 pairs");
-// the histograms are largest just below the count where tiles grow
-constexpr size_t kNoAllocSortHistBytes = std::max(RsHistBytes(kNoAllocSortMax), RsHistBytes(kRsMidFrom - 1u));
-constexpr size_t kNoAllocSortBytes =
-    kNoAllocSortHistBytes + size_t(kNoAllocSortMax) * (sizeof(uint64_t) + sizeof(uint32_t)) + 256;
+constexpr size_t kNoAllocSortBytes = RsNeed(RsHistBytesUpTo(kNoAllocSortMax), kNoAllocSortMax);
 static __device__ __align__(256) unsigned char scratch[kNoAllocSortBytes];
 
 namespace

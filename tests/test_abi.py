@@ -41,3 +41,17 @@ def test_error_path_without_gpu_work():
     assert b"NULL" in L.mray_last_error()
     assert L.mray_renderer_iterate(None, 1, None) == 1
     assert L.mray_radix_sort_temp_bytes(10000) > 10000 * 12
+
+
+def test_workspaces_serve_smaller_counts():
+    """A caller sizes a build's workspaces once, for its largest mesh: the
+    reported sizes never fall as the count grows, also where the sort's tiles
+    do (2^19 and 2^21 pairs)."""
+    L = native.lib()
+    for f in (L.mray_radix_sort_temp_bytes, L.mray_lbvh_temp_bytes):
+        last = 0
+        for lo, hi in ((0, 20000), ((1 << 19) - 5000, (1 << 19) + 50000), ((1 << 21) - 5000, (1 << 21) + 50000)):
+            for n in range(lo, hi, 7):
+                b = f(n)
+                assert b >= last, (f.__name__, n)
+                last = b

@@ -261,3 +261,24 @@ def test_malformed_reference_tree_is_rebuilt(torch_gpu):
     leaves = gnodes[:, :2][gnodes[:, :2] >= 0x80000000] & 0x7FFFFFFF
     assert np.array_equal(np.sort(leaves), np.arange(n))
     acc.close()
+
+
+@pytest.mark.parametrize("cap", [1 << 19, (1 << 21) + 1])
+def test_sort_workspace_of_a_larger_count(torch_gpu, cap):
+    """One workspace, sized for `cap` pairs, sorts counts on either side of
+    the steps where tiles grow (more tiles just below them)."""
+    from mray_amd import native
+    torch = torch_gpu
+    L = native.lib()
+    nb = L.mray_radix_sort_temp_bytes(cap)
+    tmp = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    rng = np.random.default_rng(cap)
+    for n in (cap, cap - 1, cap - 2, (1 << 19) - 1, 504065):
+        keys = rng.integers(0, 1 << 64, size=n, dtype=np.uint64)
+        dk = torch.from_numpy(keys.view(np.int64).copy()).cuda()
+        dv = torch.arange(n, dtype=torch.int32, device="cuda")
+        native.check(L.mray_radix_sort_u64_u32(native._ptr(dk), native._ptr(dv), n, native._ptr(tmp), nb,
+                                               native._stream()))
+        order = np.argsort(keys, kind="stable")
+        assert np.array_equal(dk.cpu().numpy().view(np.uint64), keys[order])
+        assert np.array_equal(dv.cpu().numpy().view(np.uint32), order.astype(np.uint32))
