@@ -439,8 +439,17 @@ KNrcInferEncoded(NrcView v, const float* __restrict__ rec, const uint32_t* __res
 }
 
 // ---- training: forward and data gradients -----------------------------------
+// What a training call leaves for later ones, in device memory: a captured call
+// runs again at each replay, which the host does not see.
+struct NrcState
+{
+    uint32_t pending;  // gradients of a backward pass that no Adam step has applied
+    uint32_t apply;    // of the running fused step: it applies pending gradients
+    uint32_t tiles;    // tiles of the last batch
+};
 struct NrcTrainBuf
 {
+    NrcState* state;
     uint32_t* x;       // [6][B/32][64 features][32 samples] bf16 layer inputs
     uint32_t* dz;      // the same for the gradients of the layer outputs
     float2* dx0;       // [16 levels][B] gradient of the grid features
@@ -472,9 +481,16 @@ __device__ __forceinline__ void StoreTransposed(uint32_t* __restrict__ rows, con
 // from 53 + 55 us as two LDS-staged kernels.
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2)))
 KNrcTrain(NrcView v, const float* __restrict__ rec, const float* __restrict__ target, NrcTrainBuf tb,
-          uint32_t batch)
+          uint32_t batch, uint32_t step)
 {
     const uint32_t lane = threadIdx.x & 63u, tiles = batch / 32u, tile = blockIdx.x;
+    if(tile == 0u && lane == 0u)
+    {
+        // a fused step (step = 1) takes over what is pending, a backward pass adds to it
+        tb.state->apply = tb.state->pending;
+        tb.state->pending = step ? 0u : 1u;
+        tb.state->tiles = tiles;
+    }
     const uint32_t s = tile * 32u + (lane & 31u);
     const float* r = rec + size_t(s) * 11u;
     const uint4* __restrict__ wT = reinterpret_cast<const uint4*>(v.wT);
@@ -614,9 +630,10 @@ __device__ __forceinline__ void AdamWeight(const MlpAdam& u, uint32_t i, float g
 }
 
 __global__ void __launch_bounds__(256)
-KNrcAdamMlp(MlpAdam u, float* __restrict__ g, AdamArgs a)
+KNrcAdamMlp(MlpAdam u, float* __restrict__ g, AdamArgs a, NrcState* __restrict__ state)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if(i == 0) state->pending = 0u;
     if(i >= kMlpParams) return;
     const float gg = g[i];
     g[i] = 0.0f;
@@ -628,7 +645,7 @@ KNrcAdamMlp(MlpAdam u, float* __restrict__ g, AdamArgs a)
 // take every 16th sample tile (one v_mfma_f32_16x16x32_bf16 each; with samples
 // contiguous both operands are 1 KiB contiguous loads) and are summed through
 // LDS in wave order, so there are no atomics and the sum is deterministic.
-// ADAM: the block also updates its 256 parameters (wgrad must be clear).
+// ADAM: the block also updates its 256 parameters, pending gradients included.
 // Bound by L2 reads (each operand tile is read by four blocks): 17 us a batch of
 // 16384 (17.9 with atomics and LDS transposes, plus the MLP's Adam pass, 4.9).
 constexpr uint32_t kWgradWaves = 16;
@@ -644,6 +661,7 @@ KNrcWgrad(NrcTrainBuf tb, uint32_t batch, float* __restrict__ wgrad, MlpAdam u, 
     if(l >= kNrcLayers) return;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, tiles = batch / 32u;
     v4f acc = v4f{0};
+    const bool apply = ADAM && tb.state->apply != 0u;
     // outputs past the third have no gradient (and none is stored)
     const bool live = l + 1u < kNrcLayers || nt == 0u;
     if(live)
@@ -679,7 +697,11 @@ KNrcWgrad(NrcTrainBuf tb, uint32_t batch, float* __restrict__ wgrad, MlpAdam u, 
     for(uint32_t w = 0; w < kWgradWaves; w++) g += part[w][threadIdx.x];
     const uint32_t k = kt * 16u + (threadIdx.x >> 4), n = nt * 16u + (threadIdx.x & 15u);
     const uint32_t i = l * kLayerParams + k * kW + n;
-    if constexpr(ADAM) AdamWeight(u, i, g, a);
+    if constexpr(ADAM)
+    {
+        if(apply) { g += wgrad[i]; wgrad[i] = 0.0f; }
+        AdamWeight(u, i, g, a);
+    }
     else if(live && g != 0.0f) wgrad[i] += g;
 }
 
@@ -762,6 +784,8 @@ KNrcGridOwner(NrcView v, NrcTrainBuf tb, uint32_t batch, OwnerLevels ol, float* 
     while(blockIdx.x >= ol.first[l + 1]) l++;
     const uint32_t base = (blockIdx.x - ol.first[l]) * ol.size[l];
     const uint32_t count = min(ol.size[l], ol.used[l] - base);
+    const size_t first = ((size_t(l) << v.log2T) + base) / 2u;      // in pairs of entries
+    const bool apply = MODE != OWNER_ADD && tb.state->apply != 0u;
     for(uint32_t e = threadIdx.x; e < (count + 1u) / 2u; e += kOwnerTPB)
         reinterpret_cast<float4*>(seg)[e] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     __syncthreads();
@@ -795,10 +819,9 @@ KNrcGridOwner(NrcView v, NrcTrainBuf tb, uint32_t batch, OwnerLevels ol, float* 
         }
     }
     __syncthreads();
-    const size_t first = ((size_t(l) << v.log2T) + base) / 2u;      // in pairs of entries
     for(uint32_t e = threadIdx.x; e < (count + 1u) / 2u; e += kOwnerTPB)
     {
-        const float4 g4 = reinterpret_cast<const float4*>(seg)[e];
+        float4 g4 = reinterpret_cast<const float4*>(seg)[e];
         if constexpr(MODE == OWNER_ADD)
         {
             if(g4.x == 0.0f && g4.y == 0.0f && g4.z == 0.0f && g4.w == 0.0f) continue;
@@ -806,7 +829,16 @@ KNrcGridOwner(NrcView v, NrcTrainBuf tb, uint32_t batch, OwnerLevels ol, float* 
             t.x += g4.x; t.y += g4.y; t.z += g4.z; t.w += g4.w;
             reinterpret_cast<float4*>(ggrad)[first + e] = t;
         }
-        else AdamGrid4<MODE == OWNER_LAZY>(u, first + e, g4, a);
+        else
+        {
+            if(apply)
+            {
+                const float4 t = reinterpret_cast<const float4*>(ggrad)[first + e];
+                g4.x += t.x; g4.y += t.y; g4.z += t.z; g4.w += t.w;
+                reinterpret_cast<float4*>(ggrad)[first + e] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+            AdamGrid4<MODE == OWNER_LAZY>(u, first + e, g4, a);
+        }
     }
 }
 
@@ -858,8 +890,6 @@ struct MRayNrc
     uint32_t maxBatch = 0;
     uint64_t step = 0;
     uint32_t inferBlocks = 0;     // resident inference blocks
-    uint32_t lossTiles = 0;       // tiles of the last backward pass
-    bool gradsClear = true;       // no backward pass since the last Adam or clear
     OwnerLevels owner{};
     uint32_t ownerSegs = 0;       // segments of the largest level
     // features of one chunk of queries (InferSplit)
@@ -984,6 +1014,7 @@ int mray_nrc_create(const MRayNrcConfig* hCfg, MRayNrc** out)
     if((rv = A((void**)&n->tb.dx0, B * 32 * 4)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->tb.pos, B * 3 * 4)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->tb.loss, B / 32 * 4)) != MRAY_OK) return fail(rv);
+    if((rv = A((void**)&n->tb.state, sizeof(NrcState))) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->feat, size_t(kSplitChunk) * kNrcMaxLevels * 4u)) != MRAY_OK) return fail(rv);
     if(hipEventCreateWithFlags(&n->featDone, hipEventDisableTiming) != hipSuccess)
     {
@@ -1019,6 +1050,7 @@ int mray_nrc_create(const MRayNrcConfig* hCfg, MRayNrc** out)
     KNrcZero<<<256, 256>>>(n->wm, kMlpParams);
     KNrcZero<<<256, 256>>>(n->wv, kMlpParams);
     KNrcZero<<<256, 256>>>(n->wg, kMlpParams);
+    KNrcZero<<<1, 64>>>(reinterpret_cast<float*>(n->tb.state), sizeof(NrcState) / 4u);
     KNrcZero<<<2048, 256>>>(n->gm, n->gridCount);
     KNrcZero<<<2048, 256>>>(n->gv, n->gridCount);
     KNrcZero<<<2048, 256>>>(n->gg, n->gridCount);
@@ -1128,11 +1160,11 @@ static int CheckBatch(const MRayNrc* n, const float* dRecords, const float* dTar
 }
 
 // Forward and data gradients of one batch.
-static void LaunchTrain(MRayNrc* n, const float* dRecords, const float* dTargets, uint32_t count, hipStream_t s)
+static void LaunchTrain(MRayNrc* n, const float* dRecords, const float* dTargets, uint32_t count, uint32_t step,
+                        hipStream_t s)
 {
     NrcTimer t(n, 1, s);
-    KNrcTrain<<<count / 32u, 64, 0, s>>>(n->view, dRecords, dTargets, n->tb, count);
-    n->lossTiles = count / 32u;
+    KNrcTrain<<<count / 32u, 64, 0, s>>>(n->view, dRecords, dTargets, n->tb, count, step);
 }
 
 int mray_nrc_backward(MRayNrc* n, const float* dRecords, const float* dTargets, uint32_t count,
@@ -1140,8 +1172,7 @@ int mray_nrc_backward(MRayNrc* n, const float* dRecords, const float* dTargets, 
 {
     MRAY_TRY(CheckBatch(n, dRecords, dTargets, count));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    n->gradsClear = false;
-    LaunchTrain(n, dRecords, dTargets, count, s);
+    LaunchTrain(n, dRecords, dTargets, count, 0u, s);
     {
         NrcTimer t(n, 3, s);
         KNrcWgrad<false><<<kWgradBlocks, kWgradWaves * 64, 0, s>>>(n->tb, count, n->wg, MlpAdam{}, AdamArgs{});
@@ -1165,28 +1196,27 @@ int mray_nrc_adam(MRayNrc* n, void* stream)
     hipStream_t s = static_cast<hipStream_t>(stream);
     const AdamArgs a = NextAdam(n);
     NrcTimer t(n, 5, s);
-    KNrcAdamMlp<<<DivUp(kMlpParams, 256u), 256, 0, s>>>(MlpOf(n), n->wg, a);
+    KNrcAdamMlp<<<DivUp(kMlpParams, 256u), 256, 0, s>>>(MlpOf(n), n->wg, a, n->tb.state);
     if(n->cfg.flags & MRAY_NRC_LAZY_ADAM)
         KNrcAdamGrid<true><<<4096, 256, 0, s>>>(GridOf(n), n->gg, n->gridCount, a);
     else
         KNrcAdamGrid<false><<<4096, 256, 0, s>>>(GridOf(n), n->gg, n->gridCount, a);
-    n->gradsClear = true;
     return NrcLaunchCheck();
 }
 
-// Backward and Adam.  With no gradients pending from earlier backward passes
-// both gradients are applied where they are formed and never stored.
+// Backward and Adam.  Both gradients are applied where they are formed and
+// never stored, together with what earlier backward passes left pending.
 int mray_nrc_train(MRayNrc* n, const float* dRecords, const float* dTargets, uint32_t count,
                    void* stream)
 {
     MRAY_TRY(CheckBatch(n, dRecords, dTargets, count));
-    if(!n->gradsClear || n->ownerSegs > kOwnerMaxSegs)
+    if(n->ownerSegs > kOwnerMaxSegs)
     {
         MRAY_TRY(mray_nrc_backward(n, dRecords, dTargets, count, stream));
         return mray_nrc_adam(n, stream);
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
-    LaunchTrain(n, dRecords, dTargets, count, s);
+    LaunchTrain(n, dRecords, dTargets, count, 1u, s);
     const AdamArgs a = NextAdam(n);
     {
         NrcTimer t(n, 3, s);
@@ -1207,7 +1237,9 @@ int mray_nrc_last_loss(MRayNrc* n, float* hLoss)
 {
     if(!n || !hLoss) { SetError("nrc_last_loss: NULL argument"); return MRAY_ERR_INVALID; }
     MRAY_HIP_CHECK(hipDeviceSynchronize());
-    std::vector<float> part(n->lossTiles);
+    NrcState state{};
+    MRAY_HIP_CHECK(hipMemcpy(&state, n->tb.state, sizeof(state), hipMemcpyDeviceToHost));
+    std::vector<float> part(state.tiles);
     MRAY_HIP_CHECK(hipMemcpy(part.data(), n->tb.loss, part.size() * sizeof(float), hipMemcpyDeviceToHost));
     double sum = 0.0;
     for(float x : part) sum += x;
@@ -1291,7 +1323,7 @@ int mray_nrc_zero_grads(MRayNrc* n, void* stream)
     hipStream_t s = static_cast<hipStream_t>(stream);
     KNrcZero<<<256, 256, 0, s>>>(n->wg, kMlpParams);
     KNrcZero<<<2048, 256, 0, s>>>(n->gg, n->gridCount);
-    n->gradsClear = true;
+    KNrcZero<<<1, 64, 0, s>>>(reinterpret_cast<float*>(&n->tb.state->pending), 1u);
     return NrcLaunchCheck();
 }
 
