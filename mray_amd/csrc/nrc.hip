@@ -38,6 +38,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <random>
 #include <vector>
@@ -869,9 +870,75 @@ __global__ void KNrcRefresh(const float* __restrict__ w, uint16_t* __restrict__ 
 // ===========================================================================
 using namespace mray;
 
+// Features of one chunk of queries (InferSplit), between the encoding and the
+// layers of one call.  All caches of a GPU share its areas (an area in each, 32
+// MiB, is never used by a renderer's caches, whose counts only the device knows:
+// 1 GiB for 32 views), and calls on up to kFeatAreas streams have one each, so
+// that they overlap.  Released with the GPU's last cache.
+// 16 levels of 2^19 entries, one call on each of 4 streams: 256 queries 84-100 us
+// with one area, 30 with four; 4096 96 -> 29; 16384 113 -> 43; 65536 177 -> 128;
+// 262144 428 -> 465 (two streams 213 -> 210: a call fills the GPU by itself).
+constexpr uint32_t kFeatAreas = 4;
+// Queries up to which the one-kernel form is taken: its one launch costs the
+// host less than two launches, a wait and an event.  64 queries 11.3 us on one
+// stream against 11.8, on four 17.5 against 42; 128 on one stream 12.5 against 11.7.
+constexpr uint32_t kOneKernelMax = 64;
+// The same while several streams query: 256 on two 19.5 us against 19.3, on
+// four 18.9 against 40 (on one 14.7 against 12.3); 512 on two 27 against 19.
+constexpr uint32_t kOneKernelMaxStreams = 256;
+struct FeatArea
+{
+    uint32_t* feat = nullptr;
+    hipEvent_t done = nullptr;    // the area's last use
+    hipStream_t stream = nullptr; // of that use: a hint only, calls wait for the event
+    uint64_t used = 0;            // its number among the GPU's uses, 0: none yet
+};
+struct FeatPool
+{
+    uint32_t caches = 0;
+    uint64_t uses = 0;
+    FeatArea area[kFeatAreas];
+};
+// Never destroyed: a program's own static objects may end their caches late.
+static std::mutex& featLock = *new std::mutex();             // every pool
+static std::map<int, FeatPool>& featPools = *new std::map<int, FeatPool>();
+
+static bool AllocFeatArea(FeatArea& a)
+{
+    if(a.feat) return true;
+    // no stream operation: another thread's capture is none of its concern
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    void* p = nullptr;
+    if(hipMalloc(&p, size_t(kSplitChunk) * kNrcMaxLevels * 4u) == hipSuccess)
+    {
+        if(hipEventCreateWithFlags(&a.done, hipEventDisableTiming) == hipSuccess) a.feat = static_cast<uint32_t*>(p);
+        else (void)hipFree(p);
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if(!a.feat) (void)hipGetLastError();
+    return a.feat != nullptr;
+}
+
+static void ReleaseFeatPool(int device)
+{
+    std::lock_guard<std::mutex> lock(featLock);
+    FeatPool& p = featPools[device];
+    if(--p.caches != 0u) return;
+    for(FeatArea& a : p.area)
+    {
+        if(!a.feat) continue;
+        (void)hipEventSynchronize(a.done);
+        (void)hipEventDestroy(a.done);
+        (void)hipFree(a.feat);
+    }
+    featPools.erase(device);
+}
+
 struct MRayNrc
 {
     MRayNrcConfig cfg{};
+    int device = -1;              // whose pool it uses
     DeviceArena arena;
     NrcView view{};
     uint16_t* wT = nullptr;
@@ -892,10 +959,6 @@ struct MRayNrc
     uint32_t inferBlocks = 0;     // resident inference blocks
     OwnerLevels owner{};
     uint32_t ownerSegs = 0;       // segments of the largest level
-    // features of one chunk of queries (InferSplit)
-    std::mutex featLock;
-    uint32_t* feat = nullptr;
-    hipEvent_t featDone = nullptr;
     EncodePlan plan{};
     // per-kernel timing (mray_nrc_set_profiling): event pairs around each
     // launch, harvested by mray_nrc_kernel_times
@@ -996,7 +1059,18 @@ int mray_nrc_create(const MRayNrcConfig* hCfg, MRayNrc** out)
     n->maxBatch = c.maxBatch;
     auto A = [&](void** p, size_t bytes) { return DevAlloc(n->arena, p, bytes); };
     int rv = MRAY_OK;
-    auto fail = [&](int r) { n->arena.Release(); if(n->featDone) (void)hipEventDestroy(n->featDone); delete n; return r; };
+    auto fail = [&](int r) { n->arena.Release(); if(n->device >= 0) ReleaseFeatPool(n->device); delete n; return r; };
+    int dev = 0;
+    if(hipGetDevice(&dev) != hipSuccess) return fail(MRAY_ERR_HIP);
+    {
+        // the first area now, not in some call's first pass; without memory
+        // for it queries take the one-kernel form
+        std::lock_guard<std::mutex> lock(featLock);
+        FeatPool& p = featPools[dev];
+        p.caches++;
+        n->device = dev;
+        (void)AllocFeatArea(p.area[0]);
+    }
     if((rv = A((void**)&n->wT, kMlpParams * 2)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->wK, kMlpParams * 2)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->w, kMlpParams * 4)) != MRAY_OK) return fail(rv);
@@ -1015,12 +1089,6 @@ int mray_nrc_create(const MRayNrcConfig* hCfg, MRayNrc** out)
     if((rv = A((void**)&n->tb.pos, B * 3 * 4)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->tb.loss, B / 32 * 4)) != MRAY_OK) return fail(rv);
     if((rv = A((void**)&n->tb.state, sizeof(NrcState))) != MRAY_OK) return fail(rv);
-    if((rv = A((void**)&n->feat, size_t(kSplitChunk) * kNrcMaxLevels * 4u)) != MRAY_OK) return fail(rv);
-    if(hipEventCreateWithFlags(&n->featDone, hipEventDisableTiming) != hipSuccess)
-    {
-        SetError("nrc_create: event creation failed");
-        return fail(MRAY_ERR_HIP);
-    }
     v.wT = n->wT;
     v.wK = n->wK;
     v.grid = n->gridH;
@@ -1060,10 +1128,8 @@ int mray_nrc_create(const MRayNrcConfig* hCfg, MRayNrc** out)
         SetError("nrc_create: initialisation kernels failed");
         return fail(MRAY_ERR_HIP);
     }
-    int dev = 0;
     hipDeviceProp_t prop;
-    if(hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess)
-        return fail(MRAY_ERR_HIP);
+    if(hipGetDeviceProperties(&prop, dev) != hipSuccess) return fail(MRAY_ERR_HIP);
     int perCu = 0;
     if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, KNrcInfer, int(kInferTPB), 0) != hipSuccess || perCu < 1)
         perCu = 1;
@@ -1082,23 +1148,45 @@ int mray_nrc_destroy(MRayNrc* n)
         (void)hipEventDestroy(p.second.second);
     }
     for(hipEvent_t e : n->evPool) (void)hipEventDestroy(e);
-    if(n->featDone) (void)hipEventDestroy(n->featDone);
     n->arena.Release();
+    ReleaseFeatPool(n->device);
     delete n;
     return MRAY_OK;
 }
 
-// Encoding in its own pass, chunk by chunk through the cache's feature area.
-// Calls on other streams wait for the area's last use; a call under capture
-// (its graph may run beside others) takes the one-kernel form.
+// Encoding in its own pass, chunk by chunk through an area of the GPU's pool.
+// A call takes the area of its stream's last call, else one not used yet, else
+// the one whose last use is longest ago, and waits for that use.  A call under
+// capture (its graph may run beside others) takes the one-kernel form, and so
+// do small ones (kOneKernelMax) and one that finds no memory for an area.
 constexpr int kNoSplit = -1;
 static int InferSplit(MRayNrc* n, const float* dRecords, uint32_t count, float* dOut, uint32_t blocks, hipStream_t s)
 {
+    if(count <= kOneKernelMax) return kNoSplit;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     MRAY_HIP_CHECK(hipStreamIsCapturing(s, &cap));
     if(cap != hipStreamCaptureStatusNone) return kNoSplit;
-    std::lock_guard<std::mutex> lock(n->featLock);
-    MRAY_HIP_CHECK(hipStreamWaitEvent(s, n->featDone, 0));
+    std::lock_guard<std::mutex> lock(featLock);
+    FeatPool& pool = featPools[n->device];
+    if(count <= kOneKernelMaxStreams && pool.area[1].used != 0u) return kNoSplit;
+    FeatArea* a = &pool.area[0];
+    for(FeatArea& c : pool.area)
+    {
+        if(c.used && c.stream == s) { a = &c; break; }
+        if(c.used < a->used) a = &c;
+    }
+    int dev = n->device;
+    if(!a->feat)
+    {
+        (void)hipGetDevice(&dev);
+        if(dev != n->device) (void)hipSetDevice(n->device);
+        const bool ok = AllocFeatArea(*a);
+        if(dev != n->device) (void)hipSetDevice(dev);
+        if(!ok) return kNoSplit;
+    }
+    a->stream = s;
+    a->used = ++pool.uses;
+    MRAY_HIP_CHECK(hipStreamWaitEvent(s, a->done, 0));
     const EncodePlan& p = n->plan;
     for(uint32_t at = 0; at < count; at += kSplitChunk)
     {
@@ -1106,10 +1194,10 @@ static int InferSplit(MRayNrc* n, const float* dRecords, uint32_t count, float* 
         const uint32_t b = DivUp(c, kEncodeTPB), perXcd = p.own * b + p.shared * DivUp(b, 8u);
         const float* rec = dRecords + size_t(at) * 11u;
         NrcTimer t(n, 0, s);
-        KNrcEncode<<<8u * perXcd, kEncodeTPB, 0, s>>>(n->view, rec, c, p, n->feat);
-        KNrcInferEncoded<<<blocks, kInferTPB, 0, s>>>(n->view, rec, n->feat, c, dOut + size_t(at) * 3u);
+        KNrcEncode<<<8u * perXcd, kEncodeTPB, 0, s>>>(n->view, rec, c, p, a->feat);
+        KNrcInferEncoded<<<blocks, kInferTPB, 0, s>>>(n->view, rec, a->feat, c, dOut + size_t(at) * 3u);
     }
-    MRAY_HIP_CHECK(hipEventRecord(n->featDone, s));
+    MRAY_HIP_CHECK(hipEventRecord(a->done, s));
     return NrcLaunchCheck();
 }
 
