@@ -21,9 +21,13 @@ sys.path.insert(0, ROOT)
 
 METRIC = "Mpaths/s at 1080p; equal-time relMSE: radiance-cache PT vs plain PT, 1 MI355X"
 HBM_PEAK_GBS = 8000.0
-# bytes a node visit loads: BNode4 = six float4 boxes + uint4 children (112 B);
-# CNode8 = origin/exponent header + 48 B of 8-bit boxes + 32 B children (96 B)
-NODE_BYTES = {4: 64, 8: 96, "instanced": 112}   # QNode4, CNode8, BNode4
+# bytes a node visit loads, by what the kernel walks: QNode4 = grid origin and
+# step + 24 B of 8-bit boxes + 16 B children (64 B); BNode4 = six float4 boxes +
+# uint4 children (112 B), below an instance tree and in one-scene trees of at
+# most 4096 nodes; CNode8 = origin/exponent header + 48 B of 8-bit boxes + 32 B
+# children (96 B)
+NODE_BYTES = {4: 64, 8: 96, "exact": 112, "instanced": 112}
+EXACT_NODES = 4096        # kExactNodes
 TRI_BYTES = 48            # SoupTri
 RAY_BYTES = 32 + 28       # RayGMem in, hit record out (prim/t/bary + keys)
 
@@ -103,6 +107,11 @@ SHADE_BYTES = {False: 96 + 208 + 112, True: 112 + 224 + 112}
 # any-hit ray outside the tree walk: queue index 4, shadow ray 32, its
 # radiance 16, path radiance read and written 32
 SHADOW_RAY_BYTES = 4 + 32 + 16 + 32
+
+
+def node_kind(accel, width):
+    """What a one-scene renderer on `accel` walks (a key of NODE_BYTES)."""
+    return "exact" if width == 4 and accel.info()["wide_nodes"] <= EXACT_NODES else width
 
 
 def kernel_rooflines(cst, ptotals, phases, width, spectral, queues):
@@ -795,13 +804,14 @@ def main():
     assert np.isfinite(film).all()
     nodes_per_ray = cst["node_visits"] / max(1, cst["ext_rays"])
     tris_per_ray = cst["tri_tests"] / max(1, cst["ext_rays"])
+    kind = node_kind(accel, args.bvh_width)
 
     mpaths = totals["dead_paths"] / elapsed / 1e6
     mrays = (totals["ext_rays"] + totals["shadow_rays"]) / elapsed / 1e6
     trace_ms, trace_launches = phases["trace"]
     trace_avg_ms = trace_ms / max(1, trace_launches)
     rays_per_launch = ptotals["ext_rays"] / max(1, trace_launches)
-    bytes_per_ray = RAY_BYTES + nodes_per_ray * NODE_BYTES[args.bvh_width] + tris_per_ray * TRI_BYTES
+    bytes_per_ray = RAY_BYTES + nodes_per_ray * NODE_BYTES[kind] + tris_per_ray * TRI_BYTES
     achieved = rays_per_launch * bytes_per_ray / (trace_avg_ms * 1e-3) / 1e9
     traffic = traffic_from_profiles(rays_per_launch)
     result = {
@@ -858,7 +868,7 @@ def main():
             "avg_launch_ms": round(trace_avg_ms, 4),
             "rays_per_launch": round(rays_per_launch, 1),
         },
-        "kernel_rooflines": kernel_rooflines(cst, ptotals, phases, args.bvh_width, spectral,
+        "kernel_rooflines": kernel_rooflines(cst, ptotals, phases, kind, spectral,
                                              args.queues),
     }
     r.close()

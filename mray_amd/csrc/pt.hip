@@ -932,7 +932,7 @@ struct ChunkSource
 // longest of its 64 rays.  Each ray's walk is the same as KTrace's, so hits
 // are identical; only the order rays are walked in changes.
 constexpr uint32_t kRefillAt = 16;
-template<bool COUNT, bool BATCH>
+template<int W, bool COUNT, bool BATCH>
 __global__ void __launch_bounds__(kTraceTPB)
 KTraceRefill(TraceCtx ctx, SlotSoA S, const uint32_t* __restrict__ active, Sched* __restrict__ sched,
              const ViewGPU* __restrict__ views, uint32_t* __restrict__ ctr)
@@ -992,7 +992,7 @@ KTraceRefill(TraceCtx ctx, SlotSoA S, const uint32_t* __restrict__ active, Sched
         if(has)
         {
             // a walk visits at most maxVisits nodes (as TraceW)
-            bool over = WalkStep<4, false, COUNT>(ctx, lstack, gtid, w, 0u, &nodes, &tris);
+            bool over = WalkStep<W, false, COUNT>(ctx, lstack, gtid, w, 0u, &nodes, &tris);
             if(++visits >= ctx.maxVisits) over = true;
             if(over)
             {
@@ -2114,14 +2114,21 @@ static void LaunchTrace(MRayRenderer* r, hipStream_t s)
     }
     if(ctx.width == 8) KTrace<8, COUNT, BATCH><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dActive, r->dSched, r->dViews, r->dCtr);
     else if(r->params.flags & MRAY_RENDER_LANE_REFILL)
-        KTraceRefill<COUNT, BATCH><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dActive, r->dSched, r->dViews, r->dCtr);
-    else
     {
-        // counted walks are the QNode4 ones, like the lane-refill kernel's
-        if constexpr(!BATCH && !COUNT)
+        if constexpr(!BATCH)
             if(ctx.exact)
             {
-                KTrace<kNodesB4, false, false><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dActive, r->dSched, r->dViews, r->dCtr);
+                KTraceRefill<kNodesB4, COUNT, false><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dActive, r->dSched, r->dViews, r->dCtr);
+                return;
+            }
+        KTraceRefill<kNodesQ4, COUNT, BATCH><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dActive, r->dSched, r->dViews, r->dCtr);
+    }
+    else
+    {
+        if constexpr(!BATCH)
+            if(ctx.exact)
+            {
+                KTrace<kNodesB4, COUNT, false><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dActive, r->dSched, r->dViews, r->dCtr);
                 return;
             }
         KTrace<4, COUNT, BATCH><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dActive, r->dSched, r->dViews, r->dCtr);
@@ -2151,10 +2158,10 @@ static void LaunchShadow(MRayRenderer* r, hipStream_t s)
     if(ctx.width == 8) KShadow<8, BATCH, kTraceTPB, false, COUNT><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dShadowQ, r->dSched, r->dViews, r->rc.nrc, r->dCtr, r->rc.N);
     else
     {
-        if constexpr(!BATCH && !COUNT)
+        if constexpr(!BATCH)
             if(ctx.exact)
             {
-                KShadow<kNodesB4, false><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dShadowQ, r->dSched, r->dViews, r->rc.nrc, r->dCtr, r->rc.N);
+                KShadow<kNodesB4, false, kTraceTPB, false, COUNT><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dShadowQ, r->dSched, r->dViews, r->rc.nrc, r->dCtr, r->rc.N);
                 return;
             }
         KShadow<4, BATCH, kTraceTPB, false, COUNT><<<nb, kTraceTPB, 0, s>>>(ctx, r->S, r->dShadowQ, r->dSched, r->dViews, r->rc.nrc, r->dCtr, r->rc.N);
@@ -2530,7 +2537,8 @@ static int SizeLaunches(MRayRenderer* r)
     else if(!r->batch)
     {
         r->traceBlocks = uint32_t(w8 ? resident(KTrace<8, false, false>, tpb, maxTraceBlocks)
-                                : refill ? resident(KTraceRefill<false, false>, tpb, maxTraceBlocks)
+                                : refill && r->ctx.exact ? resident(KTraceRefill<kNodesB4, false, false>, tpb, maxTraceBlocks)
+                                : refill ? resident(KTraceRefill<kNodesQ4, false, false>, tpb, maxTraceBlocks)
                                 : r->ctx.exact ? resident(KTrace<kNodesB4, false, false>, tpb, maxTraceBlocks)
                                          : resident(KTrace<4, false, false>, tpb, maxTraceBlocks));
         r->shadowBlocks = uint32_t(w8 ? resident(KShadow<8, false>, tpb, maxTraceBlocks)
@@ -2547,7 +2555,7 @@ static int SizeLaunches(MRayRenderer* r)
     else
     {
         r->traceBlocks = uint32_t(w8 ? resident(KTrace<8, false, true>, tpb, maxTraceBlocks)
-                                : refill ? resident(KTraceRefill<false, true>, tpb, maxTraceBlocks)
+                                : refill ? resident(KTraceRefill<kNodesQ4, false, true>, tpb, maxTraceBlocks)
                                          : resident(KTrace<4, false, true>, tpb, maxTraceBlocks));
         r->shadowBlocks = uint32_t(w8 ? resident(KShadow<8, true>, tpb, maxTraceBlocks)
                                       : resident(KShadow<4, true>, tpb, maxTraceBlocks));

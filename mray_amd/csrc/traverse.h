@@ -550,29 +550,31 @@ template<int W, bool ANY_HIT, bool COUNT>
 __device__ __forceinline__ bool WalkStep(const TraceCtx& ctx, uint2* lstack, uint32_t gtid, Walk& w,
                                          uint32_t sp0, uint32_t* nodeVisits, uint32_t* triTests)
 {
-    static_assert(W == 4, "the walk's ray is a QNode4 tree's");
+    static_assert(W != kNodesC8, "the walk's ray is a 4-wide tree's");
+    constexpr int N = WidthOf(W);
     const uint32_t lb = StackLane<kLdsStack>();
     const uint32_t spMax = kLdsStack + ctx.gstackDepth;
     const float kGrow = 1.0000005f;
     if(COUNT) (*nodeVisits)++;
     HitRec& best = w.best;
     float curMax = (best.prim == kInvalid) ? w.tMax : best.t;
-    float tn[W];
-    uint32_t c[W];
+    float tn[N];
+    uint32_t c[N];
     uint4 ch;
-    SlabTestQ(ctx.qnodes + w.node, w.r, w.tMin, curMax, tn, ch);
+    if constexpr(W == kNodesQ4) SlabTestQ(ctx.qnodes + w.node, w.r, w.tMin, curMax, tn, ch);
+    else SlabTest4(ctx.nodes + w.node, w.r, w.tMin, curMax, tn, ch);
     c[0] = ch.x; c[1] = ch.y; c[2] = ch.z; c[3] = ch.w;
-    SortNear<W>(tn, c);
+    SortNear<N>(tn, c);
     // as in TraceW: inner children farthest first, each pushing the one
     // found before it; then the leaves nearest first
     uint32_t next = kInvalid;
     float nextT = 0.0f;
     uint32_t sp = w.sp;
     #pragma unroll
-    for(int k = W - 1; k >= 0; k--)
+    for(int k = N - 1; k >= 0; k--)
     {
         if(tn[k] == INFINITY || (c[k] & kLeafFlag)) continue;
-        if(next != kInvalid && sp < spMax)   // sp < spMax: sized (W-1) per level
+        if(next != kInvalid && sp < spMax)   // sp < spMax: sized (N-1) per level
         {
             const uint2 v = make_uint2(next, __float_as_uint(nextT));
             StackPut<kLdsStack>(ctx, lstack, sp, lb, gtid, v);
@@ -582,7 +584,7 @@ __device__ __forceinline__ bool WalkStep(const TraceCtx& ctx, uint2* lstack, uin
         nextT = tn[k];
     }
     #pragma unroll
-    for(int k = 0; k < W; k++)
+    for(int k = 0; k < N; k++)
     {
         if(tn[k] == INFINITY || !(c[k] & kLeafFlag)) continue;
         float lim = (best.prim == kInvalid) ? w.tMax : best.t;

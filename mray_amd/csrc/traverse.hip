@@ -64,6 +64,7 @@ int LaunchCastClosest(const TraceCtx& ctx, const float* dRays, uint32_t n, uint3
     if(dCounters)
     {
         if(w8) KCCastClosest<8, true><<<blocks, kTraceTPB, 0, s>>>(ctx, r, n, dPrim, dT, dBary, dCounters);
+        else if(ctx.exact) KCCastClosest<kNodesB4, true><<<blocks, kTraceTPB, 0, s>>>(ctx, r, n, dPrim, dT, dBary, dCounters);
         else KCCastClosest<4, true><<<blocks, kTraceTPB, 0, s>>>(ctx, r, n, dPrim, dT, dBary, dCounters);
     }
     else

@@ -362,3 +362,60 @@ def test_renders_of_large_scenes(torch_gpu, extent, kind):
     assert rimg.min() >= 0.49
     assert np.allclose(img, rimg, rtol=1e-5)
     acc.close()
+
+
+def _exact_visits(nodes, rays):
+    """Nodes of the 4-wide tree (words 0-23: lo/hi x, y, z of the 4 children,
+    24-27: child words) that rays without a hit enter, in float64."""
+    lo = np.stack([nodes[:, 8 * a: 8 * a + 4].view(np.float32) for a in range(3)], 2).astype(np.float64)
+    hi = np.stack([nodes[:, 8 * a + 4: 8 * a + 8].view(np.float32) for a in range(3)], 2).astype(np.float64)
+    child = nodes[:, 24:28]
+    inner = (child & 0x80000000) == 0
+    total = 0
+    for r in rays.astype(np.float64):
+        live = np.array([0])
+        while len(live):
+            total += len(live)
+            with np.errstate(divide="ignore", over="ignore", invalid="ignore"):
+                a, b = (lo[live] - r[0:3]) / r[4:7], (hi[live] - r[0:3]) / r[4:7]
+            near = np.minimum(a, b).max(axis=2)
+            far = np.maximum(a, b).min(axis=2)
+            live = child[live][(np.maximum(near, r[3]) <= np.minimum(far, r[7])) & inner[live]]
+    return total
+
+
+@pytest.mark.parametrize("cells,flags", [(16, 0), (16, abi.RENDER_LANE_REFILL), (96, 0), (96, abi.RENDER_LANE_REFILL)])
+def test_counters_are_the_timed_walk_s(torch_gpu, cells, flags):
+    """Counted nodes are those the uncounted kernels visit: on small trees the
+    exact boxes' (counted here in float64 over rays that only meet culled
+    triangles), on larger ones the quantised boxes', which are a little looser."""
+    from mray_amd import native
+    s = _lit_grid(cells, 1.0)
+    rng = np.random.default_rng(cells)
+    s.positions[:, 2] = 0.8 / cells * rng.random(len(s.positions)).astype(np.float32)
+    s.indices = s.indices[:, ::-1].copy()                        # facing away from the camera
+    s.surface_keys = np.zeros(len(s.indices), np.uint32)
+    s.light_tris, s.light_radiance = s.light_tris[:0], s.light_radiance[:0]
+    s.light_two_sided = s.light_two_sided[:0]
+    s.cull = np.ones(len(s.indices), np.uint8)
+    s.camera = {"position": (0.13, -0.2, 1.5), "gaze": (0.0, 0.1, 0.0), "up": (0, 1, 0), "fov": (1.0, 1.0),
+                "nearFar": (0.01, 100.0)}
+    params = abi.render_params(24, 24, 1, rr=(4, 4), mode=abi.SAMPLE_PURE, seed=1, flags=flags)
+    o = refcpu.OracleScene(s)
+    rays, _ = o.camera_rays(params, 24 * 24)
+    assert np.all(o.cast_closest(rays, brute=True)[0] == abi.INVALID_PRIM)
+    acc = native.Accel(s)
+    nodes, _ = acc.read_wide()
+    ref = _exact_visits(nodes, rays)
+    ctr = acc.cast_closest(torch_gpu.from_numpy(rays).cuda(), count_visits=True)[3].cpu().numpy()
+    r = native.Renderer(acc, params)
+    r.set_measurement(counting=True)
+    st = r.render_all()
+    r.close()
+    print(f"{len(nodes)} nodes: exact {ref}, cast {ctr[0]}, render {st['node_visits']}", flush=True)
+    assert st["ext_rays"] == 576 and st["node_visits"] == ctr[0]
+    if len(nodes) <= 4096:
+        assert ctr[0] == ref
+    else:
+        assert ref < ctr[0] < 1.2 * ref
+    acc.close()
