@@ -2168,11 +2168,12 @@ static void LaunchShadow(MRayRenderer* r, hipStream_t s)
     }
 }
 
-// Slot blocks up to which a block sums the earlier blocks' counts itself:
-// at 64 blocks the scan kernel took 4.4 us a bounce and its launch 1.5 more,
-// the sums 0.5; at 2025 blocks 5.2 and 1.5 against 1.2.  Beyond, the sums grow
-// with the square of the blocks.
-constexpr uint32_t kFusedRefillBlocks = 2048;
+// Slot blocks up to which a block sums the earlier blocks' counts itself; the
+// sums grow with the square of the blocks, the scan launch hardly.  The whole
+// refill of a bounce, sums against scan: 3072 blocks 26.3 / 28.7 us, 4096
+// 31.4 / 33.2, 5760 43.5 / 42.5, 8192 67.3 / 56.7.  (At 64 blocks the scan
+// kernel took 4.4 us and its launch 1.5 more, the sums 0.5.)
+constexpr uint32_t kFusedRefillBlocks = 4096;
 template<bool BATCH>
 static void LaunchRefillApply(MRayRenderer* r, bool fused, hipStream_t s)
 {

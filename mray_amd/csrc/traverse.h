@@ -29,6 +29,10 @@ static constexpr uint32_t kLdsStackInst = 12;
 // longer way.  Cornell boxes at 128^2 / 512^2 x 4, QNode4 against BNode4:
 // 19 nodes +6 / +6 %, 436 +4 / +2 %, 1394 +3 / +1 %, 6119 +1.5 / -0.3 %,
 // 30573 0 / -1.5 %.
+// Batches walk QNode4 at any size: their scenes share one array of nodes, so
+// one kind serves them all.  8 x 36, 32 x 36, 8 x 2756 and 4 x 24788 triangles
+// at 256^2 x 8: 7.25, 31.3, 10.3 and 12.0 ms (9.4, 33.9, 13.2 and 14.6 on BNode4
+// before the fused test, the fetch by position and the shorter bursts).
 static constexpr uint32_t kExactNodes = 4096;
 
 // One instance of a mesh in a two-level scene: a TRS transform (rotation

@@ -1,9 +1,9 @@
 """Renders whose slot pools outgrow the resident waves (about 393 K slots) or
-the fused refill (2048 blocks of 256 slots), against the oracle.
+the fused refill (4096 blocks of 256 slots), against the oracle.
 
 Below about 393 K slots every wave's work is its own chunk by position; above,
 the rest is handed out by counters, first of the wave's own part of the list and
-then of the parts that still hold chunks.  Up to 2048 slot blocks the refill sums
+then of the parts that still hold chunks.  Up to 4096 slot blocks the refill sums
 the blocks' counts itself, above it scans them in a launch of its own.  A chunk
 handed out twice or never would change a path's state and with it the pixel: the
 films agree pixel by pixel up to the order of their float additions, and the
@@ -27,10 +27,11 @@ def _same_film(film, ref):
     assert np.max(np.abs(film[:3] - ref[:3]) / scale) < 1e-5
 
 
-@pytest.mark.parametrize("slots", [393216, 393217, 400000, 524288, 524289, 614401])
+@pytest.mark.parametrize("slots", [393216, 393217, 400000, 614401, 1048576, 1048577])
 def test_slot_pools_match_oracle(torch_gpu, slots):
     from mray_amd import native
-    w, h, spp = 700, 301, 4                              # 842,800 paths: slots are refilled
+    # 842,800 or 1,806,000 paths: slots are refilled
+    w, h, spp = (700, 301, 4) if slots < 700000 else (1500, 301, 4)
     s = scenes.cornell(aspect=w / h)
     p = abi.render_params(w, h, spp, rr=(3, 3), seed=2, max_ray_count=slots)
     acc = native.Accel(s)
