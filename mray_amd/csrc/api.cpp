@@ -259,6 +259,8 @@ static int BuildAccel(MRayAccel* a, const MRaySceneDesc* s, uint32_t builder, ui
     {
         MRAY_TRY(DevAlloc(ar, (void**)&a->dQNodes, size_t(a->wideNodes) * sizeof(QNode4)));
         MRAY_TRY(QuantizeNodes(a->dNodes, a->wideNodes, a->dQNodes, st));
+        // the caller may walk the tree on a stream of its own
+        MRAY_HIP_CHECK(hipStreamSynchronize(st));
     }
     // Traversal stack spill area: <= width-1 entries per level below the root.
     int dev = 0;
