@@ -259,8 +259,13 @@ static int BuildAccel(MRayAccel* a, const MRaySceneDesc* s, uint32_t builder, ui
     {
         MRAY_TRY(DevAlloc(ar, (void**)&a->dQNodes, size_t(a->wideNodes) * sizeof(QNode4)));
         MRAY_TRY(QuantizeNodes(a->dNodes, a->wideNodes, a->dQNodes, st));
+        float box[6];
+        MRAY_HIP_CHECK(hipMemcpyAsync(box, a->dSceneBox, sizeof(box), hipMemcpyDeviceToHost, st));
         // the caller may walk the tree on a stream of its own
         MRAY_HIP_CHECK(hipStreamSynchronize(st));
+        float maxAbs = 0.0f;
+        for(float v : box) maxAbs = std::max(maxAbs, std::fabs(v));
+        a->ctx.maxInv = SceneMaxInv(maxAbs);
     }
     // Traversal stack spill area: <= width-1 entries per level below the root.
     int dev = 0;

@@ -20,7 +20,7 @@ KCCastClosest(TraceCtx ctx, const float4* __restrict__ rays, uint32_t n,
         float4 b = rays[2 * size_t(i) + 1];
         const V3 d = {b.x, b.y, b.z};
         HitRec h = TraceW<W, false, COUNT>(ctx, lstack, gtid, V3{a.x, a.y, a.z}, d, a.w, b.w, 0u,
-                                           &nodeVisits, &triTests, 0u, Reach(d, b.w));
+                                           &nodeVisits, &triTests, 0u, CallerReach(d, b.w, ctx.maxInv));
         prim[i] = h.prim;
         if(tOut) tOut[i] = (h.prim == kInvalid) ? b.w : h.t;
         if(bary)
@@ -49,7 +49,7 @@ KCCastVisibility(TraceCtx ctx, const float4* __restrict__ rays, uint32_t n,
         float4 b = rays[2 * size_t(i) + 1];
         const V3 d = {b.x, b.y, b.z};
         HitRec h = TraceW<W, true, false>(ctx, lstack, gtid, V3{a.x, a.y, a.z}, d, a.w, b.w, 0u,
-                                          nullptr, nullptr, 0u, Reach(d, b.w));
+                                          nullptr, nullptr, 0u, CallerReach(d, b.w, ctx.maxInv));
         visible[i] = (h.prim == kInvalid) ? 1u : 0u;
     }
 }

@@ -104,7 +104,11 @@ int main(int argc, char** argv)
         const float m = std::fmax(std::fabs(d[0]), std::fmax(std::fabs(d[1]), std::fabs(d[2])));
         if(m == 0.0f) continue;
         const V3 dir = {d[0], d[1], d[2]};
-        const RayQ r = MakeRayQ(V3{o[0], o[1], o[2]}, dir, Reach(dir, tMax));
+        // the caller's form, and the renderers' for unit vectors
+        const float maxInv = SceneMaxInv(std::fmax(coord[0], std::fmax(coord[1], coord[2])));
+        const bool unit = m >= 0.5f && m < 2.0f && it % 2 == 0;
+        const RayReach reach = unit ? kUnitReach : CallerReach(dir, tMax, maxInv);
+        const RayQ r = MakeRayQ(V3{o[0], o[1], o[2]}, dir, reach);
         for(int kind = 0; kind < 2; kind++)
         {
             float tn[4];
@@ -128,11 +132,12 @@ int main(int argc, char** argv)
                     continue;
                 }
                 LD grow[3];
-                bool bounded = true;
+                // (directions so short that the scene's size caps their reciprocal may be loose)
+                bool bounded = LD(reach.maxInv) * m >= 1e19L;
                 for(int a = 0; a < 3; a++)
                 {
                     const LD ext = LD(H[a]) - L[a];
-                    grow[a] = 0.02L * ext + 2e-6L * (coord[a] + std::fabs(LD(o[a]))) + 2e-6L / std::fmin(1.0f, m) + 1e-26L;
+                    grow[a] = 0.02L * ext + 2e-6L * (coord[a] + std::fabs(LD(o[a]))) + 2.0L * reach.reach * reach.minDir + 1e-26L;
                     bounded = bounded && coord[a] + 6 * ext < 1e18L;
                 }
                 if(bounded && !Interval(o, d, box[k], grow, 0.0f, tMax, n, f))

@@ -327,6 +327,7 @@ def test_axis_parallel_rays_in_large_scenes(torch_gpu, extent, cells):
     # direction lengths of 1e-9 and 1e9: t grows and shrinks with them
     rays[100:150, 4:7] *= np.float32(1e-9)
     rays[150:200, 4:7] *= np.float32(1e9)
+    rays[5::60, 4:7] = 0.0                                       # no direction: no hit
     along = rays[:100].copy()                                    # across the grid, above and in its plane
     along[:, 0] = -1.5 * extent
     along[:, 2] = 0.0
@@ -418,4 +419,16 @@ def test_counters_are_the_timed_walk_s(torch_gpu, cells, flags):
         assert ctr[0] == ref
     else:
         assert ref < ctr[0] < 1.2 * ref
+    # a direction's length changes t and nothing else: by a power of two, the
+    # walk is the same to the bit, with an axis it is parallel to as well
+    visits = []
+    for scale in (1.0, 2.0 ** -13, 2.0 ** 13, 2.0 ** -40):
+        r = rays.copy()
+        r[:, 4] = 0.0
+        r[::2, 5] = -0.0
+        r[:, 3] = 0.0
+        r[:, 4:7] *= np.float32(scale)
+        r[:, 7] = 3.4e38
+        visits.append(int(acc.cast_closest(torch_gpu.from_numpy(r).cuda(), count_visits=True)[3][0]))
+    assert visits[0] > 576 and len(set(visits)) == 1, visits
     acc.close()
