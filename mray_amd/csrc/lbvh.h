@@ -62,7 +62,7 @@ struct alignas(64) QNode4
 };
 static_assert(sizeof(QNode4) == 64, "QNode4 must be half a 128-byte line");
 // Sums in double (the products, 11 bits times 24, are exact).
-MRAY_HD QNode4 QuantizeNode(const BNode4& b)
+MRAY_HD QNode4 QuantizeNode(BNode4 b)
 {
     QNode4 q;
     for(int k = 0; k < 4; k++) q.child[k] = b.child[k];
