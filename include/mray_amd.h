@@ -574,7 +574,9 @@ enum
 int mray_nrc_create(const MRayNrcConfig* hCfg, MRayNrc** out);
 int mray_nrc_destroy(MRayNrc* nrc);
 /* Radiance of `count` records (or *dCount when dCount is not NULL, read on
- * the device): dOut [n][3].                                                  */
+ * the device): dOut [n][3].  Counts known on the host use a workspace that the
+ * GPU's caches share: one area of 32 MiB with the first cache, up to three more
+ * as further streams query, released with the last cache.                    */
 int mray_nrc_infer(MRayNrc* nrc, const float* dRecords, uint32_t count, const uint32_t* dCount,
                    float* dOut, void* stream);
 /* Gradients of the relative L2 loss of one batch (count a multiple of 32),
@@ -582,7 +584,7 @@ int mray_nrc_infer(MRayNrc* nrc, const float* dRecords, uint32_t count, const ui
 int mray_nrc_backward(MRayNrc* nrc, const float* dRecords, const float* dTargets, uint32_t count,
                       void* stream);
 int mray_nrc_adam(MRayNrc* nrc, void* stream);
-/* backward + adam */
+/* backward + adam (applies what earlier backward passes left pending, too) */
 int mray_nrc_train(MRayNrc* nrc, const float* dRecords, const float* dTargets, uint32_t count,
                    void* stream);
 int mray_nrc_last_loss(MRayNrc* nrc, float* hLoss);

@@ -52,7 +52,7 @@ static_assert(sizeof(BNode4) == 128, "BNode4 must be one 128-byte line");
 // on a grid of the node's own (plane p of axis a = o[a] + (1024 + q) * s[a]:
 // the walk reads a byte as the half 1024 + q), half a line.  Boxes only grow:
 // every plane stands at least 8 * 2^-24 times the node's largest coordinate
-// and 12 * 2^-24 times its extent outside the exact one (QuantizeNodes), which
+// and 12 * 2^-24 times its extent outside the exact one (QuantizeNode), which
 // covers the rounding of the walk's slab test.  Bytes k of qlo / qhi: child k.
 struct alignas(64) QNode4
 {
@@ -61,6 +61,7 @@ struct alignas(64) QNode4
     uint32_t child[4];
 };
 static_assert(sizeof(QNode4) == 64, "QNode4 must be half a 128-byte line");
+
 // Sums in double (the products, 11 bits times 24, are exact).
 MRAY_HD QNode4 QuantizeNode(BNode4 b)
 {

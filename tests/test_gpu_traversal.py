@@ -432,3 +432,28 @@ def test_counters_are_the_timed_walk_s(torch_gpu, cells, flags):
         visits.append(int(acc.cast_closest(torch_gpu.from_numpy(r).cuda(), count_visits=True)[3][0]))
     assert visits[0] > 576 and len(set(visits)) == 1, visits
     acc.close()
+
+
+@pytest.mark.parametrize("builder", ["sah", "lbvh"])
+def test_deep_stack_on_exact_nodes(torch_gpu, builder):
+    """As test_deep_stack_spills_past_lds, over few enough planes for exact
+    nodes, past the 10 LDS levels of these walks."""
+    from mray_amd import native
+    s = _plane_stack(1400)
+    acc = native.Accel(s, builder=builder, width=4)
+    nodes, _ = acc.read_wide()
+    depth = _first_descent_depth(nodes, np.float32(0.1), np.float32(-0.2))
+    print(f"{builder}: {len(nodes)} nodes, first-descent stack depth {depth}", flush=True)
+    assert len(nodes) <= 4096 and depth > 12
+    rng = np.random.default_rng(4)
+    rays = np.zeros((2000, 8), np.float32)
+    rays[:, 0:2] = rng.uniform(-0.9, 0.9, size=(2000, 2))
+    rays[:, 2] = np.where(np.arange(2000) % 3 == 2, rng.uniform(0.0, 1.0, size=2000), -1.0)
+    d = rng.normal(size=(2000, 3))
+    d[:, 2] = np.abs(d[:, 2]) + 0.2
+    d[::2] = (0.0, -0.0, 1.0)
+    rays[:, 4:7] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    rays[:, 3] = 1e-4
+    rays[:, 7] = 3.4e38
+    _compare(acc, refcpu.OracleScene(s), rays, brute=True)
+    acc.close()
