@@ -134,21 +134,21 @@ struct RayQ : RayPre
     V3 offN, offF;
 };
 
-// How a ray takes an axis it is parallel to, that is, |d| < minDir, zero included:
-// maxInv = 1 / minDir stands for the reciprocal.  Up to a distance of `reach` such
-// a ray moves less than minDir reach on the axis, so with a margin of `reach` it
-// is never taken off its origin's side of a plane, nor out of a plane it starts
-// in; the margin is reach minDir in position.
+// How a ray takes an axis it is parallel to, that is, |d| < 1 / maxInv, zero
+// included: maxInv stands for the reciprocal.  Up to a distance of `reach` such
+// a ray moves less than reach / maxInv on the axis, so with a margin of `reach`
+// it is never taken off its origin's side of a plane, nor out of a plane it
+// starts in; the margin is reach / maxInv in position.
 struct RayReach
 {
-    float minDir, maxInv, reach;
+    float maxInv, reach;
 };
 // A unit vector (a renderer's rays): no hit lies past 1e14 units of length; a
 // margin of 1e-6 in position.  1e20 and not more: a node's planes are reached
 // from an origin that lies up to four extents below its box, and every product
 // with it has to stay finite (QuantizeNode keeps origins and extents under
 // 1.5e18, and a ray's origin past 3.4e18 leaves the axis unbounded).
-constexpr RayReach kUnitReach = {1e-20f, 1e20f, 1e14f};
+constexpr RayReach kUnitReach = {1e20f, 1e14f};
 // A caller's ray: the same for a direction of any length (a division by it, down
 // to a power of two), as far as the scene's coordinates allow (`maxInv`, from
 // SceneMaxInv); and no hit lies beyond tMax.  Taken for every ray, renders of
@@ -162,7 +162,6 @@ MRAY_HD RayReach CallerReach(V3 d, float tMax, float maxInv)
     (void)frexpf(m, &e);
     RayReach r;
     r.maxInv = MinF(ldexpf(kUnitReach.maxInv, -e), maxInv);
-    r.minDir = 1.0f / r.maxInv;
     // A zero direction hits nothing (its determinants vanish): no box is entered
     // (around its origin it would visit twice as many quantised boxes as exact
     // ones: 16 K such rays in 200 K triangles 70 us and 33, now 24).
@@ -179,7 +178,7 @@ MRAY_HD float SceneMaxInv(float maxAbs)
 // its own rounding (SlabTestQ).
 MRAY_HD void MakeAxis(float o, float d, const RayReach& c, float& inv, float& offN, float& offF, uint32_t& s)
 {
-    const bool parallel = fabsf(d) < c.minDir;
+    const bool parallel = fabsf(d) * c.maxInv < 1.0f;
     inv = parallel ? copysignf(c.maxInv, d) : 1.0f / d;
     const float off = -o * inv;
     const float e = fabsf(off) * 3e-7f + (parallel ? c.reach : 0.0f);   // 5 * 2^-24, rounded up

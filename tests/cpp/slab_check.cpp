@@ -137,7 +137,7 @@ int main(int argc, char** argv)
                 for(int a = 0; a < 3; a++)
                 {
                     const LD ext = LD(H[a]) - L[a];
-                    grow[a] = 0.02L * ext + 2e-6L * (coord[a] + std::fabs(LD(o[a]))) + 2.0L * reach.reach * reach.minDir + 1e-26L;
+                    grow[a] = 0.02L * ext + 2e-6L * (coord[a] + std::fabs(LD(o[a]))) + 2.0L * reach.reach / reach.maxInv + 1e-26L;
                     bounded = bounded && coord[a] + 6 * ext < 1e18L;
                 }
                 if(bounded && !Interval(o, d, box[k], grow, 0.0f, tMax, n, f))
