@@ -876,9 +876,14 @@ using namespace mray;
 // 1 GiB for 32 views), and calls on up to kFeatAreas streams have one each, so
 // that they overlap.  Released with the GPU's last cache.
 // 16 levels of 2^19 entries, one call on each of 4 streams: 256 queries 84-100 us
-// with one area, 30 with four; 4096 96 -> 29; 16384 113 -> 43; 65536 177 -> 128;
-// 262144 428 -> 465 (two streams 213 -> 210: a call fills the GPU by itself).
+// with one area, 30 with four; 4096 96 -> 42; 16384 113 -> 44; 65536 179 -> 129;
+// 131072 265 -> 241.
 constexpr uint32_t kFeatAreas = 4;
+// Larger calls fill the GPU by themselves and take turns in the first area: side
+// by side they share the L2s that the encoding counts on.  On 4 streams, taking
+// turns against side by side: 196608 queries 344 / 364 us, 262144 429 / 451,
+// 10^6 1428 / 1500 (on two streams 711 / 773).
+constexpr uint32_t kOverlapMax = 1u << 17;
 // Queries up to which the one-kernel form is taken: its one launch costs the
 // host less than two launches, a wait and an event.  64 queries 11.3 us on one
 // stream against 11.8, on four 17.5 against 42; 128 on one stream 12.5 against 11.7.
@@ -1156,7 +1161,8 @@ int mray_nrc_destroy(MRayNrc* n)
 
 // Encoding in its own pass, chunk by chunk through an area of the GPU's pool.
 // A call takes the area of its stream's last call, else one not used yet, else
-// the one whose last use is longest ago, and waits for that use.  A call under
+// the one whose last use is longest ago (large ones the first, kOverlapMax), and
+// waits for that area's last use.  A call under
 // capture (its graph may run beside others) takes the one-kernel form, and so
 // do small ones (kOneKernelMax) and one that finds no memory for an area.
 constexpr int kNoSplit = -1;
@@ -1172,6 +1178,7 @@ static int InferSplit(MRayNrc* n, const float* dRecords, uint32_t count, float* 
     FeatArea* a = &pool.area[0];
     for(FeatArea& c : pool.area)
     {
+        if(count > kOverlapMax) break;
         if(c.used && c.stream == s) { a = &c; break; }
         if(c.used < a->used) a = &c;
     }

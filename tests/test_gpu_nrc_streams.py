@@ -37,8 +37,8 @@ def test_caches_share_query_memory(torch_gpu):
     # size class up to 2 MiB
     assert held < 24 * (8 << 20)
     rng = np.random.default_rng(5)
-    rec = torch.from_numpy(_records(rng, 70000)).cuda()
-    sizes = (100, 4096, 4097, 70000, 33, 20000)
+    rec = torch.from_numpy(_records(rng, 131073)).cuda()
+    sizes = (100, 4096, 4097, 70000, 33, 20000, 131072, 131073)
     one = {}
     for k in range(6):
         for n in sizes:
@@ -74,10 +74,10 @@ def test_queries_on_two_streams_overlap(torch_gpu):
     torch = torch_gpu
     nrc = native.Nrc(levels=16, log2_table=16, max_batch=64, seed=1)
     rec = torch.rand((1 << 19, 11), device="cuda")
-    long, short = torch.empty((1 << 19, 3), device="cuda"), torch.empty((4, 64, 3), device="cuda")
+    long, short = torch.empty((1 << 19, 3), device="cuda"), torch.empty((4, 512, 3), device="cuda")
     streams = [torch.cuda.Stream() for _ in range(5)]
     for k in range(5):                                   # areas allocated, kernels loaded
-        _infer(nrc, rec, 64, short[k % 4], stream=streams[k])
+        _infer(nrc, rec, 512, short[k % 4], stream=streams[k])
     torch.cuda.synchronize()
     early = []
     for k in range(4):
@@ -85,7 +85,7 @@ def test_queries_on_two_streams_overlap(torch_gpu):
         for _ in range(100):                             # tens of ms
             _infer(nrc, rec, 1 << 19, long, stream=streams[0])
         done[0].record(streams[0])
-        _infer(nrc, rec, 64, short[k], stream=streams[1 + k])
+        _infer(nrc, rec, 512, short[k], stream=streams[1 + k])
         done[1].record(streams[1 + k])
         done[1].synchronize()
         early.append(not done[0].query())
